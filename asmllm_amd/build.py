@@ -28,6 +28,7 @@ SOURCES = [
     "matvec_mfma.hip",
     "measure.hip",
     "decode_ops.hip",
+    "prompt_attention.hip",
     "quant.hip",
     "gemm.hip",
     "capi.hip",

@@ -7,7 +7,6 @@
 //   softmax        softmax_avx2.asm:48-130       max, exp(x - max), / sum
 //   silu_hadamard  swiglu_avx2.asm:45-81         gate = gate / (1 + exp(-gate)) * up
 //   swiglu_pairs   the same product over gate/up values interleaved in groups of 8
-//   attention      attention_avx2.asm:59-218     softmax(q k^T * scale) v, all rows (non-causal)
 //
 // plus the device-side pieces of the decode engine: RoPE fused with the fp16
 // KV-cache write, split-K attention over the fp16 cache, embedding-row
@@ -161,39 +160,6 @@ __global__ __launch_bounds__(kBlock) void swiglu_pairs_kernel(const float* __res
     if (j < H) {
         const int i = 16 * (j >> 3) + (j & 7);
         h[j] = silu_mul(gu[i], gu[i + 8]);
-    }
-}
-
-// ---- reference attention: one workgroup per query row, scores in LDS ----------------
-__global__ __launch_bounds__(kBlock) void attention_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                           const float* __restrict__ v, float* __restrict__ y,
-                                                           int seq, int hd, float scale) {
-    extern __shared__ float sc[];  // seq scores
-    __shared__ float red[kBlock / kWave];
-    const int row = blockIdx.x;
-    const float* qi = q + (size_t)row * hd;
-    for (int j = threadIdx.x; j < seq; j += kBlock) {
-        const float* kj = k + (size_t)j * hd;
-        float d = 0.f;
-        for (int t = 0; t < hd; ++t) d = fmaf(qi[t], kj[t], d);
-        sc[j] = d * scale;
-    }
-    __syncthreads();
-    float m = -INFINITY;
-    for (int j = threadIdx.x; j < seq; j += kBlock) m = fmaxf(m, sc[j]);
-    m = block_max<kBlock>(m, red);
-    float s = 0.f;
-    for (int j = threadIdx.x; j < seq; j += kBlock) {
-        const float e = expf(sc[j] - m);
-        sc[j] = e;
-        s += e;
-    }
-    s = block_sum<kBlock>(s, red);
-    __syncthreads();
-    for (int t = threadIdx.x; t < hd; t += kBlock) {
-        float a = 0.f;
-        for (int j = 0; j < seq; ++j) a = fmaf(sc[j], v[(size_t)j * hd + t], a);
-        y[(size_t)row * hd + t] = a / s;
     }
 }
 
@@ -614,11 +580,6 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float* __restrict__ 
 
 }  // namespace
 
-// The single-workgroup kernels step an int index by up to 32768 (argmax) and
-// loop while it is below the length: lengths within that stride of INT32_MAX
-// would overflow the index and never end the loop.
-constexpr int64_t kMaxStridedLen = INT32_MAX - 65536;
-
 int rmsnorm_launch(const float* x, const float* w, float* y, int64_t dim, float eps, hipStream_t st) {
     if (dim <= 0 || dim > kMaxStridedLen) return fail(kInvalidArgument, "rmsnorm: bad dim %lld", (long long)dim);
     hipLaunchKernelGGL(rmsnorm_kernel, dim3(1), dim3(1024), 0, st, x, w, y, (int)dim, eps);
@@ -667,19 +628,6 @@ int silu_launch(float* g, const float* u, int64_t dim, hipStream_t st) {
     if (dim <= 0 || dim > kMaxStridedLen) return fail(kInvalidArgument, "silu_hadamard: bad dim");
     hipLaunchKernelGGL(silu_kernel, dim3((unsigned)((dim + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, g, u,
                        (int)dim);
-    ASMHIP_TRY(hipGetLastError());
-    return kOk;
-}
-
-int attention_launch(const float* q, const float* k, const float* v, float* y, int64_t seq, int64_t hd, float scale,
-                     hipStream_t st) {
-    if (seq <= 0 || hd <= 0) return fail(kInvalidArgument, "attention: need seq > 0 and head_dim > 0");
-    if (hd > kMaxStridedLen) return fail(kInvalidArgument, "attention: head_dim %lld", (long long)hd);
-    if (seq > 40000) return fail(kUnsupported, "attention: seq_len %lld exceeds the LDS score buffer", (long long)seq);
-    const int rc = dynamic_lds((const void*)attention_kernel, (size_t)seq * sizeof(float));
-    if (rc) return rc;
-    hipLaunchKernelGGL(attention_kernel, dim3((unsigned)seq), dim3(kBlock), (size_t)seq * sizeof(float), st, q, k,
-                       v, y, (int)seq, (int)hd, scale);
     ASMHIP_TRY(hipGetLastError());
     return kOk;
 }

@@ -135,6 +135,11 @@ int random_blocks_launch(QuantType qt, void* blocks, int64_t rows, int64_t K, ui
 int random_f16_launch(void* out, int64_t n, uint64_t seed, float stddev, hipStream_t stream);
 int fill_f32_launch(float* out, int64_t n, float value, hipStream_t stream);
 
+// The single-workgroup kernels step an int index by up to 32768 (argmax) and
+// loop while it is below the length: lengths within that stride of INT32_MAX
+// would overflow the index and never end the loop.
+constexpr int64_t kMaxStridedLen = INT32_MAX - 65536;
+
 // Decode-step ops.
 int rmsnorm_launch(const float* x, const float* w, float* y, int64_t dim, float eps, hipStream_t st);
 int rope_launch(float* q, float* k, int64_t n_q_heads, int64_t n_k_heads, int64_t hd, const int* pos_ptr,
