@@ -110,29 +110,17 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// Softmax merge of the S split states of one attention head, dimension t:
-// state s is [m, l, -, -, acc[hd]] at ph + s * stride; the result is
-// (sum_s acc_s[t] f_s) / (sum_s l_s f_s) with f_s = exp(m_s - max_s m_s), both
-// sums in split order; 0 when no split saw a position (every m = -inf).
-__device__ __forceinline__ float attn_merge_value(const float* ph, int S, int stride, int t) {
-    float M = -INFINITY;
-    for (int i = 0; i < S; ++i) M = fmaxf(M, ph[(size_t)i * stride]);
-    float L = 0.f, a = 0.f;
-    if (M != -INFINITY) {
-        for (int i = 0; i < S; ++i) {
-            const float f = __expf(ph[(size_t)i * stride] - M);
-            L = fmaf(ph[(size_t)i * stride + 1], f, L);
-            a = fmaf(ph[(size_t)i * stride + 4 + t], f, a);
-        }
-    }
-    return M == -INFINITY ? 0.f : a / L;
-}
+// 2^x by the hardware's exponential (results below 2^-126 are zero).
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// attn_merge_value for the dimensions t..t+3 and t+16..t+19 of one head (t % 4
-// == 0, stride % 4 == 0, ph 16-byte aligned) over exactly S splits, bit for bit
-// the same values, in two steps: load() requests every state with
-// unconditional loads (so the wait before finish() counts them exactly),
-// finish() forms the values once they are in.
+// Softmax merge of the S split states of one attention head, dimension t: state s
+// is [m, l, -, -, acc[hd]] with m a power of two's exponent; the result is
+// (sum_s acc_s[t] f_s) / (sum_s l_s f_s) with f_s = 2^(m_s - max_s m_s), both sums
+// in split order; 0 when no split saw a position (every m = -inf).
+// AttnMergeQuads forms it for the dimensions t..t+3 and t+16..t+19 of one head (t % 4
+// == 0, stride % 4 == 0, ph 16-byte aligned) over exactly S splits, in two steps:
+// load() requests every state with unconditional loads (so the wait before finish()
+// counts them exactly), finish() forms the values once they are in.
 template <int S>
 struct AttnMergeQuads {
     float2 ml[S];
@@ -166,7 +154,7 @@ struct AttnMergeQuads {
         if (M != -INFINITY) {
 #pragma unroll
             for (int i = 0; i < S; ++i) {
-                const float f = __expf(ml[i].x - M);
+                const float f = exp2_fast(ml[i].x - M);
                 L = fmaf(ml[i].y, f, L);
                 const float v[8] = {ac[i][0].x, ac[i][0].y, ac[i][0].z, ac[i][0].w,
                                     ac[i][1].x, ac[i][1].y, ac[i][1].z, ac[i][1].w};

@@ -164,26 +164,32 @@ __global__ __launch_bounds__(kBlock) void swiglu_pairs_kernel(const float* __res
 }
 
 // ---- decode attention over the fp16 cache: one launch per layer ----------------------
-// grid (n_heads, S = ceil(max_ctx / SL)), SL = attn_split_len(max_ctx); workgroup
-// (h, s) covers positions [s*SL, (s+1)*SL) of 0..pos.  Within a workgroup
+// S = ceil(max_ctx / SL) splits, SL = attn_split_len(max_ctx); a workgroup covers
+// positions [s*SL, (s+1)*SL) of 0..pos for one query head.  Without grouped queries
+// (n_heads = n_kv) the grid is (n_heads, S) and k and v are read with nontemporal
+// loads: the cache rows are read once per token.  GQA: workgroup ids are dealt
+// round-robin to the 8 dies, so id -> (die id % 8, i = id / 8) -> pair (i / group) * 8
+// + die of kv head and split, query head i % group: the group's heads read their rows
+// at the same time behind one L2, with cached loads (32 heads on 8 kv heads, 8000
+// positions: 21.3 us in head order, 10.4 so; 9.8 with the scoring loop below, which
+// bounds it there, 7.4 us for the 7B shape's 32 x 2048 positions).  Within a workgroup
 // a position is read by HD/8 lanes (8 dims = 16 bytes each), so a wave covers
 // 64/(HD/8) positions per row and the four waves kRowPos; a lane reads
 // kAttnRows rows of k and of v per chunk (one position each), and the split is
 // kChunks chunks walked with the next two chunks' loads in flight while the
-// current one is scored (three register buffers).  k and v are read with nontemporal
-// loads: the cache rows are read once per token.  Each lane group keeps an
+// current one is scored (three register buffers).  Each lane group keeps an
 // online softmax state (max m, sum l, acc[8]) over its positions; the states of
 // all lane groups of the workgroup merge once through LDS; each workgroup
-// writes [m, l, -, -, acc[HD]] (kAttnPartStride(HD) floats, acc 16-byte
+// writes [m, l, -, -, acc[HD]] (m a power of two's exponent) (kAttnPartStride(HD) floats, acc 16-byte
 // aligned) to `part`, and attn_decode_merge, or a matvec whose x is the
 // attention output (kPreAttnMerge), combines the S partials of a head in split
-// order into acc / l (attn_merge_value).
+// order into acc / l.
 //
 // ROPE != kRopeNone also does what rope_kv_write does, inside the same launch:
 // q and the new k are rotated at `pos`, the new k and v are rounded to fp16 and
 // written to the caches at `pos` (by the workgroup of the first query head of
-// the kv group), and the lane that owns `pos` uses those fp16 values instead of
-// reading the row it writes.  kRopeTheta forms the angles (rope_angle, double
+// the kv group), and every head adds that row from those fp16 values instead of
+// reading it.  kRopeTheta forms the angles (rope_angle, double
 // precision: about 600 fp64 instructions that every wave waits for); kRopeTable
 // reads the same cos/sin values from a table that rope_table_kernel filled
 // once, a load that travels with the k/v loads.
@@ -206,6 +212,19 @@ __device__ __forceinline__ float group_sum(float v) {
 template <int E>
 struct HalfRow {
     uint32_t w[E / 2];
+    template <bool NT>
+    __device__ __forceinline__ static HalfRow load(__amdgpu_buffer_rsrc_t res, uint32_t off) {
+        HalfRow r;
+        if constexpr (E == 8) {
+            const uint4 v = NT ? buf_load_b128_nt(res, off) : buf_load_b128(res, off);
+            r.w[0] = v.x, r.w[1] = v.y, r.w[2] = v.z, r.w[3] = v.w;
+        } else {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b96(res, (int)off, 0, NT ? 2 : 0);
+#pragma unroll
+            for (int i = 0; i < E / 2; ++i) r.w[i] = v[i];
+        }
+        return r;
+    }
     __device__ static HalfRow load(const __half* p) {
         HalfRow r;
         if constexpr (E == 8) {
@@ -237,7 +256,7 @@ constexpr uint32_t kAttnPastEnd = 0xFFFFFF00u;  // buffer offset that loads zero
 
 enum RopeMode : int { kRopeNone = 0, kRopeTheta = 1, kRopeTable = 2 };
 
-template <int HD, int ROPE, int SL>
+template <int HD, int ROPE, int SL, bool GQA>
 __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __restrict__ qkv, __half* kc, __half* vc,
                                                              float* __restrict__ part, int n_heads, int n_kv,
                                                              const int* __restrict__ pos_ptr, int max_ctx,
@@ -256,21 +275,37 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
     constexpr int kGroupsWg = kBlock / kLanes;  // lane groups (position slots) of the workgroup
     __shared__ float wst[kGroupsWg][HD + 2];
 
-    const int h = blockIdx.x, split = blockIdx.y;
-    const int group = n_heads / n_kv, kvh = h / group;
+    const int group = n_heads / n_kv, S = (max_ctx + SL - 1) / SL;
+    int h, split;
+    if constexpr (GQA) {
+        const int id = blockIdx.x, i = id >> 3, pair = (i / group) * 8 + (id & 7);
+        if (pair >= n_kv * S) return;
+        h = (pair % n_kv) * group + i % group;
+        split = pair / n_kv;
+    } else {
+        h = blockIdx.x;
+        split = blockIdx.y;
+    }
+    const int kvh = h / group;
     const int pos = *pos_ptr;
     const int n_pos = (pos >= 0 && pos < max_ctx) ? pos + 1 : 0;  // an invalid position reads and writes nothing
-    const int p0 = split * SL, p1 = min(p0 + SL, n_pos);
+    const int p0 = split * SL;
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x >> 6;
     const int g = lane / kLanes, c = lane % kLanes;
-    const size_t head_off = (size_t)kvh * max_ctx * HD + E * c;
-    // position of row r of chunk ch for this lane
-    auto position = [&](int ch, int r) { return p0 + ch * kChunkPos + r * kRowPos + w * kGroups + g; };
+    float* mine = part + ((size_t)h * S + split) * kStride;
+    if (p0 >= n_pos) {  // no position (the loads were out of range): an empty state
+        if (threadIdx.x < HD) mine[4 + threadIdx.x] = 0.f;
+        if (threadIdx.x == 0) mine[0] = -INFINITY, mine[1] = 0.f;
+        return;
+    }
+    // positions 0..pos-1 come from the cache in chunks; the row at pos, which this
+    // launch may write, is added after them by lane group 0 of wave 0
+    const int n_old = max(n_pos - 1, 0);
+    const size_t head_off = (size_t)kvh * max_ctx * HD;
 
     // q first, then the first chunk's k rows, then its v rows: loads return in
-    // order, so the scores can start while v is in flight.  HD % 64 == 0:
-    // branch-free buffer loads, a row outside the split (or the row at pos,
-    // which this launch writes) reading zeros from past the end of the buffer.
+    // order, so the scores can start while v is in flight.  Branch-free buffer
+    // loads: rows from pos on lie past the end of the descriptors and read zeros.
     float qv[E];
 #pragma unroll
     for (int t = 0; t < E; t += 2) {
@@ -280,7 +315,7 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
     // cos, sin of this lane's E / 2 pairs (pair E/2 c + i at 2i, 2i + 1)
     float csl[E];
     if constexpr (ROPE == kRopeTable) {
-        const float* row = rope_table + (size_t)(n_pos > 0 ? pos : 0) * HD + E * c;
+        const float* row = rope_table + (size_t)n_old * HD + E * c;
 #pragma unroll
         for (int t = 0; t < E; t += 2) {
             const float2 a = *reinterpret_cast<const float2*>(row + t);
@@ -292,51 +327,36 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
     // 384 positions: 7.65 us with two buffers, 7.55 with three, 7.68 with four)
     constexpr int NB = kChunks >= 3 ? 3 : kChunks;
     HalfRow<E> kr[NB][R], vr[NB][R];
-    const uint32_t cache_bytes = (uint32_t)n_kv * (uint32_t)max_ctx * (uint32_t)(2 * HD);  // < 4 GB, checked at launch
-    const auto kres = make_rsrc(kc, cache_bytes), vres = make_rsrc(vc, cache_bytes);
+    const uint32_t old_bytes = (uint32_t)n_old * (uint32_t)(2 * HD);
+    const auto kres = make_rsrc(kc + head_off, old_bytes), vres = make_rsrc(vc + head_off, old_bytes);
+    const uint32_t off0 = (uint32_t)(p0 + w * kGroups + g) * (uint32_t)(2 * HD) + (uint32_t)(2 * E * c);
     auto issue = [&](int b, int ch) {
-        uint32_t off[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int p = position(ch, r);
-            const bool live = p < p1 && !(ROPE != kRopeNone && p == pos);
-            off[r] = live ? 2u * (uint32_t)(head_off + (size_t)p * HD) : kAttnPastEnd;
-            if constexpr (E == 8) {
-                const uint4 a = buf_load_b128_nt(kres, off[r]);
-                kr[b][r].w[0] = a.x, kr[b][r].w[1] = a.y, kr[b][r].w[2] = a.z, kr[b][r].w[3] = a.w;
-            } else {
-                kr[b][r] = live ? HalfRow<E>::load(kc + off[r] / 2) : HalfRow<E>::zero();
-            }
-        }
+        for (int r = 0; r < R; ++r) kr[b][r] = HalfRow<E>::template load<!GQA>(kres, off0 + (uint32_t)((ch * R + r) * kRowPos * 2 * HD));
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if constexpr (E == 8) {
-                const uint4 a = buf_load_b128_nt(vres, off[r]);
-                vr[b][r].w[0] = a.x, vr[b][r].w[1] = a.y, vr[b][r].w[2] = a.z, vr[b][r].w[3] = a.w;
-            } else {
-                vr[b][r] = off[r] != kAttnPastEnd ? HalfRow<E>::load(vc + off[r] / 2) : HalfRow<E>::zero();
-            }
-        }
+        for (int r = 0; r < R; ++r) vr[b][r] = HalfRow<E>::template load<!GQA>(vres, off0 + (uint32_t)((ch * R + r) * kRowPos * 2 * HD));
     };
 #pragma unroll
     for (int c = 0; c < NB - 1; ++c) issue(c, c);
     if constexpr (ROPE == kRopeTheta) {
-        if (threadIdx.x < HD / 2 && n_pos > 0)
+        if (threadIdx.x < HD / 2)
             rope_angle(threadIdx.x, HD, pos, theta, &cs[2 * threadIdx.x], &cs[2 * threadIdx.x + 1]);
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < E; ++t) csl[t] = cs[E * c + t];
     }
-    // the new row: rotated k and v of kv head kvh, rounded to fp16, used by
-    // the lane that owns position pos (chunk nch, row nr)
-    HalfRow<E> kq = HalfRow<E>::zero(), vq = HalfRow<E>::zero();
-    int nch = -1, nr = -1;
     if constexpr (ROPE != kRopeNone) {
-        if (n_pos > 0) {
 #pragma unroll
-            for (int i = 0; i < E / 2; ++i) rotate(&qv[2 * i], csl[2 * i], csl[2 * i + 1]);
-        }
-        if (p0 <= pos && pos < p1) {
+        for (int i = 0; i < E / 2; ++i) rotate(&qv[2 * i], csl[2 * i], csl[2 * i + 1]);
+    }
+    // the row at pos, in the one split that holds it: rotated k and v of kv head
+    // kvh rounded to fp16 and written to the caches, or read from them
+    const bool has_new = pos < p0 + SL;  // wave-uniform
+    HalfRow<E> kq = HalfRow<E>::zero(), vq = HalfRow<E>::zero();
+    if (has_new) {
+        __half* krow = kc + head_off + (size_t)pos * HD + E * c;
+        __half* vrow = vc + head_off + (size_t)pos * HD + E * c;
+        if constexpr (ROPE != kRopeNone) {
             const float* kn = qkv + (size_t)(n_heads + kvh) * HD + E * c;
             const float* vn = qkv + (size_t)(n_heads + n_kv + kvh) * HD + E * c;
 #pragma unroll
@@ -348,67 +368,82 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
                 vq.w[i] = (uint32_t)__half_as_ushort(__float2half_rn(vn[2 * i])) |
                           ((uint32_t)__half_as_ushort(__float2half_rn(vn[2 * i + 1])) << 16);
             }
-            const int rel = pos - p0, rem = rel % kRowPos;
-            if (w == rem / kGroups && g == rem % kGroups) {
-                nch = rel / kChunkPos;
-                nr = (rel % kChunkPos) / kRowPos;
-                if (h % group == 0) {
-                    kq.store(kc + head_off + (size_t)pos * HD);
-                    vq.store(vc + head_off + (size_t)pos * HD);
-                }
+            if (w == 0 && g == 0 && h % group == 0) {
+                kq.store(krow);
+                vq.store(vrow);
             }
+        } else {
+            kq = HalfRow<E>::load(krow);
+            vq = HalfRow<E>::load(vrow);
         }
     }
-    const float scale = 1.0f / sqrtf((float)HD);
+    // scores in powers of two: exp(s) = 2^(s log2 e)
+    const float scale = 1.44269504088896340736f / sqrtf((float)HD);
 #pragma unroll
     for (int t = 0; t < E; ++t) qv[t] *= scale;
 
     // chunk by chunk: request the next chunk, then score this one and fold it
-    // into the lane group's online softmax state
-    float m = -INFINITY, l = 0.f, acc[E];
+    // into the lane group's online softmax state.  m follows the maximum only when
+    // it has grown by more than kSlack (weights up to 2^kSlack lose nothing in
+    // fp32), so the sums are rescaled in a wave's first chunk and rarely again;
+    // base stands for m while every score so far is -inf.
+    constexpr float kSlack = 10.f;
+    float m = -INFINITY, base = 0.f, l = 0.f, acc[E];
 #pragma unroll
     for (int t = 0; t < E; ++t) acc[t] = 0.f;
+    auto score = [&](const HalfRow<E>& k) {
+        float d = 0.f;
+#pragma unroll
+        for (int t = 0; t < E / 2; ++t) {
+            d = fmaf(qv[2 * t], half_lo(k.w[t]), d);
+            d = fmaf(qv[2 * t + 1], half_hi(k.w[t]), d);
+        }
+        return group_sum<kLanes>(d);
+    };
+    auto grow = [&](float mc) {  // makes m the base of scores up to mc
+        if (__any(mc > m + kSlack || m == -INFINITY)) {
+            const float mn = fmaxf(m, mc);
+            base = mn == -INFINITY ? 0.f : mn;
+            const float f = exp2_fast(m - base);  // 0 while the state is empty
+            m = mn;
+            l *= f;
+#pragma unroll
+            for (int t = 0; t < E; ++t) acc[t] *= f;
+        }
+    };
+    auto fold = [&](float s, const HalfRow<E>& v) {
+        const float e = exp2_fast(s - base);  // 0 for positions past the split
+        l += e;
+#pragma unroll
+        for (int t = 0; t < E / 2; ++t) {
+            acc[2 * t] = fmaf(e, half_lo(v.w[t]), acc[2 * t]);
+            acc[2 * t + 1] = fmaf(e, half_hi(v.w[t]), acc[2 * t + 1]);
+        }
+    };
+    const bool whole = p0 + SL <= n_old;  // wave-uniform
 #pragma unroll
     for (int ch = 0; ch < kChunks; ++ch) {
         const int b = ch % NB;
         if (ch + NB - 1 < kChunks) issue((ch + NB - 1) % NB, ch + NB - 1);
-        if (ch == nch) {
+        float sc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) sc[r] = score(kr[b][r]);
+        if (!whole) {
 #pragma unroll
             for (int r = 0; r < R; ++r)
-                if (r == nr) kr[b][r] = kq, vr[b][r] = vq;
+                if (p0 + (ch * R + r) * kRowPos + w * kGroups + g >= n_old) sc[r] = -INFINITY;
         }
-        float sc[R];
-        float mc = -INFINITY;
+        float mc = sc[0];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            float d = 0.f;
+        for (int r = 1; r < R; ++r) mc = fmaxf(mc, sc[r]);
+        grow(mc);
 #pragma unroll
-            for (int t = 0; t < E / 2; ++t) {
-                d = fmaf(qv[2 * t], half_lo(kr[b][r].w[t]), d);
-                d = fmaf(qv[2 * t + 1], half_hi(kr[b][r].w[t]), d);
-            }
-            d = group_sum<kLanes>(d);
-            sc[r] = position(ch, r) < p1 ? d : -INFINITY;
-            mc = fmaxf(mc, sc[r]);
-        }
-        const float mn = fmaxf(m, mc);
-        if (mn != -INFINITY) {
-            const float f = __expf(m - mn);  // 0 while the state is empty
-            l *= f;
-#pragma unroll
-            for (int t = 0; t < E; ++t) acc[t] *= f;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float e = __expf(sc[r] - mn);  // 0 for positions past the split
-                l += e;
-#pragma unroll
-                for (int t = 0; t < E / 2; ++t) {
-                    acc[2 * t] = fmaf(e, half_lo(vr[b][r].w[t]), acc[2 * t]);
-                    acc[2 * t + 1] = fmaf(e, half_hi(vr[b][r].w[t]), acc[2 * t + 1]);
-                }
-            }
-            m = mn;
-        }
+        for (int r = 0; r < R; ++r) fold(sc[r], vr[b][r]);
+    }
+    if (has_new) {
+        const float d = score(kq), s = w == 0 && g == 0 ? d : -INFINITY;
+        grow(s);
+        fold(s, vq);
     }
     // every lane group's softmax state to LDS (no cross-lane shuffles), then one
     // merge over all groups of the workgroup in group order; thread t < HD owns
@@ -420,7 +455,6 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
         if (c == 0) wst[gs][0] = m, wst[gs][1] = l;
     }
     __syncthreads();
-    float* mine = part + ((size_t)h * gridDim.y + split) * kStride;
     if (threadIdx.x < HD) {
         float M = -INFINITY;
 #pragma unroll
@@ -429,7 +463,7 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
         if (M != -INFINITY) {
 #pragma unroll
             for (int i = 0; i < kGroupsWg; ++i) {
-                const float f = __expf(wst[i][0] - M);  // 0 for groups that saw no position
+                const float f = exp2_fast(wst[i][0] - M);  // 0 for groups that saw no position
                 L = fmaf(wst[i][1], f, L);
                 a = fmaf(wst[i][2 + threadIdx.x], f, a);
             }
@@ -439,14 +473,42 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
     }
 }
 
-// Merge of the S partials of head h (blockIdx.x) in split order; thread t owns
-// dimension t.  Splits past the last position hold m = -inf, l = 0.
+// Merge of the S <= 64 partials of head h (blockIdx.x) in split order; thread t owns
+// dimension t: the sums of AttnMergeQuads, bit for bit.  Splits past the last position
+// hold m = -inf, l = 0.  Bound by the latency of the partials, which other dies'
+// workgroups wrote: every wave reads all (m, l) with one load, a lane each, and the
+// accumulators kMergeBatch splits at a time (32 heads, 16 splits: 4.0 us a launch one
+// split after another, 2.8 so).
+constexpr int kMergeBatch = 32;
+
 template <int HD>
-__global__ __launch_bounds__(HD) void attn_decode_merge(const float* __restrict__ part, float* __restrict__ out,
-                                                        int S) {
-    const int h = blockIdx.x;
-    out[(size_t)h * HD + threadIdx.x] = attn_merge_value(part + (size_t)h * S * kAttnPartStride(HD), S,
-                                                         kAttnPartStride(HD), threadIdx.x);
+__global__ __launch_bounds__((HD + 63) / 64 * 64) void attn_decode_merge(const float* __restrict__ part,
+                                                                         float* __restrict__ out, int S) {
+    constexpr int kStride = kAttnPartStride(HD);
+    const int h = blockIdx.x, t = threadIdx.x, lane = t & (kWave - 1);
+    const float* ph = part + (size_t)h * S * kStride;
+    const int d = min(t, HD - 1);
+    const float2 ml = *reinterpret_cast<const float2*>(ph + (size_t)min(lane, S - 1) * kStride);
+    float L = 0.f, a = 0.f, M = -INFINITY, f = 0.f;
+    for (int i0 = 0; i0 < S; i0 += kMergeBatch) {
+        float v[kMergeBatch];
+#pragma unroll
+        for (int i = 0; i < kMergeBatch; ++i)
+            if (i0 + i < S) v[i] = ph[(size_t)(i0 + i) * kStride + 4 + d];
+        if (i0 == 0) {
+            M = wave_max(ml.x);  // lanes past the last split repeat it
+            f = M == -INFINITY ? 0.f : exp2_fast(ml.x - M);
+        }
+#pragma unroll
+        for (int i = 0; i < kMergeBatch; ++i)
+            if (i0 + i < S) {
+                const float fi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), i0 + i));
+                const float li = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.y), i0 + i));
+                L = fmaf(li, fi, L);
+                a = fmaf(v[i], fi, a);
+            }
+    }
+    if (t < HD) out[(size_t)h * HD + t] = M == -INFINITY ? 0.f : a / L;
 }
 
 // ---- embedding row of a Q4_0 table -----------------------------------------------------
@@ -642,31 +704,27 @@ int64_t attn_decode_workspace(int n_heads, int hd, int max_ctx) {
 }
 
 namespace {
-template <int HD, int SL>
-void launch_attn_split(int mode, dim3 grid, hipStream_t st, const float* qkv, __half* kc, __half* vc, float* part,
+template <int HD, int SL, bool GQA>
+void launch_attn_split(int mode, int splits, hipStream_t st, const float* qkv, __half* kc, __half* vc, float* part,
                        int n_heads, int n_kv, const int* pos_ptr, int max_ctx, float theta, const float* rope_table) {
-    if (mode == kRopeTable)
-        hipLaunchKernelGGL((attn_decode_kernel<HD, kRopeTable, SL>), grid, dim3(kBlock), 0, st, qkv, kc, vc, part,
-                           n_heads, n_kv, pos_ptr, max_ctx, theta, rope_table);
-    else if (mode == kRopeTheta)
-        hipLaunchKernelGGL((attn_decode_kernel<HD, kRopeTheta, SL>), grid, dim3(kBlock), 0, st, qkv, kc, vc, part,
-                           n_heads, n_kv, pos_ptr, max_ctx, theta, rope_table);
-    else
-        hipLaunchKernelGGL((attn_decode_kernel<HD, kRopeNone, SL>), grid, dim3(kBlock), 0, st, qkv, kc, vc, part,
-                           n_heads, n_kv, pos_ptr, max_ctx, theta, rope_table);
+    const dim3 grid = GQA ? dim3((unsigned)((n_kv * splits + 7) / 8 * 8 * (n_heads / n_kv))) : dim3(n_heads, splits);
+    const auto kern = mode == kRopeTable   ? attn_decode_kernel<HD, kRopeTable, SL, GQA>
+                      : mode == kRopeTheta ? attn_decode_kernel<HD, kRopeTheta, SL, GQA>
+                                           : attn_decode_kernel<HD, kRopeNone, SL, GQA>;
+    hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, st, qkv, kc, vc, part, n_heads, n_kv, pos_ptr, max_ctx, theta,
+                       rope_table);
 }
 
 template <int HD>
-void launch_attn_decode(int mode, dim3 grid, hipStream_t st, const float* qkv, __half* kc, __half* vc, float* part,
+void launch_attn_decode(int mode, int splits, hipStream_t st, const float* qkv, __half* kc, __half* vc, float* part,
                         float* out, int n_heads, int n_kv, const int* pos_ptr, int max_ctx, float theta,
                         const float* rope_table) {
-    if (attn_split_len(max_ctx) == kAttnSplitShort)
-        launch_attn_split<HD, kAttnSplitShort>(mode, grid, st, qkv, kc, vc, part, n_heads, n_kv, pos_ptr, max_ctx,
-                                               theta, rope_table);
-    else
-        launch_attn_split<HD, kAttnSplitLong>(mode, grid, st, qkv, kc, vc, part, n_heads, n_kv, pos_ptr, max_ctx,
-                                              theta, rope_table);
-    if (out) hipLaunchKernelGGL((attn_decode_merge<HD>), dim3(n_heads), dim3(HD), 0, st, part, out, (int)grid.y);
+    const bool is_short = attn_split_len(max_ctx) == kAttnSplitShort, gqa = n_heads > n_kv;
+    const auto split = is_short ? (gqa ? launch_attn_split<HD, kAttnSplitShort, true> : launch_attn_split<HD, kAttnSplitShort, false>)
+                                : (gqa ? launch_attn_split<HD, kAttnSplitLong, true> : launch_attn_split<HD, kAttnSplitLong, false>);
+    split(mode, splits, st, qkv, kc, vc, part, n_heads, n_kv, pos_ptr, max_ctx, theta, rope_table);
+    if (out) hipLaunchKernelGGL((attn_decode_merge<HD>), dim3(n_heads), dim3((HD + 63) / 64 * 64), 0, st, part,
+                                out, splits);
 }
 }  // namespace
 
@@ -685,17 +743,16 @@ int attn_decode_launch(const float* qkv, void* k_cache, void* v_cache, float* pa
     if ((int64_t)n_kv * max_ctx * hd * 2 >= (int64_t)kAttnPastEnd)
         return fail(kUnsupported, "attention: caches of 4 GB or more per layer are not supported");
     const int mode = !rope ? kRopeNone : rope_table ? kRopeTable : kRopeTheta;
-    const dim3 grid(n_heads, splits);
     __half* kc = (__half*)k_cache;
     __half* vc = (__half*)v_cache;
     if (hd == 128)
-        launch_attn_decode<128>(mode, grid, st, qkv, kc, vc, part, out, n_heads, n_kv, pos_ptr, max_ctx, theta,
+        launch_attn_decode<128>(mode, splits, st, qkv, kc, vc, part, out, n_heads, n_kv, pos_ptr, max_ctx, theta,
                                 rope_table);
     else if (hd == 64)
-        launch_attn_decode<64>(mode, grid, st, qkv, kc, vc, part, out, n_heads, n_kv, pos_ptr, max_ctx, theta,
+        launch_attn_decode<64>(mode, splits, st, qkv, kc, vc, part, out, n_heads, n_kv, pos_ptr, max_ctx, theta,
                                rope_table);
     else if (hd == 48)
-        launch_attn_decode<48>(mode, grid, st, qkv, kc, vc, part, out, n_heads, n_kv, pos_ptr, max_ctx, theta,
+        launch_attn_decode<48>(mode, splits, st, qkv, kc, vc, part, out, n_heads, n_kv, pos_ptr, max_ctx, theta,
                                rope_table);
     else
         return fail(kUnsupported, "attention: head_dim %d (supported: 48, 64, 128)", hd);
@@ -713,7 +770,7 @@ int attn_merge_launch(const float* part, float* out, int n_heads, int hd, int ma
     else if (hd == 64)
         hipLaunchKernelGGL((attn_decode_merge<64>), dim3(n_heads), dim3(64), 0, st, part, out, splits);
     else if (hd == 48)
-        hipLaunchKernelGGL((attn_decode_merge<48>), dim3(n_heads), dim3(48), 0, st, part, out, splits);
+        hipLaunchKernelGGL((attn_decode_merge<48>), dim3(n_heads), dim3(64), 0, st, part, out, splits);
     else
         return fail(kUnsupported, "attention merge: head_dim %d (supported: 48, 64, 128)", hd);
     ASMHIP_TRY(hipGetLastError());

@@ -31,7 +31,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_at(const float* x, int b,
 // sums is left out for all but a wave's first block as a rule).  base stands for m
 // while every score so far is -inf: such scores then weigh 0, and a NaN stays one.
 constexpr float kSlack = 10.f;
-__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float base_of(float m) { return m == -INFINITY ? 0.f : m; }
 
 // The merge of NW softmax states of one row, a quad of dimensions: state w is
