@@ -695,8 +695,12 @@ extern "C" int asmhip_matmul_attn_output(int qtype, const void* blocks, const fl
     o.accumulate = accumulate != 0;
     o.attn_splits = splits;
     o.attn_hd = head_dim;
-    // one launch where the int8-MFMA stream takes the shape: the merge is its x prologue
-    if (get_q4_kernel() != kQ4KernelFp32) {
+    // one launch where the matvec kernel of the shape takes the merge as its x prologue
+    const int bits = qt == QuantType::Q4_0 ? 4 : 8, sel = get_q4_kernel();
+    if (K <= kSmallK && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0) &&
+        matvec_rows_takes(bits, true, blocks, nullptr, nullptr, workspace, M, K, o))
+        return matvec_rows_launch(bits, true, blocks, nullptr, nullptr, workspace, y, M, K, st, o);
+    if (sel != kQ4KernelFp32) {
         if (qt == QuantType::Q4_0 && q4_0_mfma_eligible(blocks, workspace, o, M, K))
             return q4_0_mfma_launch(blocks, workspace, y, M, K, st, o);
         if (qt == QuantType::Q8_0 && q8_0_mfma_eligible(blocks, workspace, o, M, K))

@@ -85,6 +85,19 @@ bool split_mfma_eligible(int bits, const void* qs, const uint8_t* qh, const floa
 int split_mfma_launch(int bits, const void* qs, const uint8_t* qh, const float* scales, const float* x, float* y,
                       int64_t M, int64_t K, hipStream_t stream);
 
+// The fp32 row kernels over GGUF blocks or split planes (bits = 4, 5 or 8; qh for
+// split Q5, scales for split): any K % 32 == 0 whose x fits LDS, 4-byte aligned
+// operands, every pre-op and post-op (kPreAttnMerge: K <= kSmallK; kPostSwiGlu8: M %
+// 16).  Up to kSmallK they are also faster than the int8-MFMA stream, whose units of
+// 256 columns then leave 12 of its 16 waves idle (Q4_0 288 x 768 3.1 -> 2.3 us, 1536 x
+// 768 3.2 -> 2.5, 32000 x 256 6.9 -> 4.5; at K = 1536 from 4096 rows on it is not: 3.5
+// against 3.7).
+constexpr int kSmallK = 1024;
+bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const float* scales, const float* x,
+                       int64_t M, int64_t K, const MatvecOpts& opts);
+int matvec_rows_launch(int bits, bool gguf, const void* w, const uint8_t* qh, const float* scales, const float* x,
+                       float* y, int64_t M, int64_t K, hipStream_t stream, const MatvecOpts& opts);
+
 // C[T][M] = A (Q8_0 blocks [T][K/32]) x W (Q8_0 blocks [M][K/32])^T, block dots
 // scaled by both fp16 scales and accumulated in block order.
 int gemm_q8_0_launch(const void* w, const void* a, float* c, int64_t T, int64_t M, int64_t K, hipStream_t stream);

@@ -652,6 +652,12 @@ int matvec_launch(QuantType qt, bool gguf, const void* w, const float* scales, c
     int rc = kOk;
 
     const int sel = g_q4_kernel.load(std::memory_order_relaxed);
+    const int bits = qt == QuantType::Q4_0 ? 4 : 8;
+    // pre-ops: only for the shapes the pair kernels take (the entry points' contract)
+    const bool rows = (opts.pre == kPreNone || pairs) &&
+                      matvec_rows_takes(bits, gguf, w, nullptr, scales, x, M, K, opts);
+    if (rows && K <= kSmallK && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
+        return matvec_rows_launch(bits, gguf, w, nullptr, scales, x, y, M, K, stream, opts);
     if (qt == QuantType::Q4_0 && gguf) {
         const bool mfma_ok = q4_0_mfma_eligible(w, x, opts, M, K);
         if (sel == kQ4KernelMfma && !mfma_ok)
@@ -669,6 +675,7 @@ int matvec_launch(QuantType qt, bool gguf, const void* w, const float* scales, c
         if (!gguf && opts.pre == kPreNone && !opts.accumulate && split_mfma_eligible(8, w, nullptr, scales, x, M, K))
             return split_mfma_launch(8, w, nullptr, scales, x, y, M, K, stream);
     }
+    if (rows) return matvec_rows_launch(bits, gguf, w, nullptr, scales, x, y, M, K, stream, opts);
     if (pairs && qt == QuantType::Q4_0) {
         const int r = pick_rows_per_wave(M, 8);
         if (gguf) {
@@ -749,11 +756,20 @@ int matvec_swiglu_launch(QuantType qt, const void* w, const float* x, float* h, 
     MatvecOpts po = opts;
     po.post = kPostSwiGlu8;
     const int64_t M = 2 * H;
-    const int sel = g_q4_kernel.load(std::memory_order_relaxed);
+    const int sel = g_q4_kernel.load(std::memory_order_relaxed), bits = qt == QuantType::Q4_0 ? 4 : 8;
+    // the row kernels combine the pairs of a shape that their plain launch takes too
+    // (h over x: only the two launches below read all of x before they write h)
+    const bool apart = h + H <= x || x + K <= h;
+    const bool rows = apart && (opts.pre == kPreNone || (opts.pre <= kPreSwiGlu && K % 64 == 0)) &&
+                      matvec_rows_takes(bits, true, w, nullptr, nullptr, x, M, K, po);
+    if (rows && K <= kSmallK && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
+        return matvec_rows_launch(bits, true, w, nullptr, nullptr, x, h, M, K, stream, po);
     if (sel != kQ4KernelFp32) {
         if (qt == QuantType::Q4_0 && q4_0_mfma_eligible(w, x, po, M, K)) return q4_0_mfma_launch(w, x, h, M, K, stream, po);
         if (qt == QuantType::Q8_0 && q8_0_mfma_eligible(w, x, po, M, K)) return q8_0_mfma_launch(w, x, h, M, K, stream, po);
     }
+    if (rows && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
+        return matvec_rows_launch(bits, true, w, nullptr, nullptr, x, h, M, K, stream, po);
     // any other shape or kernel: the 2H rows to `work`, then the pairs combined
     const int rc = matvec_launch(qt, true, w, nullptr, x, work, M, K, stream, opts);
     return rc ? rc : swiglu_pairs_launch(work, h, H, stream);
@@ -775,10 +791,13 @@ int q5_matvec_launch(bool gguf, const void* w, const uint8_t* qh, const float* s
     const int m = (int)M, k = (int)K;
     int rc = kOk;
     const int sel = g_q4_kernel.load(std::memory_order_relaxed);
-    const bool mfma = sel != kQ4KernelFp32;
+    const bool mfma = sel != kQ4KernelFp32, rows = matvec_rows_takes(5, gguf, w, qh, scales, x, M, K, MatvecOpts());
+    if (rows && K <= kSmallK)
+        return matvec_rows_launch(5, gguf, w, qh, scales, x, y, M, K, stream, MatvecOpts());
     if (mfma && gguf && q5_0_mfma_eligible(w, x, M, K)) return q5_0_mfma_launch(w, x, y, M, K, stream);
     if (mfma && !gguf && split_mfma_eligible(5, w, qh, scales, x, M, K))
         return split_mfma_launch(5, w, qh, scales, x, y, M, K, stream);
+    if (rows) return matvec_rows_launch(5, gguf, w, qh, scales, x, y, M, K, stream, MatvecOpts());
     if (pairs) {
         const int r = pick_rows_per_wave(M, 4);
         if (gguf) {

@@ -1,0 +1,150 @@
+"""GPU parity of the fp32 row kernels over the forms their dispatch divides: every
+block type and layout, ragged K around each register pass and LDS unit, few and many
+rows, the fused pre-ops, SwiGLU and the residual add, against float64 on the same
+bytes.
+
+Bar, per row: each product is exact; the sums are 17 roundings deep within a block,
+at most 96 over the blocks of a short row (whole rows in one wave) or K / 2048 + 8 over
+a lane's, 8 over lanes and waves, and a pre-op adds 8: |y - y64| <= (48 + min(K / 32,
+96) + K / 2048) 2^-24 sum |w| |x|.
+"""
+
+import numpy as np
+import pytest
+
+from asmllm_amd import gguf, native
+from asmllm_amd.device import DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(rng, q, M, K):
+    """GGUF blocks and the exact float64 matrix."""
+    nb = K // 32
+    d = (rng.standard_normal((M, nb)) * 0.01).astype(np.float16)
+    if q == 8:
+        n = rng.integers(-128, 128, (M, nb, 32)).astype(np.int8)
+        b = np.concatenate([d[..., None].view(np.uint8), n.view(np.uint8)], -1)
+        v = n.astype(np.float64)
+    elif q == 4:
+        qs = rng.integers(0, 256, (M, nb, 16)).astype(np.uint8)
+        b = np.concatenate([d[..., None].view(np.uint8), qs], -1)
+        v = np.concatenate([qs & 15, qs >> 4], -1).astype(np.float64) - 8
+    else:
+        ql = rng.integers(0, 256, (M, nb, 16)).astype(np.uint8)
+        qh = rng.integers(0, 256, (M, nb, 4)).astype(np.uint8)
+        b = gguf.pack_q5_0(ql, qh, d)
+        return b, gguf.dequantize_q5_0(b).astype(np.float64)
+    return np.ascontiguousarray(b), (v * d[..., None].astype(np.float64)).reshape(M, K)
+
+
+def _bar(w, x, K):
+    return (48 + min(K / 32, 96) + K / 2048) * 2.0 ** -24 * (np.abs(w) @ np.abs(x).astype(np.float64)) + 1e-30
+
+
+def _call(hip, q, split, b, x, M, K):
+    dx, dy = DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(np.full(M, np.nan, np.float32))
+    if split:
+        parts = {4: gguf.split_q4_0, 5: gguf.split_q5_0, 8: gguf.split_q8_0}[q](b)
+        bufs = [DeviceBuffer.from_numpy(np.ascontiguousarray(p).view(np.uint8)) for p in parts]
+        fn = {4: hip.asmhip_matmul_q4_split, 5: hip.asmhip_matmul_q5_split, 8: hip.asmhip_matmul_q8_split}[q]
+        rc = fn(*[t.ptr for t in bufs], dx.ptr, dy.ptr, M, K, None)
+    else:
+        bufs = [DeviceBuffer.from_numpy(b)]
+        fn = {4: hip.asmhip_matmul_q4_0, 5: hip.asmhip_matmul_q5_0, 8: hip.asmhip_matmul_q8_0}[q]
+        rc = fn(bufs[0].ptr, dx.ptr, dy.ptr, M, K, None)
+    assert rc == 0, hip.asmhip_last_error()
+    return dy.download(np.float32, (M,))
+
+
+SHAPES = [(1, 32), (5, 64), (17, 96), (300, 288), (700, 512), (33, 544), (2100, 768), (63, 1024), (520, 1056),
+          (70, 2080), (2100, 2080), (3, 4128), (600, 5504), (40, 8160), (24, 8224), (20, 16416), (9, 21024),
+          (9000, 288), (17000, 544)]
+
+
+@pytest.mark.parametrize("q", [4, 5, 8])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("M,K", SHAPES)
+def test_row_kernels_shapes(hip, q, split, M, K):
+    rng = np.random.default_rng(M + K + q)
+    b, w = _weights(rng, q, M, K)
+    x = (rng.standard_normal(K) * np.exp(rng.standard_normal(K))).astype(np.float32)
+    y = _call(hip, q, split, b, x, M, K)
+    assert np.all(np.abs(y - w @ x.astype(np.float64)) <= _bar(w, x, K))
+    for col in (0, K // 2 - 1, K - 1):  # one column, exactly: its bytes and no others
+        one = np.zeros(K, np.float32)
+        one[col] = 1.0
+        assert np.array_equal(_call(hip, q, split, b, one, M, K).astype(np.float64), w[:, col])
+
+
+@pytest.mark.parametrize("M,K", [(4096, 5504), (16400, 2080), (5000, 8224)])
+def test_row_kernels_many_units(hip, M, K):
+    """Several units per wave, and rows cut into chunks (matvec_rows' stream)."""
+    rng = np.random.default_rng(M)
+    b, w = _weights(rng, 8, M, K)
+    x = rng.standard_normal(K).astype(np.float32)
+    y = _call(hip, 8, False, b, x, M, K)
+    assert np.all(np.abs(y - w @ x.astype(np.float64)) <= _bar(w, x, K))
+
+
+@pytest.mark.parametrize("q", [4, 8])
+@pytest.mark.parametrize("M,K", [(16, 64), (304, 320), (1040, 768), (64, 1088), (160, 8256), (16400, 576)])
+@pytest.mark.parametrize("pre", ["none", "rmsnorm", "swiglu"])
+@pytest.mark.parametrize("form", ["plain", "accumulate", "pairs"])
+def test_row_kernels_fused(hip, q, M, K, pre, form):
+    rng = np.random.default_rng(M * 7 + K + q)
+    b, w = _weights(rng, q, M, K)
+    x, arg, y0 = (rng.standard_normal(n).astype(np.float32) for n in (K, K, M))
+    x64, a64 = x.astype(np.float64), arg.astype(np.float64)
+    xin = {"none": x64, "rmsnorm": x64 / np.sqrt((x64 ** 2).mean() + 1e-5) * a64,
+           "swiglu": x64 / (1 + np.exp(-x64)) * a64}[pre]
+    op = {"none": native.PRE_NONE, "rmsnorm": native.PRE_RMSNORM, "swiglu": native.PRE_SWIGLU}[pre]
+    db, dx, da = DeviceBuffer.from_numpy(b), DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(arg)
+    dy = DeviceBuffer.from_numpy(y0)
+    qt = native.Q4_0 if q == 4 else native.Q8_0
+    ref, bar = w @ xin, _bar(w, xin, K)
+    if form == "pairs":
+        work = DeviceBuffer(4 * M)
+        rc = hip.asmhip_matmul_swiglu(qt, db.ptr, dx.ptr, dy.ptr, M // 2, K, op, da.ptr, 1e-5, work.ptr, None)
+        assert rc == 0, hip.asmhip_last_error()
+        y = dy.download(np.float32, (M // 2,))
+        g, u = (ref.reshape(-1, 2, 8)[:, i].reshape(-1) for i in (0, 1))
+        bg, bu = (bar.reshape(-1, 2, 8)[:, i].reshape(-1) for i in (0, 1))
+        sg = g / (1 + np.exp(-g))
+        # |d silu| <= 1.1 |dg|; the division, exponential and product: 8 roundings
+        assert np.all(np.abs(y - sg * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(sg) * bu + 2.0 ** -21 * np.abs(sg * u) + 1e-30)
+        return
+    rc = hip.asmhip_matmul_fused(qt, db.ptr, dx.ptr, dy.ptr, M, K, op, da.ptr, 1e-5, int(form == "accumulate"), None)
+    assert rc == 0, hip.asmhip_last_error()
+    y = dy.download(np.float32, (M,))
+    if form == "accumulate":
+        ref, bar = ref + y0, bar + 2.0 ** -23 * (np.abs(y0) + np.abs(ref))
+    assert np.all(np.abs(y - ref) <= bar)
+
+
+@pytest.mark.parametrize("qt", [native.Q4_0, native.Q8_0])
+@pytest.mark.parametrize("n_heads,hd,max_ctx,pos,M", [(6, 48, 256, 100, 288), (6, 48, 3072, 3000, 288), (2, 64, 900, 899, 70),
+                                                       (8, 128, 770, 5, 1024), (16, 64, 3072, 1, 3000)])
+def test_row_kernels_merge_attention(hip, qt, n_heads, hd, max_ctx, pos, M):
+    """The split states merged by the o matvec give the bits of the merge launch and
+    the matvec over its output."""
+    rng = np.random.default_rng(pos + M)
+    K = n_heads * hd
+    b, _ = _weights(rng, 4 if qt == native.Q4_0 else 8, M, K)
+    qkv = rng.standard_normal(3 * K).astype(np.float32)
+    cache = [rng.standard_normal((n_heads, max_ctx, hd)).astype(np.float16).view(np.uint16) for _ in range(2)]
+    db, dq, dk, dv = (DeviceBuffer.from_numpy(a) for a in (b, qkv, *cache))
+    dpos = DeviceBuffer.from_numpy(np.array([pos], np.int32))
+    ws = DeviceBuffer(4 * hip.asmhip_attention_decode_workspace(n_heads, hd, max_ctx))
+    table, attn, work = DeviceBuffer(4 * max_ctx * hd), DeviceBuffer(4 * K), DeviceBuffer(4 * K)
+    y0 = rng.standard_normal(M).astype(np.float32)
+    d1, d2 = DeviceBuffer.from_numpy(y0), DeviceBuffer.from_numpy(y0)
+    calls = [hip.asmhip_rope_table(table.ptr, hd, max_ctx, 10000.0, None),
+             hip.asmhip_attention_decode_partials_rope_table(dq.ptr, dk.ptr, dv.ptr, ws.ptr, n_heads, n_heads, hd,
+                                                             dpos.ptr, max_ctx, table.ptr, None),
+             hip.asmhip_matmul_attn_output(qt, db.ptr, ws.ptr, work.ptr, d1.ptr, M, n_heads, hd, max_ctx, 1, None),
+             hip.asmhip_attention_decode_rope_table(dq.ptr, dk.ptr, dv.ptr, ws.ptr, attn.ptr, n_heads, n_heads, hd,
+                                                    dpos.ptr, max_ctx, table.ptr, None),
+             hip.asmhip_matmul_fused(qt, db.ptr, attn.ptr, d2.ptr, M, K, native.PRE_NONE, None, 0.0, 1, None)]
+    assert calls == [0] * 5, hip.asmhip_last_error()
+    assert np.array_equal(d1.download(np.uint32, (M,)), d2.download(np.uint32, (M,)))
