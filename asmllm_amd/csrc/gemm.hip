@@ -42,6 +42,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
 constexpr int kTT = 64;            // T rows per workgroup
@@ -703,6 +704,312 @@ __global__ __launch_bounds__(kSplitThreads) void gemm_q8_split(const int8_t* __r
     }
 }
 
+// ---------------------------------------------------------------------------
+// Few rows of A: a workgroup of NW <= 4 waves computes 16 NW (T) x 16 (M) outputs, one
+// 16x16 tile a wave, so that a short prompt still reaches every compute unit (24 x 4096
+// x 4096: 32 workgroups of the 64 x 128 tile, 256 of these).  The same products in the
+// same order, so C keeps its bits:
+//   v_mfma_i32_16x16x32_i8    the block's int32 dots: lane l holds 8 of the 32 quants of
+//                             row l % 16, the same 8 places for A and W;
+//   v_mfma_f32_16x16x16_f16   blocks: the outer product of the fp16 scales, each in the
+//                             first place of all four lane groups (4 d_a d_w, exact);
+//   v_mfma_f32_16x16x4_f32    split planes: d_a d_w, rounded once, with the scales in
+//                             lane group 0 and zeros in the others;
+//   cvt + fma                 acc += dot * scale, block by block.
+// A step's rows are fetched by 16-byte loads that write
+// LDS themselves (slot = lane, so rows get their pitch from the slots they are given),
+// two steps in flight.  Bound by the issue of one wave's operand reads, matrix
+// instructions and sums at the smallest T (about 1000 cycles for eight blocks: the sums
+// of an output follow each other, so its blocks stay with one wave), and by the LDS reads
+// and vector work of 16x16 tiles, about 1.6 times the 32x32 tile's per output, at larger
+// T.
+// ---------------------------------------------------------------------------
+enum NarrowForm : int { kNarrowBlocks = 0, kNarrowTiled = 1, kNarrowSplit = 2 };
+
+template <int FORM, int NW>
+struct Narrow {
+    // blocks per step: 8, for runs of 256 or 272 bytes a row; the tile layout's runs are
+    // whole at any step, and at four tiles four blocks leave room for four workgroups a
+    // unit (200 x 4096 x 11008 71 -> 65 us; 93 -> 102 for the split planes' 128-byte runs)
+    static constexpr int B = FORM == kNarrowTiled && NW == 4 ? 4 : 8;
+    // 16-byte slots of a region: rows of kPitchSlots (blocks: the 34 B bytes of a step in
+    // their aligned window, plus one; split: 32 B bytes plus one; all pitches keep the
+    // operand reads of 16 rows on distinct banks), or the B / 2 16-row pair steps of the
+    // tile layout (68 bytes a row)
+    static constexpr int kReal = FORM == kNarrowSplit ? 2 * B : (34 * B + 12 + 15) / 16, kPitchSlots = kReal + 1;
+    static constexpr int kPitch = 16 * kPitchSlots;
+    static constexpr int kWSlots = FORM == kNarrowTiled ? B / 2 * 68 : 16 * kPitchSlots;
+    static constexpr int kWLoads = (kWSlots + 63) / 64, kALoads = (NW * kWSlots + 63) / 64;
+    // split: the scales of 64 / B rows x B blocks a 4-byte load
+    static constexpr int kWSc = FORM == kNarrowSplit ? 16 * B / 64 : 0, kASc = kWSc * NW;
+    static constexpr int kLoads = kWLoads + kALoads + kWSc + kASc;  // wave-wide loads a step
+    // up to two tiles leave whole SIMDs to waves that only load: a load costs its wave
+    // about 30 cycles of issue, a quarter of a tile's step (5 rows 12.2 -> 10.3 us, split
+    // 20.4 -> 10.2)
+    static constexpr int NL = NW <= 2 ? 4 - NW : 4, kFirst = NW <= 2 ? NW : 0, kThreads = 256;
+    static constexpr int kPerWave = (kLoads + NL - 1) / NL;
+    static constexpr int kAOff = kWLoads * 1024, kScOff = kAOff + kALoads * 1024;
+    static constexpr int kSpare = kScOff + (kWSc + kASc) * 256;     // landing place of padding loads
+    static constexpr int kStage = kSpare + (kPerWave * NL > kLoads ? 1024 : 0);
+    // three stages, two steps in flight: more (up to 150 KB) changed nothing where a
+    // workgroup has a compute unit to itself and cost the others their company (24 x
+    // 11008 x 4096 37.7 us against 17.5)
+    static constexpr int S = 3;
+    static_assert((S - 1) * kPerWave < 64, "the wait counts to 63");
+};
+
+struct NarrowArgs {
+    const uint8_t* w;
+    const uint8_t* a;
+    const float* wsc;  // split
+    const float* asc;
+    float* c;
+    int T, M, K, tiles_t, n_tiles;
+};
+
+template <int kCount>
+__device__ __forceinline__ void wait_loads() {  // at most kCount of the wave's loads outstanding
+    static_assert(kCount < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt(0xF70 | (kCount & 15) | ((kCount >> 4) << 14));
+}
+
+template <int FORM, int NW>
+__global__ __launch_bounds__(256) void gemm_narrow(const NarrowArgs g) {
+    using N = Narrow<FORM, NW>;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    // XCD-aware tile order, as gemm_q8_0_coalesced: T fastest
+    const int chunk = (int)gridDim.x >> 3;
+    const int tile = ((int)blockIdx.x & 7) * chunk + ((int)blockIdx.x >> 3);
+    if (tile >= g.n_tiles) return;
+    const int nb = g.K >> 5, nsteps = (nb + N::B - 1) / N::B;
+    const int t0 = (tile % g.tiles_t) * 16 * NW, j0 = (tile / g.tiles_t) * 16;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row_bytes = FORM == kNarrowSplit ? (uint32_t)g.K : (uint32_t)nb * 34u, sc_bytes = (uint32_t)nb * 4u;
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) void*)lds;
+
+    // tile layout: the 16-row slab of W inside its 128-row tile, A's rows inside their 64-row tile
+    const uint8_t *wbase = g.w, *abase = g.a;
+    uint32_t wsize = row_bytes * (uint32_t)g.M, asize = row_bytes * (uint32_t)g.T;
+    if constexpr (FORM == kNarrowTiled) {
+        const int64_t wt = (int64_t)(nb >> 1) * (kGemmTileW * 68), at = (int64_t)(nb >> 1) * (kGemmTileA * 68);
+        const int wr = (j0 % kGemmTileW) * 68, ar = (t0 % kGemmTileA) * 68;
+        wbase += (j0 / kGemmTileW) * wt + wr;
+        abase += (t0 / kGemmTileA) * at + ar;
+        wsize = (uint32_t)(wt - wr);
+        asize = (uint32_t)(at - ar);
+    }
+    const bool loads = wave >= N::kFirst;  // wave-uniform
+    const int lw = wave - N::kFirst;
+    // this lane's offset in load j of a step, from the step's descriptor
+    uint32_t off[N::kPerWave];
+#pragma unroll
+    for (int u = 0; u < N::kPerWave; ++u) {
+        const int j = lw + N::NL * u;
+        uint32_t o = kPastEnd;
+        if (j < N::kWLoads + N::kALoads) {
+            const bool is_w = j < N::kWLoads;
+            const int q = 64 * (is_w ? j : j - N::kWLoads) + lane;
+            if constexpr (FORM == kNarrowTiled) {
+                const int per = is_w ? 68 : 68 * NW, p = q / per;
+                if (p < N::B / 2) o = (uint32_t)(p * (is_w ? kGemmTileW : kGemmTileA) * 68 + 16 * (q - p * per));
+            } else {
+                const int r = q / N::kPitchSlots, k = q - r * N::kPitchSlots;
+                const int row = (is_w ? j0 : t0) + r;
+                if (r < (is_w ? 16 : 16 * NW) && k < N::kReal && row < (is_w ? g.M : g.T))
+                    o = (((uint32_t)row * row_bytes) & ~15u) + 16u * (uint32_t)k;
+            }
+        } else if (j < N::kLoads) {
+            const int js = j - N::kWLoads - N::kALoads;
+            const bool is_w = js < N::kWSc;
+            const int q = 64 * (is_w ? js : js - N::kWSc) + lane, row = (is_w ? j0 : t0) + q / N::B;
+            if (row < (is_w ? g.M : g.T)) o = (uint32_t)row * sc_bytes + 4u * (uint32_t)(q % N::B);
+        }
+        off[u] = o;
+    }
+    auto fetch = [&](int stage, int s) {
+        // blocks: in whole 16 bytes, so that the loads stay aligned (a step of four starts 8
+        // bytes on in its rows' windows every other time)
+        const uint32_t wofs = (uint32_t)s * (uint32_t)(FORM == kNarrowTiled ? N::B / 2 * kGemmTileW * 68 : FORM == kNarrowSplit ? 32 * N::B : 34 * N::B) & (FORM == kNarrowBlocks ? ~15u : ~0u);
+        const uint32_t aofs = FORM == kNarrowTiled ? (uint32_t)s * (uint32_t)(N::B / 2 * kGemmTileA * 68) : wofs;
+        const v4i wr = raw_rsrc(wbase + wofs, wsize - wofs), ar = raw_rsrc(abase + aofs, asize - aofs);
+#pragma unroll
+        for (int u = 0; u < N::kPerWave; ++u) {
+            const int j = lw + N::NL * u;  // wave-uniform
+            const int ld = j < N::kWLoads + N::kALoads ? 1024 * j
+                           : j < N::kLoads             ? N::kScOff + 256 * (j - N::kWLoads - N::kALoads)
+                                                       : N::kSpare;
+            const uint32_t m0 = lds0 + (uint32_t)(stage * N::kStage + ld);
+            // M0 has no other user in this kernel (as in gemm_q8_0_tiled)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+            if (FORM != kNarrowSplit || j < N::kWLoads + N::kALoads || j >= N::kLoads) {
+                asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, 0 offen lds" ::"v"(off[u]), "s"(m0),
+                             "s"(j < N::kWLoads ? wr : ar)
+                             : "memory", "m0");
+            } else {
+                const bool is_w = j < N::kWLoads + N::kALoads + N::kWSc;
+                const v4i sr = raw_rsrc((is_w ? g.wsc : g.asc) + N::B * s,
+                                        sc_bytes * (uint32_t)(is_w ? g.M : g.T) - 4u * (uint32_t)(N::B * s));
+                asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dword %0, %2, 0 offen lds" ::"v"(off[u]), "s"(m0), "s"(sr)
+                             : "memory", "m0");
+            }
+#pragma clang diagnostic pop
+        }
+    };
+
+    const int m = lane & 15, grp = lane >> 4;
+    const uint32_t sel = grp ? 0x07060504u : 0x07060100u;
+    [[maybe_unused]] const uint32_t first = grp ? 0u : ~0u;  // split: the scales of lane group 0
+    // byte offsets of this lane's A and W rows in a stage (blocks: the row's data start
+    // where its aligned window leaves them)
+    const int arow = 16 * wave + m;
+    int a_at = N::kAOff + arow * (FORM == kNarrowTiled ? 68 : N::kPitch), w_at = m * (FORM == kNarrowTiled ? 68 : N::kPitch);
+    if constexpr (FORM == kNarrowBlocks) {
+        a_at += (int)(((uint32_t)(t0 + arow) * row_bytes) & 15u);
+        w_at += (int)(((uint32_t)(j0 + m) * row_bytes) & 15u);
+    }
+    constexpr int kAPair = FORM == kNarrowTiled ? 1088 * NW : 68, kWPair = FORM == kNarrowTiled ? 1088 : 68;
+    const int as_at = N::kScOff + N::kWSc * 256 + arow * (4 * N::B), ws_at = N::kScOff + m * (4 * N::B);  // split scales
+
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    // block BLK of the pair at p (the lane's row of one operand): 8 quants and the scale
+    auto operand = [&](auto blk_c, const uint8_t* p, uint32_t* d) -> long {
+        constexpr int BLK = decltype(blk_c)::value;
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(p + 36 * BLK) + 2 * grp;
+        uint32_t lo = q[0];
+        const uint32_t hi = q[1];
+        if constexpr (BLK == 0) lo = __builtin_amdgcn_perm(lo, *reinterpret_cast<const uint32_t*>(p + 32), sel);
+        *d = *reinterpret_cast<const uint16_t*>(p + 34 * BLK);
+        return (long)(((uint64_t)hi << 32) | lo);
+    };
+    struct Operands {
+        long a, w;
+        uint32_t da, dw;
+    };
+    auto read = [&](auto blk_c, const uint8_t* stage, int p) {
+        constexpr int BLK = decltype(blk_c)::value;
+        Operands o;
+        if constexpr (FORM == kNarrowSplit) {
+            const int b = 2 * p + BLK;
+            o.a = *reinterpret_cast<const long*>(stage + a_at + 32 * b + 8 * grp);
+            o.w = *reinterpret_cast<const long*>(stage + w_at + 32 * b + 8 * grp);
+            o.da = *reinterpret_cast<const uint32_t*>(stage + as_at + 4 * b) & first;
+            o.dw = *reinterpret_cast<const uint32_t*>(stage + ws_at + 4 * b) & first;
+        } else {
+            o.a = operand(blk_c, stage + a_at + kAPair * p, &o.da);
+            o.w = operand(blk_c, stage + w_at + kWPair * p, &o.dw);
+            asm("" : "+v"(o.da));
+            asm("" : "+v"(o.dw));
+        }
+        return o;
+    };
+    const v4i zi = {0, 0, 0, 0};
+    const v4f zf = {0.f, 0.f, 0.f, 0.f};
+    auto dots = [&](const Operands& o) { return __builtin_amdgcn_mfma_i32_16x16x32_i8(o.a, o.w, zi, 0, 0, 0); };
+    auto scales = [&](const Operands& o) {
+        if constexpr (FORM == kNarrowSplit) {
+            return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(o.da), __uint_as_float(o.dw), zf, 0, 0, 0);
+        } else {
+            typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+            return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, (v2u){o.da, 0u}),
+                                                         __builtin_bit_cast(v4h, (v2u){o.dw, 0u}), zf, 0, 0, 0);
+        }
+    };
+    auto add = [&](const v4i& dd, const v4f& ss) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = fmaf((float)dd[i], ss[i], acc[i]);
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+
+#pragma unroll
+    for (int s = 0; s < N::S - 1; ++s)
+        if (loads) fetch(s, min(s, nsteps - 1));
+    int cur = 0, next = N::S - 1;
+    for (int s = 0; s < nsteps; ++s) {
+        // a wave's loads of step s have landed once at most the next S - 2 steps' are
+        // outstanding; then every wave's
+        if (loads) wait_loads<(N::S - 2) * N::kPerWave>();
+        __builtin_amdgcn_s_barrier();
+        // stage `next` was read in step s - 1, which every wave finished before the
+        // barrier; past the end the last step is loaded again
+        if (loads) fetch(next, min(s + N::S - 1, nsteps - 1));
+        const uint8_t* stage = lds + cur * N::kStage + (FORM == kNarrowBlocks ? (34 * N::B * s) & 15 : 0);
+        if (wave < NW) {
+            // the step's operands, then its matrix instructions, then its sums: one block
+            // after another a wave waited for each read, product and conversion in turn
+            // (24 x 4096 x 4096 16.8 us against 13.2).  Blocks past the last add nothing.
+            Operands o[N::B];
+#pragma unroll
+            for (int p = 0; p < N::B / 2; ++p) {
+                o[2 * p] = read(even, stage, p);
+                o[2 * p + 1] = read(odd, stage, p);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            v4i dd[N::B];
+            v4f ss[N::B];
+#pragma unroll
+            for (int b = 0; b < N::B; ++b) {
+                dd[b] = dots(o[b]);
+                ss[b] = scales(o[b]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (N::B * s + N::B <= nb) {
+#pragma unroll
+                for (int b = 0; b < N::B; ++b) add(dd[b], ss[b]);
+            } else {
+#pragma unroll
+                for (int b = 0; b < N::B; ++b)
+                    if (N::B * s + b < nb) add(dd[b], ss[b]);
+            }
+        }
+        cur = cur + 1 == N::S ? 0 : cur + 1;
+        next = next + 1 == N::S ? 0 : next + 1;
+    }
+    wait_loads<0>();  // no wave ends with loads into LDS in flight
+    if (wave >= NW) return;
+    // lane l, register i: row 4 (l / 16) + i, column l % 16
+    const int col = j0 + m;
+    if (col < g.M) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = t0 + 16 * wave + 4 * grp + i;
+            if (row < g.T) g.c[(size_t)row * g.M + col] = FORM == kNarrowSplit ? acc[i] : 0.25f * acc[i];
+        }
+    }
+}
+
+template <int FORM, int NW>
+int narrow_launch_nw(NarrowArgs g, hipStream_t st) {
+    using N = Narrow<FORM, NW>;
+    g.tiles_t = (g.T + 16 * NW - 1) / (16 * NW);
+    const int64_t n = (int64_t)g.tiles_t * ((g.M + 15) / 16);
+    g.n_tiles = (int)n;
+    const int rc = dynamic_lds((const void*)gemm_narrow<FORM, NW>, (size_t)N::S * N::kStage);
+    if (rc) return rc;
+    hipLaunchKernelGGL((gemm_narrow<FORM, NW>), dim3((unsigned)((n + 7) / 8 * 8)), dim3(N::kThreads),
+                       (size_t)N::S * N::kStage, st, g);
+    ASMHIP_TRY(hipGetLastError());
+    return kOk;
+}
+
+template <int FORM>
+int narrow_launch(const NarrowArgs& g, hipStream_t st) {
+    if (g.T <= 16) return narrow_launch_nw<FORM, 1>(g, st);
+    if (g.T <= 32) return narrow_launch_nw<FORM, 2>(g, st);
+    if (g.T <= 48) return narrow_launch_nw<FORM, 3>(g, st);
+    return narrow_launch_nw<FORM, 4>(g, st);
+}
+
+// While the 16-column workgroups come to at most four a compute unit: 24 x 4096 x 4096
+// blocks 32.5 -> 11.9 us, split 41.3 -> 12.0, tiled 26.8 -> 11.4; 200 x 4096 x 11008 (1024
+// of them) 84 -> 78, 122 -> 93, 69 -> 65.  Past that the larger tiles' fewer reads per
+// output win: 128 x 11008 x 4096 (1376) 37 / 50 / 28 us against 53 / 58 / 38.
+bool use_narrow(int64_t T, int64_t M) {
+    return (T + 63) / 64 * ((M + 15) / 16) <= 1024;
+}
+
 // Two blocks per staged K step, two steps of loads in flight per thread, at
 // 80 VGPRs: six waves per SIMD, so three 8-wave workgroups share a compute unit.
 // Deeper rings and 4- or 8-block steps cost occupancy on MI355X, and so did
@@ -727,6 +1034,9 @@ int gemm_q8_0_launch(const void* w, const void* a, float* c, int64_t T, int64_t 
     if ((uintptr_t)w % 4 || (uintptr_t)a % 4) return fail(kInvalidArgument, "gemm: blocks must be 4-byte aligned");
     const dim3 grid((unsigned)((M + kTM - 1) / kTM), (unsigned)((T + kTT - 1) / kTT));
     if (grid.y > 65535) return fail(kInvalidArgument, "gemm: T too large");
+    if ((K / 32) % 2 == 0 && use_narrow(T, M) && ((uintptr_t)w | (uintptr_t)a) % 16 == 0)
+        return narrow_launch<kNarrowBlocks>({static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(a), nullptr,
+                                             nullptr, c, (int)T, (int)M, (int)K, 0, 0}, st);
     if ((K / 32) % kGemmKB == 0) {
         const int tiles_t = (int)((T + kCoTT - 1) / kCoTT), n_tiles = tiles_t * (int)((M + kCoTM - 1) / kCoTM);
         const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);
@@ -762,6 +1072,9 @@ int gemm_q8_split_launch(const int8_t* wq, const float* wsc, const int8_t* aq, c
         return fail(kInvalidArgument, "gemm_split: qs planes must be 16-byte aligned, scales 4-byte aligned");
     const int64_t tiles_t = (T + kTT - 1) / kTT, n_tiles = tiles_t * ((M + kTM - 1) / kTM);
     if (n_tiles > (1 << 24)) return fail(kInvalidArgument, "gemm_split: T x M too large");
+    if (use_narrow(T, M))
+        return narrow_launch<kNarrowSplit>({reinterpret_cast<const uint8_t*>(wq), reinterpret_cast<const uint8_t*>(aq),
+                                            wsc, asc, c, (int)T, (int)M, (int)K, 0, 0}, st);
     const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);
     const size_t lds = 2 * (size_t)kSplitStage;
     const int rc = dynamic_lds((const void*)gemm_q8_split, lds);
@@ -782,6 +1095,9 @@ int gemm_q8_0_tiled_launch(const void* w_tiled, const void* a_tiled, float* c, i
         return fail(kInvalidArgument, "gemm_tiled: operands must be 16-byte aligned");
     const int64_t tiles_t = (T + kGemmTileA - 1) / kGemmTileA, n_tiles = tiles_t * ((M + kGemmTileW - 1) / kGemmTileW);
     if (n_tiles > (1 << 24)) return fail(kInvalidArgument, "gemm_tiled: T x M too large");
+    if (use_narrow(T, M) && K <= (1 << 24))  // a tile's bytes in 32 bits
+        return narrow_launch<kNarrowTiled>({static_cast<const uint8_t*>(w_tiled), static_cast<const uint8_t*>(a_tiled),
+                                            nullptr, nullptr, c, (int)T, (int)M, (int)K, 0, 0}, st);
     const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);
     hipLaunchKernelGGL((gemm_q8_0_tiled<kGemmTileA, kGemmTileW>), dim3(padded), dim3(kGemmTileA * kGemmTileW / 16), 0, st,
                        static_cast<const uint8_t*>(w_tiled), static_cast<const uint8_t*>(a_tiled), c, (int)T, (int)M,
