@@ -515,6 +515,27 @@ extern "C" int asmhip_matmul_swiglu(int qtype, const void* blocks, const float* 
     return matvec_swiglu_launch(qt, blocks, x, h, H, K, work, (hipStream_t)stream, o);
 }
 
+extern "C" int asmhip_matmul_rmsnorm(int qtype, const void* blocks, const float* x, const float* norm, float eps,
+                                     float* y, int64_t M, int64_t K, int swiglu, void* stream) {
+    QuantType qt;
+    int rc = check_ptrs(blocks, x, y);
+    if (!rc && !norm) rc = fail(kInvalidArgument, "null pointer argument");
+    if (!rc) rc = quant_type(qtype, &qt);
+    if (rc) return rc;
+    if (M <= 0 || K <= 0 || K % 32 || K > INT32_MAX || (swiglu && M % 16))
+        return fail(kInvalidArgument, "matvec_rmsnorm: need M, K > 0, K %% 32 == 0 and M %% 16 == 0 with swiglu");
+    MatvecOpts o;
+    o.pre = kPreRmsNorm;
+    o.pre_arg = norm;
+    o.eps = eps;
+    o.post = swiglu ? kPostSwiGlu8 : kPostNone;
+    const int bits = qt == QuantType::Q4_0 ? 4 : 8;
+    if (!matvec_rows_takes(bits, true, blocks, nullptr, nullptr, x, M, K, o))
+        return fail(kUnsupported, "matvec_rmsnorm: the row kernels do not take M=%lld K=%lld or its alignment",
+                    (long long)M, (long long)K);
+    return matvec_rows_launch(bits, true, blocks, nullptr, nullptr, x, y, M, K, (hipStream_t)stream, o);
+}
+
 extern "C" int asmhip_gemm_q8_0(const void* w_blocks, const void* a_blocks, float* c, int64_t T, int64_t M,
                                 int64_t K, void* stream) {
     int rc = check_ptrs(w_blocks, a_blocks, c);

@@ -30,8 +30,8 @@ stream, so it can be captured once into a HIP graph and replayed per token:
   * the KV cache is fp16, head-major [n_kv_heads][max_ctx][head_dim] per layer
     (the reference keeps fp32 [128][heads][head_dim], generate.py:252-253);
   * head_dim 48 (the reference's stories15M demo model, dim 288), 64 or 128;
-    where dim is not a multiple of 64 the RMSNorm runs as its own launch
-    before the matvec instead of inside it.
+    where dim is not a multiple of 64 the RMSNorm is fused by the row kernels'
+    own entry point (asmhip_matmul_rmsnorm).
 
 All weights are Q4_0 GGUF blocks, including the token embedding and the
 lm-head (generate.py:182-184 loads both through get_tensor).
@@ -186,10 +186,13 @@ class DecodeEngine:
         self.gu = DeviceBuffer(4 * 2 * s.hidden_dim)  # work buffer of asmhip_matmul_swiglu
         self.ffn = DeviceBuffer(4 * s.hidden_dim)     # silu(gate) * up
         self.logits = DeviceBuffer(4 * s.vocab)
-        # The matvecs fuse RMSNorm into their read of x when K % 64 == 0;
-        # otherwise (stories15M: dim 288) it runs as its own launch first.
+        # The matvecs fuse RMSNorm into their read of x: asmhip_matmul_fused and
+        # asmhip_matmul_swiglu when K % 64 == 0, otherwise (stories15M: dim 288)
+        # asmhip_matmul_rmsnorm.  Widths past its row kernels run the RMSNorm as its
+        # own launch first.
         self.fuse_norm = s.dim % 64 == 0
-        self.xn = None if self.fuse_norm else DeviceBuffer(4 * s.dim)
+        self.rows_norm = not self.fuse_norm and s.dim <= 16384
+        self.xn = None if self.fuse_norm or self.rows_norm else DeviceBuffer(4 * s.dim)
         ws = self.lib.asmhip_attention_decode_workspace(s.n_heads, s.head_dim, self.max_ctx)
         self.workspace = DeviceBuffer(4 * max(int(ws), 1))
         # cos/sin of every RoPE angle, formed once instead of in every attention launch
@@ -344,7 +347,12 @@ class DecodeEngine:
             check(L.asmhip_rmsnorm(self.x.ptr, norm.ptr, self.xn.ptr, d, eps, st), "rmsnorm")
             return self.xn.ptr, NONE, None
 
+        def rows_normed(norm, M, w, y, what, qtype=Q4, swiglu=0):
+            check(L.asmhip_matmul_rmsnorm(qtype, w.ptr, self.x.ptr, norm.ptr, eps, y, M, d, swiglu, st), what)
+
         def normed(norm, M, w, y, what, qtype=Q4):  # y = W rmsnorm(x; norm)
+            if self.rows_norm:
+                return rows_normed(norm, M, w, y, what, qtype)
             xin, pre, arg = norm_in(norm)
             mv(w, xin, y, M, d, pre, arg, 0, what, qtype)
 
@@ -355,6 +363,8 @@ class DecodeEngine:
                   "rope + attention")
 
         def gate_up(ly):
+            if self.rows_norm:
+                return rows_normed(ly.ffn_norm, 2 * h, ly.wgu, self.ffn.ptr, "gate/up matvec + swiglu", swiglu=1)
             xin, pre, arg = norm_in(ly.ffn_norm)
             check(L.asmhip_matmul_swiglu(Q4, ly.wgu.ptr, xin, self.ffn.ptr, h, d, pre, arg, eps, self.gu.ptr, st),
                   "gate/up matvec + swiglu")

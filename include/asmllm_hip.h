@@ -173,6 +173,15 @@ ASMHIP_API int asmhip_matmul_fused(int qtype, const void* blocks, const float* x
  * matvec then writes its 2H outputs there and a second launch combines them). */
 ASMHIP_API int asmhip_matmul_swiglu(int qtype, const void* blocks, const float* x, float* h, int64_t H, int64_t K,
                                     int pre_op, const float* pre_arg, float eps, float* work, void* stream);
+/* y = W rmsnorm(x; norm) in one launch for the widths whose RMSNorm asmhip_matmul_fused
+ * does not take, K % 64 == 32 included (generate.py:266-275 and 302-313 run
+ * asm_rmsnorm and then the matvecs): GGUF blocks (qtype Q4_0 or Q8_0) W [M][K/32].
+ * swiglu != 0: W's rows interleave gate and up in groups of 8 (M % 16 == 0) and
+ * h = silu(gate) * up is written instead, M / 2 floats, as asmhip_matmul_swiglu
+ * writes it.  y must not overlap x.  ASMHIP_ERR_UNSUPPORTED where the row kernels do
+ * not take the shape (K above about 21000, operands not 4-byte aligned). */
+ASMHIP_API int asmhip_matmul_rmsnorm(int qtype, const void* blocks, const float* x, const float* norm, float eps,
+                                     float* y, int64_t M, int64_t K, int swiglu, void* stream);
 /* Prefill GEMM: C[T][M] = sum over blocks b of int32 dot(A[t,b], W[j,b]) * d_w[j,b] * d_a[t,b],
  * accumulated in fp32 in block order; A = T activation rows and W = M weight rows, both
  * Q8_0 blocks [rows][K/32] (quantize activations with asmhip_quantize(ASMHIP_Q8_0, ...)).

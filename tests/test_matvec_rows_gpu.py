@@ -148,3 +148,40 @@ def test_row_kernels_merge_attention(hip, qt, n_heads, hd, max_ctx, pos, M):
              hip.asmhip_matmul_fused(qt, db.ptr, attn.ptr, d2.ptr, M, K, native.PRE_NONE, None, 0.0, 1, None)]
     assert calls == [0] * 5, hip.asmhip_last_error()
     assert np.array_equal(d1.download(np.uint32, (M,)), d2.download(np.uint32, (M,)))
+
+
+@pytest.mark.parametrize("q", [4, 8])
+@pytest.mark.parametrize("M,K", [(16, 32), (864, 288), (2096, 544), (64, 1056), (176, 4128), (32, 8224), (16400, 1056)])
+@pytest.mark.parametrize("swiglu", [0, 1])
+def test_row_kernels_rmsnorm_any_width(hip, q, M, K, swiglu):
+    rng = np.random.default_rng(M + K + q + 1)
+    b, w = _weights(rng, q, M, K)
+    x, g = (rng.standard_normal(K).astype(np.float32) for _ in range(2))
+    x64 = x.astype(np.float64)
+    xin = x64 / np.sqrt((x64 ** 2).mean() + 1e-5) * g.astype(np.float64)
+    db, dx, dg, dy = (DeviceBuffer.from_numpy(a) for a in (b, x, g, np.full(M, np.nan, np.float32)))
+    rc = hip.asmhip_matmul_rmsnorm(native.Q4_0 if q == 4 else native.Q8_0, db.ptr, dx.ptr, dg.ptr, 1e-5, dy.ptr, M, K,
+                                   swiglu, None)
+    assert rc == 0, hip.asmhip_last_error()
+    y, ref, bar = dy.download(np.float32, (M,)), w @ xin, _bar(w, xin, K)
+    if not swiglu:
+        assert np.all(np.abs(y - ref) <= bar)
+        return
+    gate, up = (ref.reshape(-1, 2, 8)[:, i].reshape(-1) for i in (0, 1))
+    bg, bu = (bar.reshape(-1, 2, 8)[:, i].reshape(-1) for i in (0, 1))
+    sg = gate / (1 + np.exp(-gate))
+    assert np.all(np.abs(y[: M // 2] - sg * up) <= 1.1 * bg * (np.abs(up) + bu) + np.abs(sg) * bu +
+                  2.0 ** -21 * np.abs(sg * up) + 1e-30)
+    assert np.all(np.isnan(y[M // 2:]))
+
+
+def test_row_kernels_rmsnorm_refusals(hip):
+    d = DeviceBuffer(1 << 16)
+    args = (d.ptr, d.ptr, d.ptr, 1e-5, d.ptr)
+    assert hip.asmhip_matmul_rmsnorm(native.Q4_0, *args, 16, 40, 0, None) == native.ERR_INVALID_ARGUMENT
+    assert hip.asmhip_matmul_rmsnorm(native.Q4_0, *args, 24, 32, 1, None) == native.ERR_INVALID_ARGUMENT
+    assert hip.asmhip_matmul_rmsnorm(native.Q4_0, *args, 16, 64000, 0, None) == native.ERR_UNSUPPORTED
+    assert hip.asmhip_matmul_rmsnorm(native.Q5_0, *args, 16, 32, 0, None) == native.ERR_INVALID_ARGUMENT
+    # the fused entry points keep refusing the widths they refused
+    assert hip.asmhip_matmul_fused(native.Q4_0, d.ptr, d.ptr, d.ptr, 16, 288, native.PRE_RMSNORM, d.ptr, 1e-5, 0,
+                                   None) == native.ERR_UNSUPPORTED
