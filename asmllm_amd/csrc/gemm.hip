@@ -705,8 +705,8 @@ __global__ __launch_bounds__(kSplitThreads) void gemm_q8_split(const int8_t* __r
 }
 
 // ---------------------------------------------------------------------------
-// Few rows of A: a workgroup of NW <= 4 waves computes 16 NW (T) x 16 (M) outputs, one
-// 16x16 tile a wave, so that a short prompt still reaches every compute unit (24 x 4096
+// Few rows of A: a workgroup computes NW <= 4 by MW <= 2 tiles of 16 (T) x 16 (M) outputs,
+// a wave each, so that a short prompt still reaches every compute unit (24 x 4096
 // x 4096: 32 workgroups of the 64 x 128 tile, 256 of these).  The same products in the
 // same order, so C keeps its bits:
 //   v_mfma_i32_16x16x32_i8    the block's int32 dots: lane l holds 8 of the 32 quants of
@@ -726,7 +726,7 @@ __global__ __launch_bounds__(kSplitThreads) void gemm_q8_split(const int8_t* __r
 // ---------------------------------------------------------------------------
 enum NarrowForm : int { kNarrowBlocks = 0, kNarrowTiled = 1, kNarrowSplit = 2 };
 
-template <int FORM, int NW>
+template <int FORM, int NW, int MW>
 struct Narrow {
     // blocks per step: 8, for runs of 256 or 272 bytes a row; the tile layout's runs are
     // whole at any step, and at four tiles four blocks leave room for four workgroups a
@@ -738,23 +738,25 @@ struct Narrow {
     // tile layout (68 bytes a row)
     static constexpr int kReal = FORM == kNarrowSplit ? 2 * B : (34 * B + 12 + 15) / 16, kPitchSlots = kReal + 1;
     static constexpr int kPitch = 16 * kPitchSlots;
-    static constexpr int kWSlots = FORM == kNarrowTiled ? B / 2 * 68 : 16 * kPitchSlots;
-    static constexpr int kWLoads = (kWSlots + 63) / 64, kALoads = (NW * kWSlots + 63) / 64;
+    static constexpr int kRowSlots = FORM == kNarrowTiled ? B / 2 * 68 : 16 * kPitchSlots;  // of 16 rows
+    static constexpr int kWLoads = (MW * kRowSlots + 63) / 64, kALoads = (NW * kRowSlots + 63) / 64;
     // split: the scales of 64 / B rows x B blocks a 4-byte load
-    static constexpr int kWSc = FORM == kNarrowSplit ? 16 * B / 64 : 0, kASc = kWSc * NW;
+    static constexpr int kSc16 = FORM == kNarrowSplit ? 16 * B / 64 : 0, kWSc = kSc16 * MW, kASc = kSc16 * NW;
     static constexpr int kLoads = kWLoads + kALoads + kWSc + kASc;  // wave-wide loads a step
     // up to two tiles leave whole SIMDs to waves that only load: a load costs its wave
     // about 30 cycles of issue, a quarter of a tile's step (5 rows 12.2 -> 10.3 us, split
     // 20.4 -> 10.2)
-    static constexpr int NL = NW <= 2 ? 4 - NW : 4, kFirst = NW <= 2 ? NW : 0, kThreads = 256;
+    static constexpr int kTiles = NW * MW, kWaves = kTiles < 4 ? 4 : kTiles;
+    static constexpr int kFirst = kTiles <= 2 ? kTiles : 0, NL = kWaves - kFirst, kThreads = kWaves * 64;
     static constexpr int kPerWave = (kLoads + NL - 1) / NL;
     static constexpr int kAOff = kWLoads * 1024, kScOff = kAOff + kALoads * 1024;
     static constexpr int kSpare = kScOff + (kWSc + kASc) * 256;     // landing place of padding loads
     static constexpr int kStage = kSpare + (kPerWave * NL > kLoads ? 1024 : 0);
     // three stages, two steps in flight: more (up to 150 KB) changed nothing where a
     // workgroup has a compute unit to itself and cost the others their company (24 x
-    // 11008 x 4096 37.7 us against 17.5)
-    static constexpr int S = 3;
+    // 11008 x 4096 37.7 us against 17.5); two where two columns of tiles share A, so that
+    // two such workgroups share a unit (200 x 4096 x 11008 split 71 us; 101 with three)
+    static constexpr int S = MW > 1 ? 2 : 3;
     static_assert((S - 1) * kPerWave < 64, "the wait counts to 63");
 };
 
@@ -773,16 +775,16 @@ __device__ __forceinline__ void wait_loads() {  // at most kCount of the wave's 
     __builtin_amdgcn_s_waitcnt(0xF70 | (kCount & 15) | ((kCount >> 4) << 14));
 }
 
-template <int FORM, int NW>
-__global__ __launch_bounds__(256) void gemm_narrow(const NarrowArgs g) {
-    using N = Narrow<FORM, NW>;
+template <int FORM, int NW, int MW>
+__global__ __launch_bounds__((Narrow<FORM, NW, MW>::kThreads)) void gemm_narrow(const NarrowArgs g) {
+    using N = Narrow<FORM, NW, MW>;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     // XCD-aware tile order, as gemm_q8_0_coalesced: T fastest
     const int chunk = (int)gridDim.x >> 3;
     const int tile = ((int)blockIdx.x & 7) * chunk + ((int)blockIdx.x >> 3);
     if (tile >= g.n_tiles) return;
     const int nb = g.K >> 5, nsteps = (nb + N::B - 1) / N::B;
-    const int t0 = (tile % g.tiles_t) * 16 * NW, j0 = (tile / g.tiles_t) * 16;
+    const int t0 = (tile % g.tiles_t) * 16 * NW, j0 = (tile / g.tiles_t) * 16 * MW;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t row_bytes = FORM == kNarrowSplit ? (uint32_t)g.K : (uint32_t)nb * 34u, sc_bytes = (uint32_t)nb * 4u;
@@ -811,12 +813,12 @@ __global__ __launch_bounds__(256) void gemm_narrow(const NarrowArgs g) {
             const bool is_w = j < N::kWLoads;
             const int q = 64 * (is_w ? j : j - N::kWLoads) + lane;
             if constexpr (FORM == kNarrowTiled) {
-                const int per = is_w ? 68 : 68 * NW, p = q / per;
+                const int per = 68 * (is_w ? MW : NW), p = q / per;
                 if (p < N::B / 2) o = (uint32_t)(p * (is_w ? kGemmTileW : kGemmTileA) * 68 + 16 * (q - p * per));
             } else {
                 const int r = q / N::kPitchSlots, k = q - r * N::kPitchSlots;
                 const int row = (is_w ? j0 : t0) + r;
-                if (r < (is_w ? 16 : 16 * NW) && k < N::kReal && row < (is_w ? g.M : g.T))
+                if (r < 16 * (is_w ? MW : NW) && k < N::kReal && row < (is_w ? g.M : g.T))
                     o = (((uint32_t)row * row_bytes) & ~15u) + 16u * (uint32_t)k;
             }
         } else if (j < N::kLoads) {
@@ -863,14 +865,14 @@ __global__ __launch_bounds__(256) void gemm_narrow(const NarrowArgs g) {
     [[maybe_unused]] const uint32_t first = grp ? 0u : ~0u;  // split: the scales of lane group 0
     // byte offsets of this lane's A and W rows in a stage (blocks: the row's data start
     // where its aligned window leaves them)
-    const int arow = 16 * wave + m;
-    int a_at = N::kAOff + arow * (FORM == kNarrowTiled ? 68 : N::kPitch), w_at = m * (FORM == kNarrowTiled ? 68 : N::kPitch);
+    const int arow = 16 * (wave % NW) + m, wrow = 16 * (wave / NW) + m;
+    int a_at = N::kAOff + arow * (FORM == kNarrowTiled ? 68 : N::kPitch), w_at = wrow * (FORM == kNarrowTiled ? 68 : N::kPitch);
     if constexpr (FORM == kNarrowBlocks) {
         a_at += (int)(((uint32_t)(t0 + arow) * row_bytes) & 15u);
-        w_at += (int)(((uint32_t)(j0 + m) * row_bytes) & 15u);
+        w_at += (int)(((uint32_t)(j0 + wrow) * row_bytes) & 15u);
     }
-    constexpr int kAPair = FORM == kNarrowTiled ? 1088 * NW : 68, kWPair = FORM == kNarrowTiled ? 1088 : 68;
-    const int as_at = N::kScOff + N::kWSc * 256 + arow * (4 * N::B), ws_at = N::kScOff + m * (4 * N::B);  // split scales
+    constexpr int kAPair = FORM == kNarrowTiled ? 1088 * NW : 68, kWPair = FORM == kNarrowTiled ? 1088 * MW : 68;
+    const int as_at = N::kScOff + N::kWSc * 256 + arow * (4 * N::B), ws_at = N::kScOff + wrow * (4 * N::B);  // split scales
 
     v4f acc = {0.f, 0.f, 0.f, 0.f};
     // block BLK of the pair at p (the lane's row of one operand): 8 quants and the scale
@@ -936,7 +938,7 @@ __global__ __launch_bounds__(256) void gemm_narrow(const NarrowArgs g) {
         // barrier; past the end the last step is loaded again
         if (loads) fetch(next, min(s + N::S - 1, nsteps - 1));
         const uint8_t* stage = lds + cur * N::kStage + (FORM == kNarrowBlocks ? (34 * N::B * s) & 15 : 0);
-        if (wave < NW) {
+        if (wave < N::kTiles) {
             // the step's operands, then its matrix instructions, then its sums: one block
             // after another a wave waited for each read, product and conversion in turn
             // (24 x 4096 x 4096 16.8 us against 13.2).  Blocks past the last add nothing.
@@ -968,27 +970,27 @@ __global__ __launch_bounds__(256) void gemm_narrow(const NarrowArgs g) {
         next = next + 1 == N::S ? 0 : next + 1;
     }
     wait_loads<0>();  // no wave ends with loads into LDS in flight
-    if (wave >= NW) return;
+    if (wave >= N::kTiles) return;
     // lane l, register i: row 4 (l / 16) + i, column l % 16
-    const int col = j0 + m;
+    const int col = j0 + wrow;
     if (col < g.M) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = t0 + 16 * wave + 4 * grp + i;
+            const int row = t0 + 16 * (wave % NW) + 4 * grp + i;
             if (row < g.T) g.c[(size_t)row * g.M + col] = FORM == kNarrowSplit ? acc[i] : 0.25f * acc[i];
         }
     }
 }
 
-template <int FORM, int NW>
+template <int FORM, int NW, int MW>
 int narrow_launch_nw(NarrowArgs g, hipStream_t st) {
-    using N = Narrow<FORM, NW>;
+    using N = Narrow<FORM, NW, MW>;
     g.tiles_t = (g.T + 16 * NW - 1) / (16 * NW);
-    const int64_t n = (int64_t)g.tiles_t * ((g.M + 15) / 16);
+    const int64_t n = (int64_t)g.tiles_t * ((g.M + 16 * MW - 1) / (16 * MW));
     g.n_tiles = (int)n;
-    const int rc = dynamic_lds((const void*)gemm_narrow<FORM, NW>, (size_t)N::S * N::kStage);
+    const int rc = dynamic_lds((const void*)gemm_narrow<FORM, NW, MW>, (size_t)N::S * N::kStage);
     if (rc) return rc;
-    hipLaunchKernelGGL((gemm_narrow<FORM, NW>), dim3((unsigned)((n + 7) / 8 * 8)), dim3(N::kThreads),
+    hipLaunchKernelGGL((gemm_narrow<FORM, NW, MW>), dim3((unsigned)((n + 7) / 8 * 8)), dim3(N::kThreads),
                        (size_t)N::S * N::kStage, st, g);
     ASMHIP_TRY(hipGetLastError());
     return kOk;
@@ -996,18 +998,25 @@ int narrow_launch_nw(NarrowArgs g, hipStream_t st) {
 
 template <int FORM>
 int narrow_launch(const NarrowArgs& g, hipStream_t st) {
-    if (g.T <= 16) return narrow_launch_nw<FORM, 1>(g, st);
-    if (g.T <= 32) return narrow_launch_nw<FORM, 2>(g, st);
-    if (g.T <= 48) return narrow_launch_nw<FORM, 3>(g, st);
-    return narrow_launch_nw<FORM, 4>(g, st);
+    if (g.T <= 16) return narrow_launch_nw<FORM, 1, 1>(g, st);
+    if (g.T <= 32) return narrow_launch_nw<FORM, 2, 1>(g, st);
+    if (g.T <= 48) return narrow_launch_nw<FORM, 3, 1>(g, st);
+    // two columns of tiles a workgroup once single ones would come to more than two a
+    // compute unit: 200 x 4096 x 11008 split 95 -> 71 us, blocks 77 either way; 128 x 4096 x
+    // 4096 (512 of them) 19.9 against 21.0, and the tile layout's are no faster
+    if (FORM != kNarrowTiled && (int64_t)((g.T + 63) / 64) * ((g.M + 15) / 16) > 512)
+        return narrow_launch_nw<FORM, 4, 2>(g, st);
+    return narrow_launch_nw<FORM, 4, 1>(g, st);
 }
 
-// While the 16-column workgroups come to at most four a compute unit: 24 x 4096 x 4096
-// blocks 32.5 -> 11.9 us, split 41.3 -> 12.0, tiled 26.8 -> 11.4; 200 x 4096 x 11008 (1024
-// of them) 84 -> 78, 122 -> 93, 69 -> 65.  Past that the larger tiles' fewer reads per
-// output win: 128 x 11008 x 4096 (1376) 37 / 50 / 28 us against 53 / 58 / 38.
-bool use_narrow(int64_t T, int64_t M) {
-    return (T + 63) / 64 * ((M + 15) / 16) <= 1024;
+// While the 16-column workgroups come to at most four a compute unit (six for the split
+// planes, whose larger tiles stage the slowest): 24 x 4096 x 4096 blocks 32.5 -> 11.9 us,
+// split 41.3 -> 12.0, tiled 26.8 -> 11.4; 200 x 4096 x 11008 (1024 of them) 84 -> 77, 122
+// -> 71, 69 -> 66; 128 x 11008 x 4096 split (1376) 50 -> 45.  Past that the larger tiles'
+// fewer reads per output win: 128 x 11008 x 4096 blocks 37 us against 45, tiled 28 / 39,
+// 512 x 4096 x 4096 split (2048) 48 / 55.
+bool use_narrow(int form, int64_t T, int64_t M) {
+    return (T + 63) / 64 * ((M + 15) / 16) <= (form == kNarrowSplit ? 1536 : 1024);
 }
 
 // Two blocks per staged K step, two steps of loads in flight per thread, at
@@ -1034,7 +1043,7 @@ int gemm_q8_0_launch(const void* w, const void* a, float* c, int64_t T, int64_t 
     if ((uintptr_t)w % 4 || (uintptr_t)a % 4) return fail(kInvalidArgument, "gemm: blocks must be 4-byte aligned");
     const dim3 grid((unsigned)((M + kTM - 1) / kTM), (unsigned)((T + kTT - 1) / kTT));
     if (grid.y > 65535) return fail(kInvalidArgument, "gemm: T too large");
-    if ((K / 32) % 2 == 0 && use_narrow(T, M) && ((uintptr_t)w | (uintptr_t)a) % 16 == 0)
+    if ((K / 32) % 2 == 0 && use_narrow(kNarrowBlocks, T, M) && ((uintptr_t)w | (uintptr_t)a) % 16 == 0)
         return narrow_launch<kNarrowBlocks>({static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(a), nullptr,
                                              nullptr, c, (int)T, (int)M, (int)K, 0, 0}, st);
     if ((K / 32) % kGemmKB == 0) {
@@ -1072,7 +1081,7 @@ int gemm_q8_split_launch(const int8_t* wq, const float* wsc, const int8_t* aq, c
         return fail(kInvalidArgument, "gemm_split: qs planes must be 16-byte aligned, scales 4-byte aligned");
     const int64_t tiles_t = (T + kTT - 1) / kTT, n_tiles = tiles_t * ((M + kTM - 1) / kTM);
     if (n_tiles > (1 << 24)) return fail(kInvalidArgument, "gemm_split: T x M too large");
-    if (use_narrow(T, M))
+    if (use_narrow(kNarrowSplit, T, M))
         return narrow_launch<kNarrowSplit>({reinterpret_cast<const uint8_t*>(wq), reinterpret_cast<const uint8_t*>(aq),
                                             wsc, asc, c, (int)T, (int)M, (int)K, 0, 0}, st);
     const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);
@@ -1095,7 +1104,7 @@ int gemm_q8_0_tiled_launch(const void* w_tiled, const void* a_tiled, float* c, i
         return fail(kInvalidArgument, "gemm_tiled: operands must be 16-byte aligned");
     const int64_t tiles_t = (T + kGemmTileA - 1) / kGemmTileA, n_tiles = tiles_t * ((M + kGemmTileW - 1) / kGemmTileW);
     if (n_tiles > (1 << 24)) return fail(kInvalidArgument, "gemm_tiled: T x M too large");
-    if (use_narrow(T, M) && K <= (1 << 24))  // a tile's bytes in 32 bits
+    if (use_narrow(kNarrowTiled, T, M) && K <= (1 << 24))  // a tile's bytes in 32 bits
         return narrow_launch<kNarrowTiled>({static_cast<const uint8_t*>(w_tiled), static_cast<const uint8_t*>(a_tiled),
                                             nullptr, nullptr, c, (int)T, (int)M, (int)K, 0, 0}, st);
     const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);

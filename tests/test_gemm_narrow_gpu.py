@@ -53,14 +53,16 @@ def _run(hip, form, w, a, T, M, K):
 @pytest.mark.parametrize("T,M,K", [
     (1, 1, 64), (5, 17, 192), (16, 100, 256), (17, 130, 320), (24, 15, 576), (32, 129, 64), (33, 16, 448), (48, 33, 1088),
     (49, 31, 128), (64, 130, 384), (65, 17, 704), (130, 250, 512), (200, 40, 1984), (3, 300, 4096), (40, 48, 2112),
+    (50, 8300, 64), (130, 2800, 576), (64, 8225, 192),  # two columns of tiles a workgroup
     (1, 16384, 64), (1, 16385, 64), (70, 8200, 128),  # 1024 workgroups, and the larger tiles from there
+    (65, 12288, 64), (65, 12289, 64),  # 1536, the split planes'
 ])
 def test_narrow_gemm_is_the_oracle(hip, oracle, form, T, M, K):
     w, a = _operands(T * 31 + M + K, T, M, K)
     np.testing.assert_array_equal(_run(hip, form, w, a, T, M, K), oracle.gemm_q8_0(w, a, 8))
 
 
-@pytest.mark.parametrize("T,M,K", [(5, 17, 32), (24, 40, 96), (50, 33, 544), (64, 20, 1120)])
+@pytest.mark.parametrize("T,M,K", [(5, 17, 32), (24, 40, 96), (50, 33, 544), (64, 20, 1120), (100, 4200, 96)])
 def test_narrow_gemm_odd_block_counts(hip, oracle, T, M, K):
     """The split planes take the narrow tiles at any K % 32; blocks keep the general kernel."""
     w, a = _operands(T + M + K, T, M, K)
