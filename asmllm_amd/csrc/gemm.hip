@@ -1000,7 +1000,9 @@ template <int FORM>
 int narrow_launch(const NarrowArgs& g, hipStream_t st) {
     if (g.T <= 16) return narrow_launch_nw<FORM, 1, 1>(g, st);
     if (g.T <= 32) return narrow_launch_nw<FORM, 2, 1>(g, st);
-    if (g.T <= 48) return narrow_launch_nw<FORM, 3, 1>(g, st);
+    // three tiles of rows leave the planes and the tile layout uneven loads, which four a compute
+    // unit feel: 40 x 9000 x 4096 is 12% slower with them than with four tiles, one of them idle
+    if (g.T <= 48 && (FORM == kNarrowBlocks || (g.M + 15) / 16 <= 512)) return narrow_launch_nw<FORM, 3, 1>(g, st);
     // two columns of tiles a workgroup once single ones would come to more than two a
     // compute unit: 200 x 4096 x 11008 split 95 -> 71 us, blocks 77 either way; 128 x 4096 x
     // 4096 (512 of them) 19.9 against 21.0, and the tile layout's are no faster
@@ -1009,14 +1011,20 @@ int narrow_launch(const NarrowArgs& g, hipStream_t st) {
     return narrow_launch_nw<FORM, 4, 1>(g, st);
 }
 
-// While the 16-column workgroups come to at most four a compute unit (six for the split
-// planes, whose larger tiles stage the slowest): 24 x 4096 x 4096 blocks 32.5 -> 11.9 us,
-// split 41.3 -> 12.0, tiled 26.8 -> 11.4; 200 x 4096 x 11008 (1024 of them) 84 -> 77, 122
-// -> 71, 69 -> 66; 128 x 11008 x 4096 split (1376) 50 -> 45.  Past that the larger tiles'
-// fewer reads per output win: 128 x 11008 x 4096 blocks 37 us against 45, tiled 28 / 39,
-// 512 x 4096 x 4096 split (2048) 48 / 55.
-bool use_narrow(int form, int64_t T, int64_t M) {
-    return (T + 63) / 64 * ((M + 15) / 16) <= (form == kNarrowSplit ? 1536 : 1024);
+// While the 16-column workgroups come to at most four a compute unit: 24 x 4096 x 4096 blocks
+// 32.5 -> 11.9 us, split 41.3 -> 12.0, tiled 26.8 -> 11.4; 200 x 4096 x 11008 (1024 of them)
+// blocks 84 -> 77, split 122 -> 71.  Three for the tile layout, whose larger kernel is the
+// fastest of the three (200 x 4096 x 1344: 11.2 us against 12.0, at 1024).  Where K is short the
+// first loads and the launch outweigh the K loop, and more workgroups than fit at once pay
+// them again: two a compute unit for blocks (200 x 4096 x 1344 13.1 us against 13.4, and from
+// K = 2048 on the narrow ones are 5-19% faster), three for 17 to 32 rows (20 x 14336 x 512 is 8-18% slower).  Past these
+// the larger tiles' fewer reads per output win: 128 x 11008 x 4096 blocks 37 us against 45,
+// tiled 28 / 39; 171 x 7003 x 1344 split (1314) 16.5 / 20.0.
+bool use_narrow(int form, int64_t T, int64_t M, int64_t K) {
+    const int64_t n = (T + 63) / 64 * ((M + 15) / 16);
+    if (T <= 32) return n <= (T <= 16 || K >= 2048 ? 1024 : 768);
+    if (form == kNarrowTiled) return n <= 768;
+    return n <= (form == kNarrowSplit || K >= 2048 ? 1024 : 512);
 }
 
 // Two blocks per staged K step, two steps of loads in flight per thread, at
@@ -1043,7 +1051,7 @@ int gemm_q8_0_launch(const void* w, const void* a, float* c, int64_t T, int64_t 
     if ((uintptr_t)w % 4 || (uintptr_t)a % 4) return fail(kInvalidArgument, "gemm: blocks must be 4-byte aligned");
     const dim3 grid((unsigned)((M + kTM - 1) / kTM), (unsigned)((T + kTT - 1) / kTT));
     if (grid.y > 65535) return fail(kInvalidArgument, "gemm: T too large");
-    if ((K / 32) % 2 == 0 && use_narrow(kNarrowBlocks, T, M) && ((uintptr_t)w | (uintptr_t)a) % 16 == 0)
+    if ((K / 32) % 2 == 0 && use_narrow(kNarrowBlocks, T, M, K) && ((uintptr_t)w | (uintptr_t)a) % 16 == 0)
         return narrow_launch<kNarrowBlocks>({static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(a), nullptr,
                                              nullptr, c, (int)T, (int)M, (int)K, 0, 0}, st);
     if ((K / 32) % kGemmKB == 0) {
@@ -1081,7 +1089,7 @@ int gemm_q8_split_launch(const int8_t* wq, const float* wsc, const int8_t* aq, c
         return fail(kInvalidArgument, "gemm_split: qs planes must be 16-byte aligned, scales 4-byte aligned");
     const int64_t tiles_t = (T + kTT - 1) / kTT, n_tiles = tiles_t * ((M + kTM - 1) / kTM);
     if (n_tiles > (1 << 24)) return fail(kInvalidArgument, "gemm_split: T x M too large");
-    if (use_narrow(kNarrowSplit, T, M))
+    if (use_narrow(kNarrowSplit, T, M, K))
         return narrow_launch<kNarrowSplit>({reinterpret_cast<const uint8_t*>(wq), reinterpret_cast<const uint8_t*>(aq),
                                             wsc, asc, c, (int)T, (int)M, (int)K, 0, 0}, st);
     const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);
@@ -1104,7 +1112,7 @@ int gemm_q8_0_tiled_launch(const void* w_tiled, const void* a_tiled, float* c, i
         return fail(kInvalidArgument, "gemm_tiled: operands must be 16-byte aligned");
     const int64_t tiles_t = (T + kGemmTileA - 1) / kGemmTileA, n_tiles = tiles_t * ((M + kGemmTileW - 1) / kGemmTileW);
     if (n_tiles > (1 << 24)) return fail(kInvalidArgument, "gemm_tiled: T x M too large");
-    if (use_narrow(kNarrowTiled, T, M) && K <= (1 << 24))  // a tile's bytes in 32 bits
+    if (use_narrow(kNarrowTiled, T, M, K) && K <= (1 << 24))  // a tile's bytes in 32 bits
         return narrow_launch<kNarrowTiled>({static_cast<const uint8_t*>(w_tiled), static_cast<const uint8_t*>(a_tiled),
                                             nullptr, nullptr, c, (int)T, (int)M, (int)K, 0, 0}, st);
     const unsigned padded = (unsigned)((n_tiles + 7) / 8 * 8);

@@ -55,7 +55,10 @@ def _run(hip, form, w, a, T, M, K):
     (49, 31, 128), (64, 130, 384), (65, 17, 704), (130, 250, 512), (200, 40, 1984), (3, 300, 4096), (40, 48, 2112),
     (50, 8300, 64), (130, 2800, 576), (64, 8225, 192),  # two columns of tiles a workgroup
     (1, 16384, 64), (1, 16385, 64), (70, 8200, 128),  # 1024 workgroups, and the larger tiles from there
-    (65, 12288, 64), (65, 12289, 64),  # 1536, the split planes'
+    (17, 12288, 64), (17, 12289, 64), (17, 16384, 2048),  # 768 for 17 to 32 rows of a short K
+    (65, 6144, 64), (65, 6145, 64),  # 768, the tile layout's
+    (65, 4096, 64), (65, 4097, 64), (65, 8192, 2048), (65, 8193, 2048),  # 512 blocks, 1024 from K = 2048
+    (40, 8192, 64), (40, 8193, 64), (40, 8300, 2048),  # three tiles of rows, and four with one idle
 ])
 def test_narrow_gemm_is_the_oracle(hip, oracle, form, T, M, K):
     w, a = _operands(T * 31 + M + K, T, M, K)
