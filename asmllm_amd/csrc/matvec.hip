@@ -11,6 +11,11 @@
 // Byte j of a Q4 block holds weight j in its low nibble and weight j+16 in its
 // high nibble (matmul_q4_avx2.asm:122-153, tests/reference/ops.py:24-28).
 //
+// The dispatch at the end sends a shape to the int8-MFMA stream (matvec_mfma.hip), to
+// the row kernels (matvec_rows.hip), or here: the pair kernels take rows too long for
+// the row kernels' LDS (K above about 21000, K % 64 == 0), the generic ones everything
+// else (operands without 4-byte alignment, x too large for LDS).
+//
 // Work mapping (one wave = 64 lanes):
 //   * a lane owns one PAIR of consecutive blocks (64 columns) of a 64-pair
 //     column chunk, so a wave's loads for one row cover a contiguous
@@ -306,8 +311,8 @@ __global__ __launch_bounds__(kThreads) void q8_matvec_pairs(const uint8_t* __res
 
 // ---------------------------------------------------------------------------
 // Generic kernel: one wave per row, one block per lane, byte loads.  Covers
-// what the pair kernels do not (odd K/32, rows not dword aligned, x too large
-// for LDS).  Correct for every K % 32 == 0, not tuned.
+// what the others do not (operands not dword aligned, x too large for LDS).
+// Correct for every K % 32 == 0, not tuned.
 // ---------------------------------------------------------------------------
 template <bool kQ8, bool kGguf>
 __global__ __launch_bounds__(kThreads) void matvec_generic(const uint8_t* __restrict__ w,

@@ -64,7 +64,7 @@ extern "C" {
  * keeps Q5_0 and Q8_0 on the fp32 kernels.  The MFMA stream needs
  * K % 256 == 0, K <= 16384 and 16-byte aligned x (and, for split planes,
  * 16-byte aligned planes). */
-#define ASMHIP_Q4_KERNEL_AUTO 0 /* int8 MFMA kernel where eligible, else fp32             */
+#define ASMHIP_Q4_KERNEL_AUTO 0 /* int8 MFMA kernel where eligible and K > 1024, else fp32 */
 #define ASMHIP_Q4_KERNEL_FP32 1 /* fp32 VALU kernel only                                   */
 #define ASMHIP_Q4_KERNEL_MFMA 2 /* int8 MFMA kernel only (GGUF shapes it cannot take:
                                    UNSUPPORTED; split planes fall back to fp32) */
@@ -169,8 +169,9 @@ ASMHIP_API int asmhip_matmul_fused(int qtype, const void* blocks, const float* x
  * (rows 16g..16g+7 = gate rows 8g..8g+7, rows 16g+8..16g+15 = up rows 8g..8g+7;
  * H % 8 == 0), and h[j] = gate_j / (1 + exp(-gate_j)) * up_j, with x
  * transformed by pre_op as in asmhip_matmul_fused.  work: 2H floats of device
- * memory, written only where the int8-MFMA stream cannot take the shape (the
- * matvec then writes its 2H outputs there and a second launch combines them). */
+ * memory, written only where neither the int8-MFMA stream nor the row kernels take
+ * the shape, or h overlaps x (the matvec then writes its 2H outputs there and a
+ * second launch combines them). */
 ASMHIP_API int asmhip_matmul_swiglu(int qtype, const void* blocks, const float* x, float* h, int64_t H, int64_t K,
                                     int pre_op, const float* pre_arg, float eps, float* work, void* stream);
 /* y = W rmsnorm(x; norm) in one launch for the widths whose RMSNorm asmhip_matmul_fused
@@ -299,11 +300,12 @@ ASMHIP_API int asmhip_attention_decode_rope_table(const float* qkv, void* k_cach
  * (asmhip_attention_decode_workspace() floats, 16-byte aligned).
  * asmhip_matmul_attn_output then computes y = W . attn (accumulate: y += W .
  * attn) for GGUF blocks W [M][n_heads * head_dim / 32] (qtype Q4_0 or Q8_0),
- * where attn is the merged attention output: for Q4_0 where the int8-MFMA
- * stream takes the shape (head_dim 64 or 128, n_heads * head_dim a multiple of
- * 256 and at most 8192, max_ctx <= 4096) the merge runs inside the matvec's
- * read of x; otherwise a merge launch writes attn to `work` (n_heads *
- * head_dim floats) and a matvec reads it.  Results equal the merge launch + asmhip_matmul_fused, bit for bit.
+ * where attn is the merged attention output.  The merge runs inside the matvec's
+ * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024,
+ * and for Q4_0 where the int8-MFMA stream takes the shape (head_dim 64 or 128, n_heads
+ * * head_dim a multiple of 256 and at most 8192); otherwise a merge launch writes attn
+ * to `work` (n_heads * head_dim floats) and a matvec reads it.  Results equal the
+ * merge launch + asmhip_matmul_fused, bit for bit.
  * `workspace` and `max_ctx` must be those of the attention call. */
 ASMHIP_API int asmhip_attention_decode_partials_rope_table(const float* qkv, void* k_cache, void* v_cache,
                                                            float* workspace, int n_heads, int n_kv_heads,
