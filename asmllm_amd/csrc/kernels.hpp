@@ -87,12 +87,16 @@ int split_mfma_launch(int bits, const void* qs, const uint8_t* qh, const float* 
 
 // The fp32 row kernels over GGUF blocks or split planes (bits = 4, 5 or 8; qh for
 // split Q5, scales for split): any K % 32 == 0 whose x fits LDS, 4-byte aligned
-// operands, every pre-op and post-op (kPreAttnMerge: K <= kSmallK; kPostSwiGlu8: M %
+// operands, every pre-op and post-op (kPreAttnMerge: rows_before_stream; kPostSwiGlu8: M %
 // 16).  Up to kSmallK they are also faster than the int8-MFMA stream, whose units of
 // 256 columns then leave 12 of its 16 waves idle (Q4_0 288 x 768 3.1 -> 2.3 us, 1536 x
 // 768 3.2 -> 2.5, 32000 x 256 6.9 -> 4.5; at K = 1536 from 4096 rows on it is not: 3.5
 // against 3.7).
+// Past 512 columns only up to 6144 rows (6000 x 1024 Q4_0 4% faster, 8192 x 1024 2% slower,
+// 16384 x 768 9%).  A wave holds whole rows there, whose 64-bit sums leave less error than
+// the stream's integers and fp32 sums.
 constexpr int kSmallK = 1024;
+inline bool rows_before_stream(int64_t M, int64_t K) { return K <= 512 || (K <= kSmallK && M <= 6144); }
 bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const float* scales, const float* x,
                        int64_t M, int64_t K, const MatvecOpts& opts);
 int matvec_rows_launch(int bits, bool gguf, const void* w, const uint8_t* qh, const float* scales, const float* x,

@@ -23,6 +23,7 @@
 // Bound by the read of the weights and, at the smallest shapes, by the chain x ->
 // barrier -> dot -> reduction -> store of one workgroup.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -317,6 +318,24 @@ __device__ __forceinline__ T load_at(const uint8_t* p) {  // any 2-byte aligned 
     return v;
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+    return v + __longlong_as_double((long long)hi << 32 | (uint32_t)lo);
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)hi << 32 | (uint32_t)lo);
+}
+__device__ __forceinline__ double wave_total_dpp(double v) {
+    v = dpp_add<kDppQuadXor1>(v), v = dpp_add<kDppQuadXor2>(v);
+    v = dpp_add<kDppRowHalfMirror>(v), v = dpp_add<kDppRowMirror>(v);
+    return ((lane_value(v, 0) + lane_value(v, 16)) + lane_value(v, 32)) + lane_value(v, 48);
+}
+
 template <int QT, bool GGUF, int NP, int R, int W>
 __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
     static_assert(W == 1 || W == kWaveThreads / 64, "a wave or the workgroup per row");
@@ -417,7 +436,10 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
     float tot[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        float acc = 0.f;
+        // a wave per row (K <= 1024) adds its fours of products in 64 bits: in fp32 throughout
+        // the error was 1.5 times the int8-MFMA stream's (15122 x 256 8.4e-8 against 5.6e-8
+        // of the result's norm), so it is 4.7e-8, for 0.1 us at 288 x 288 and 0.7 at 32000 x 288
+        std::conditional_t<W == 1, double, float> acc = 0;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
             uint32_t lo, hi;
@@ -432,16 +454,26 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
                 hi = ((q[r][p][0] >> 1) & 0x78787878u) | (spread_bits(nh, 4) & 0x80808080u);
             }
             lo = opaque(lo), hi = opaque(hi);
-            float t = 0.f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                t = fmaf(sbyte(lo, k), x[p][k], t);
-                t = fmaf(sbyte(hi, k), x[p][4 + k], t);
-            }
             const float d = GGUF ? half_lo(sc[r][p]) : __uint_as_float(sc[r][p]);
-            acc = live[p] ? fmaf(d, t, acc) : acc;
+            if constexpr (W == 1) {
+                float t0 = 0.f, t1 = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    t0 = fmaf(sbyte(lo, k), x[p][k], t0);
+                    t1 = fmaf(sbyte(hi, k), x[p][4 + k], t1);
+                }
+                acc = live[p] ? fma((double)d, (double)t0 + (double)t1, acc) : acc;
+            } else {
+                float t = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    t = fmaf(sbyte(lo, k), x[p][k], t);
+                    t = fmaf(sbyte(hi, k), x[p][4 + k], t);
+                }
+                acc = live[p] ? fmaf(d, t, acc) : acc;
+            }
         }
-        tot[r] = wave_total_dpp(acc);
+        tot[r] = (float)wave_total_dpp(acc);
     }
     if constexpr (W > 1) {  // the waves' parts of K meet in LDS, added in order
         __shared__ float red[R + 1][W];
@@ -590,8 +622,8 @@ bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const
                                : bits == 5 ? RowsUnit<kRows5, true, 1>::kSlot : RowsUnit<kRows4, true, 1>::kSlot;
     const size_t lds = (size_t)nb * kXPitch * 4 + (size_t)kWaves * (slot + 64 * 4);
     // the merge runs in every wave that reads x: small K only
-    if (o.pre == kPreAttnMerge && (K > kSmallK || o.attn_splits < 1 || o.attn_splits > kAttnMergeMaxSplits ||
-                                   o.attn_hd <= 0 || o.attn_hd % 4 || K % o.attn_hd || (uintptr_t)o.pre_arg % 16))
+    if (o.pre == kPreAttnMerge && (!rows_before_stream(M, K) || o.attn_splits < 1 ||
+                                   o.attn_splits > kAttnMergeMaxSplits || o.attn_hd <= 0 || o.attn_hd % 4 || K % o.attn_hd || (uintptr_t)o.pre_arg % 16))
         return false;
     return K > 0 && K % 32 == 0 && M > 0 && M <= INT32_MAX - 4096 && bytes < (int64_t)kPastEnd && lds <= kLdsBudget &&
            (uintptr_t)w % 4 == 0 && (gguf || ((uintptr_t)scales % 4 == 0 && (uintptr_t)qh % 4 == 0)) &&

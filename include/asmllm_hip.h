@@ -64,7 +64,7 @@ extern "C" {
  * keeps Q5_0 and Q8_0 on the fp32 kernels.  The MFMA stream needs
  * K % 256 == 0, K <= 16384 and 16-byte aligned x (and, for split planes,
  * 16-byte aligned planes). */
-#define ASMHIP_Q4_KERNEL_AUTO 0 /* int8 MFMA kernel where eligible and K > 1024, else fp32 */
+#define ASMHIP_Q4_KERNEL_AUTO 0 /* int8 MFMA kernel where eligible and K > 1024 (K > 512 past 6144 rows), else fp32 */
 #define ASMHIP_Q4_KERNEL_FP32 1 /* fp32 VALU kernel only                                   */
 #define ASMHIP_Q4_KERNEL_MFMA 2 /* int8 MFMA kernel only (GGUF shapes it cannot take:
                                    UNSUPPORTED; split planes fall back to fp32) */
@@ -301,7 +301,8 @@ ASMHIP_API int asmhip_attention_decode_rope_table(const float* qkv, void* k_cach
  * asmhip_matmul_attn_output then computes y = W . attn (accumulate: y += W .
  * attn) for GGUF blocks W [M][n_heads * head_dim / 32] (qtype Q4_0 or Q8_0),
  * where attn is the merged attention output.  The merge runs inside the matvec's
- * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024,
+ * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024
+ * (512 past 6144 rows),
  * and for Q4_0 where the int8-MFMA stream takes the shape (head_dim 64 or 128, n_heads
  * * head_dim a multiple of 256 and at most 8192); otherwise a merge launch writes attn
  * to `work` (n_heads * head_dim floats) and a matvec reads it.  Results equal the

@@ -59,7 +59,7 @@ def _call(hip, q, split, b, x, M, K):
 
 SHAPES = [(1, 32), (5, 64), (17, 96), (300, 288), (700, 512), (33, 544), (2100, 768), (63, 1024), (520, 1056),
           (70, 2080), (2100, 2080), (3, 4128), (600, 5504), (40, 8160), (24, 8224), (20, 16416), (9, 21024),
-          (9000, 288), (17000, 544)]
+          (9000, 288), (17000, 544), (6145, 768)]
 
 
 @pytest.mark.parametrize("q", [4, 5, 8])
@@ -75,6 +75,20 @@ def test_row_kernels_shapes(hip, q, split, M, K):
         one = np.zeros(K, np.float32)
         one[col] = 1.0
         assert np.array_equal(_call(hip, q, split, b, one, M, K).astype(np.float64), w[:, col])
+
+
+@pytest.mark.parametrize("q", [4, 5, 8])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("M,K", [(1, 32), (300, 288), (9000, 512), (6144, 768), (2100, 1024)])
+def test_row_kernels_sums_in_64_bits(hip, q, split, M, K):
+    """Up to 1024 columns only fours of products round in 32 bits (four fused multiply-adds of
+    at most u each), and the result."""
+    rng = np.random.default_rng(M + K + q)
+    b, w = _weights(rng, q, M, K)
+    x = rng.standard_normal(K).astype(np.float32)
+    y, e, u = _call(hip, q, split, b, x, M, K), w @ x.astype(np.float64), 2.0 ** -24
+    bar = 4.01 * u * (np.abs(w) @ np.abs(x).astype(np.float64)) + 1.01 * u * np.abs(e) + 1e-30
+    assert (np.abs(y - e) <= bar).all()
 
 
 @pytest.mark.parametrize("M,K", [(4096, 5504), (16400, 2080), (5000, 8224)])
@@ -123,7 +137,7 @@ def test_row_kernels_fused(hip, q, M, K, pre, form):
 
 
 @pytest.mark.parametrize("qt", [native.Q4_0, native.Q8_0])
-@pytest.mark.parametrize("n_heads,hd,max_ctx,pos,M", [(6, 48, 256, 100, 288), (6, 48, 3072, 3000, 288), (2, 64, 900, 899, 70),
+@pytest.mark.parametrize("n_heads,hd,max_ctx,pos,M", [(6, 48, 256, 100, 288), (6, 48, 3072, 3000, 288), (2, 64, 900, 899, 70), (6, 128, 256, 100, 6144), (6, 128, 256, 100, 6145),
                                                        (8, 128, 770, 5, 1024), (16, 64, 3072, 1, 3000)])
 def test_row_kernels_merge_attention(hip, qt, n_heads, hd, max_ctx, pos, M):
     """The split states merged by the o matvec give the bits of the merge launch and
