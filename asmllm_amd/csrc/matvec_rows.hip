@@ -330,7 +330,7 @@ __device__ __forceinline__ double lane_value(double v, int l) {
     const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
     return __longlong_as_double((long long)hi << 32 | (uint32_t)lo);
 }
-__device__ __forceinline__ double wave_total_dpp(double v) {
+__device__ __forceinline__ double wave_total64(double v) {
     v = dpp_add<kDppQuadXor1>(v), v = dpp_add<kDppQuadXor2>(v);
     v = dpp_add<kDppRowHalfMirror>(v), v = dpp_add<kDppRowMirror>(v);
     return ((lane_value(v, 0) + lane_value(v, 16)) + lane_value(v, 32)) + lane_value(v, 48);
@@ -473,7 +473,10 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
                 acc = live[p] ? fmaf(d, t, acc) : acc;
             }
         }
-        tot[r] = (float)wave_total_dpp(acc);
+        if constexpr (W == 1)
+            tot[r] = (float)wave_total64(acc);
+        else
+            tot[r] = wave_total_dpp(acc);
     }
     if constexpr (W > 1) {  // the waves' parts of K meet in LDS, added in order
         __shared__ float red[R + 1][W];
