@@ -762,14 +762,16 @@ int matvec_swiglu_launch(QuantType qt, const void* w, const float* x, float* h, 
     po.post = kPostSwiGlu8;
     const int64_t M = 2 * H;
     const int sel = g_q4_kernel.load(std::memory_order_relaxed), bits = qt == QuantType::Q4_0 ? 4 : 8;
+    // One launch only where h touches neither x nor the pre-op's argument: its workgroups
+    // write h while others still read both.  The two launches below write h last.
+    auto apart = [&](const float* in) { return h + H <= in || in + K <= h; };
+    const bool one = apart(x) && (opts.pre == kPreNone || apart(opts.pre_arg));
     // the row kernels combine the pairs of a shape that their plain launch takes too
-    // (h over x: only the two launches below read all of x before they write h)
-    const bool apart = h + H <= x || x + K <= h;
-    const bool rows = apart && (opts.pre == kPreNone || (opts.pre <= kPreSwiGlu && K % 64 == 0)) &&
+    const bool rows = one && (opts.pre == kPreNone || (opts.pre <= kPreSwiGlu && K % 64 == 0)) &&
                       matvec_rows_takes(bits, true, w, nullptr, nullptr, x, M, K, po);
     if (rows && rows_before_stream(M, K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
         return matvec_rows_launch(bits, true, w, nullptr, nullptr, x, h, M, K, stream, po);
-    if (sel != kQ4KernelFp32) {
+    if (one && sel != kQ4KernelFp32) {
         if (qt == QuantType::Q4_0 && q4_0_mfma_eligible(w, x, po, M, K)) return q4_0_mfma_launch(w, x, h, M, K, stream, po);
         if (qt == QuantType::Q8_0 && q8_0_mfma_eligible(w, x, po, M, K)) return q8_0_mfma_launch(w, x, h, M, K, stream, po);
     }

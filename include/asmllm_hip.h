@@ -170,8 +170,8 @@ ASMHIP_API int asmhip_matmul_fused(int qtype, const void* blocks, const float* x
  * H % 8 == 0), and h[j] = gate_j / (1 + exp(-gate_j)) * up_j, with x
  * transformed by pre_op as in asmhip_matmul_fused.  work: 2H floats of device
  * memory, written only where neither the int8-MFMA stream nor the row kernels take
- * the shape, or h overlaps x (the matvec then writes its 2H outputs there and a
- * second launch combines them). */
+ * the shape, or h overlaps x or the pre-op's pre_arg (the matvec then writes its 2H
+ * outputs there and a second launch combines them). */
 ASMHIP_API int asmhip_matmul_swiglu(int qtype, const void* blocks, const float* x, float* h, int64_t H, int64_t K,
                                     int pre_op, const float* pre_arg, float eps, float* work, void* stream);
 /* y = W rmsnorm(x; norm) in one launch for the widths whose RMSNorm asmhip_matmul_fused

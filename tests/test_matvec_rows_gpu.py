@@ -189,6 +189,35 @@ def test_row_kernels_rmsnorm_any_width(hip, q, M, K, swiglu):
     assert np.all(np.isnan(y[M // 2:]))
 
 
+@pytest.mark.parametrize("qt", [native.Q4_0, native.Q8_0])
+@pytest.mark.parametrize("H,K", [(296, 320), (1024, 1088), (2048, 2048), (520, 4096)])
+@pytest.mark.parametrize("pre,over", [("none", "x")] + [(p, o) for p in ("rmsnorm", "swiglu") for o in ("x", "arg", "arg's end")])
+def test_swiglu_over_its_inputs(hip, qt, H, K, pre, over):
+    """h over x or over the pre-op's argument: the pairs go through `work`, so that no
+    workgroup writes what another still reads, with the bits of the call into a buffer
+    of its own (which leaves `work` alone)."""
+    rng = np.random.default_rng(H + K)
+    b, _ = _weights(rng, 4 if qt == native.Q4_0 else 8, 2 * H, K)
+    op = {"none": native.PRE_NONE, "rmsnorm": native.PRE_RMSNORM, "swiglu": native.PRE_SWIGLU}[pre]
+    n = max(H, K) + K
+    x, arg = (rng.standard_normal(n).astype(np.float32) for _ in range(2))
+    db, dh = DeviceBuffer.from_numpy(b), DeviceBuffer(4 * H)
+
+    def call(target):
+        dx, da = DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(arg)
+        work = DeviceBuffer.from_numpy(np.full(2 * H, np.nan, np.float32))
+        buf, offset = {"own": (dh, 0), "x": (dx, 0), "arg": (da, 0), "arg's end": (da, 4 * (K - 1))}[target]
+        rc = hip.asmhip_matmul_swiglu(qt, db.ptr, dx.ptr, buf.ptr + offset, H, K, op, da.ptr if op else None, 1e-5,
+                                      work.ptr, None)
+        assert rc == 0, hip.asmhip_last_error()
+        return buf.download(np.uint32, (H,), offset=offset), work.download(np.float32, (2 * H,))
+
+    own, untouched = call("own")
+    y, work = call(over)
+    assert np.isnan(untouched).all() and not np.isnan(work).any()
+    assert np.array_equal(y, own)
+
+
 def test_row_kernels_rmsnorm_refusals(hip):
     d = DeviceBuffer(1 << 16)
     args = (d.ptr, d.ptr, d.ptr, 1e-5, d.ptr)
