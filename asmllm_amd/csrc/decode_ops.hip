@@ -444,9 +444,11 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float* __rest
         for (int r = 0; r < R; ++r) fold(sc[r], vr[b][r]);
     }
     if (has_new) {
-        const float d = score(kq), s = w == 0 && g == 0 ? d : -INFINITY;
+        // not with a weight of 0 by the others: v may have rounded to an infinity
+        const bool owner = w == 0 && g == 0;
+        const float d = score(kq), s = owner ? d : -INFINITY;
         grow(s);
-        fold(s, vq);
+        if (owner) fold(s, vq);
     }
     // every lane group's softmax state to LDS (no cross-lane shuffles), then one
     // merge over all groups of the workgroup in group order; thread t < HD owns

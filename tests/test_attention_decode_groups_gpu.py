@@ -56,3 +56,38 @@ def test_attention_groups_and_splits(hip, n_heads, n_kv, hd, max_ctx, pos, rope)
         ref = p @ v / p.sum()
         e = (hd + 4) * 2.0 ** -24 * (np.abs(k) @ np.abs(q[h])).max() / np.sqrt(hd)
         assert np.all(np.abs(y[h] - ref) <= (2 * e + (pos + 80) * 2.0 ** -24) * np.abs(v).max())
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,max_ctx,pos", [
+    (4, 4, 64, 300, 100), (8, 2, 128, 300, 299), (6, 3, 48, 400, 0), (6, 6, 128, 5000, 4000),
+])
+@pytest.mark.parametrize("rope", [False, True])
+def test_attention_new_row_past_fp16(hip, n_heads, n_kv, hd, max_ctx, pos, rope):
+    """A v element at the current position that rounds to an fp16 infinity gives that
+    infinity in its own dimension and leaves the others' bits alone."""
+    rng = np.random.default_rng(hd + pos)
+    qkv = rng.standard_normal((n_heads + 2 * n_kv) * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal((n_kv, max_ctx, hd)).astype(np.float16) for _ in range(2))
+    dpos = DeviceBuffer.from_numpy(np.array([pos], np.int32))
+    ws = DeviceBuffer(hip.asmhip_attention_decode_workspace(n_heads, hd, max_ctx) * 4)
+    table = DeviceBuffer(4 * max_ctx * hd)
+    assert hip.asmhip_rope_table(table.ptr, hd, max_ctx, 10000.0, None) == 0
+
+    def run(a, b):
+        new, cache = qkv.copy(), vc.copy()
+        v = new[(n_heads + n_kv) * hd:].reshape(n_kv, hd)
+        v[:, 3], v[:, hd - 1] = a, b
+        with np.errstate(over="ignore"):
+            cache[:, pos] = v.astype(np.float16)
+        dq, dk, dv = (DeviceBuffer.from_numpy(t) for t in (new, kc.view(np.uint16), cache.view(np.uint16)))
+        out = DeviceBuffer(4 * n_heads * hd)
+        args = (dq.ptr, dk.ptr, dv.ptr, ws.ptr, out.ptr, n_heads, n_kv, hd, dpos.ptr, max_ctx)
+        rc = (hip.asmhip_attention_decode_rope_table(*args, table.ptr, None) if rope
+              else hip.asmhip_attention_decode(*args, None))
+        assert rc == 0, hip.asmhip_last_error()
+        return out.download(np.float32, (n_heads, hd))
+
+    y, plain = run(1e5, -7e4), run(1.0, 1.0)
+    assert np.all(y[:, 3] == np.inf) and np.all(y[:, hd - 1] == -np.inf)
+    rest = np.setdiff1d(np.arange(hd), [3, hd - 1])
+    assert np.array_equal(y[:, rest].view(np.uint32), plain[:, rest].view(np.uint32))
