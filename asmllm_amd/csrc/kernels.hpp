@@ -199,6 +199,7 @@ constexpr int attn_split_len(int max_ctx) {
     return max_ctx <= kAttnMergeMaxSplits * kAttnSplitShort ? kAttnSplitShort : kAttnSplitLong;
 }
 constexpr int kAttnPartStride(int hd) { return hd + 4; }
+constexpr bool attn_head_dim(int hd) { return hd == 48 || hd == 64 || hd == 128; }  // what the decode attention takes
 int attn_decode_splits(int max_ctx);
 int64_t attn_decode_workspace(int n_heads, int hd, int max_ctx);
 // rope_table (optional, with rope): [max_ctx][hd] floats from rope_table_launch,

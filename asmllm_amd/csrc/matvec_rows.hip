@@ -624,9 +624,10 @@ bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const
     const int slot = bits == 8 ? RowsUnit<kRows8, true, 1>::kSlot
                                : bits == 5 ? RowsUnit<kRows5, true, 1>::kSlot : RowsUnit<kRows4, true, 1>::kSlot;
     const size_t lds = (size_t)nb * kXPitch * 4 + (size_t)kWaves * (slot + 64 * 4);
-    // the merge runs in every wave that reads x: small K only
-    if (o.pre == kPreAttnMerge && (!rows_before_stream(M, K) || o.attn_splits < 1 ||
-                                   o.attn_splits > kAttnMergeMaxSplits || o.attn_hd <= 0 || o.attn_hd % 4 || K % o.attn_hd || (uintptr_t)o.pre_arg % 16))
+    // the merge runs in every wave that reads x: small K only, and the head_dims of the merge launch
+    if (o.pre == kPreAttnMerge &&
+        (!rows_before_stream(M, K) || o.attn_splits < 1 || o.attn_splits > kAttnMergeMaxSplits ||
+         !attn_head_dim(o.attn_hd) || K % o.attn_hd || (uintptr_t)o.pre_arg % 16))
         return false;
     return K > 0 && K % 32 == 0 && M > 0 && M <= INT32_MAX - 4096 && bytes < (int64_t)kPastEnd && lds <= kLdsBudget &&
            (uintptr_t)w % 4 == 0 && (gguf || ((uintptr_t)scales % 4 == 0 && (uintptr_t)qh % 4 == 0)) &&

@@ -139,3 +139,15 @@ def test_single_workgroup_ops_refuse_lengths_near_int_max():
     for name, call in calls.items():
         assert call() == -1, name
         assert name in native.last_error(), (name, native.last_error())
+
+
+def test_attention_output_refuses_other_head_dims():
+    """Head_dims that the decode attention never leaves partials for are refused before
+    anything is launched (the pointers below are never dereferenced), but for Q4_0 heads
+    of whole 32-blocks, which the MFMA stream's merge takes."""
+    lib = native.lib()
+    p = ctypes.c_void_p(256)
+    for qt, n_heads, hd in ((native.Q8_0, 8, 32), (native.Q8_0, 3, 96), (native.Q4_0, 9, 32), (native.Q4_0, 8, 80)):
+        rc = lib.asmhip_matmul_attn_output(qt, p, p, p, p, 64, n_heads, hd, 256, 0, None)
+        assert rc == native.ERR_UNSUPPORTED, (qt, n_heads, hd, native.last_error())
+        assert "head_dim" in native.last_error()
