@@ -529,6 +529,8 @@ extern "C" int asmhip_matmul_rmsnorm(int qtype, const void* blocks, const float*
     o.pre_arg = norm;
     o.eps = eps;
     o.post = swiglu ? kPostSwiGlu8 : kPostNone;
+    if (qt == QuantType::Q4_0 && get_q4_kernel() == kQ4KernelMfma)
+        return fail(kUnsupported, "matvec_rmsnorm: the MFMA Q4_0 kernel is selected, and only the row kernels take this call");
     const int bits = qt == QuantType::Q4_0 ? 4 : 8;
     if (!matvec_rows_takes(bits, true, blocks, nullptr, nullptr, x, M, K, o))
         return fail(kUnsupported, "matvec_rmsnorm: the row kernels do not take M=%lld K=%lld or its alignment",

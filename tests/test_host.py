@@ -151,3 +151,16 @@ def test_attention_output_refuses_other_head_dims():
         rc = lib.asmhip_matmul_attn_output(qt, p, p, p, p, 64, n_heads, hd, 256, 0, None)
         assert rc == native.ERR_UNSUPPORTED, (qt, n_heads, hd, native.last_error())
         assert "head_dim" in native.last_error()
+
+
+def test_matmul_rmsnorm_obeys_the_kernel_selection():
+    """Under the MFMA-only selection a Q4_0 call that only the row kernels take is
+    refused before anything is launched, as asmhip_matmul_q4_0 refuses K = 288."""
+    lib = native.lib()
+    p = ctypes.c_void_p(256)
+    assert lib.asmhip_set_q4_kernel(native.Q4_KERNEL_MFMA) == 0
+    try:
+        assert lib.asmhip_matmul_q4_0(p, p, p, 288, 288, None) == native.ERR_UNSUPPORTED
+        assert lib.asmhip_matmul_rmsnorm(native.Q4_0, p, p, p, 1e-5, p, 288, 288, 0, None) == native.ERR_UNSUPPORTED
+    finally:
+        lib.asmhip_set_q4_kernel(native.Q4_KERNEL_AUTO)
