@@ -31,7 +31,8 @@ stream, so it can be captured once into a HIP graph and replayed per token:
     (the reference keeps fp32 [128][heads][head_dim], generate.py:252-253);
   * head_dim 48 (the reference's stories15M demo model, dim 288), 64 or 128;
     where dim is not a multiple of 64 the RMSNorm is fused by the row kernels'
-    own entry point (asmhip_matmul_rmsnorm).
+    own entry point (asmhip_matmul_rmsnorm), or runs as its own launch where
+    they refuse the matrix.
 
 All weights are Q4_0 GGUF blocks, including the token embedding and the
 lm-head (generate.py:182-184 loads both through get_tensor).
@@ -188,11 +189,10 @@ class DecodeEngine:
         self.logits = DeviceBuffer(4 * s.vocab)
         # The matvecs fuse RMSNorm into their read of x: asmhip_matmul_fused and
         # asmhip_matmul_swiglu when K % 64 == 0, otherwise (stories15M: dim 288)
-        # asmhip_matmul_rmsnorm.  Widths past its row kernels run the RMSNorm as its
-        # own launch first.
+        # asmhip_matmul_rmsnorm.  Where its row kernels refuse a matrix (of 4 GB, or too
+        # wide) the RMSNorm runs as its own launch into xn first.
         self.fuse_norm = s.dim % 64 == 0
-        self.rows_norm = not self.fuse_norm and s.dim <= 16384
-        self.xn = None if self.fuse_norm or self.rows_norm else DeviceBuffer(4 * s.dim)
+        self.xn = None if self.fuse_norm else DeviceBuffer(4 * s.dim)
         ws = self.lib.asmhip_attention_decode_workspace(s.n_heads, s.head_dim, self.max_ctx)
         self.workspace = DeviceBuffer(4 * max(int(ws), 1))
         # cos/sin of every RoPE angle, formed once instead of in every attention launch
@@ -347,12 +347,18 @@ class DecodeEngine:
             check(L.asmhip_rmsnorm(self.x.ptr, norm.ptr, self.xn.ptr, d, eps, st), "rmsnorm")
             return self.xn.ptr, NONE, None
 
-        def rows_normed(norm, M, w, y, what, qtype=Q4, swiglu=0):
-            check(L.asmhip_matmul_rmsnorm(qtype, w.ptr, self.x.ptr, norm.ptr, eps, y, M, d, swiglu, st), what)
+        def rows_normed(norm, M, w, y, what, qtype=Q4, swiglu=0):  # False: not the row kernels' shape
+            if self.fuse_norm:
+                return False
+            rc = L.asmhip_matmul_rmsnorm(qtype, w.ptr, self.x.ptr, norm.ptr, eps, y, M, d, swiglu, st)
+            if rc == native.ERR_UNSUPPORTED:
+                return False
+            check(rc, what)
+            return True
 
         def normed(norm, M, w, y, what, qtype=Q4):  # y = W rmsnorm(x; norm)
-            if self.rows_norm:
-                return rows_normed(norm, M, w, y, what, qtype)
+            if rows_normed(norm, M, w, y, what, qtype):
+                return
             xin, pre, arg = norm_in(norm)
             mv(w, xin, y, M, d, pre, arg, 0, what, qtype)
 
@@ -363,8 +369,8 @@ class DecodeEngine:
                   "rope + attention")
 
         def gate_up(ly):
-            if self.rows_norm:
-                return rows_normed(ly.ffn_norm, 2 * h, ly.wgu, self.ffn.ptr, "gate/up matvec + swiglu", swiglu=1)
+            if rows_normed(ly.ffn_norm, 2 * h, ly.wgu, self.ffn.ptr, "gate/up matvec + swiglu", swiglu=1):
+                return
             xin, pre, arg = norm_in(ly.ffn_norm)
             check(L.asmhip_matmul_swiglu(Q4, ly.wgu.ptr, xin, self.ffn.ptr, h, d, pre, arg, eps, self.gu.ptr, st),
                   "gate/up matvec + swiglu")

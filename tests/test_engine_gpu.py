@@ -94,6 +94,36 @@ def test_decode_steps_match_oracle(shape, embed_type, output_type):
     eng.close()
 
 
+@pytest.mark.parametrize("refused", ["all", "lm_head"])
+def test_steps_where_the_row_kernels_refuse_the_rmsnorm(refused):
+    """A matrix that asmhip_matmul_rmsnorm refuses (4 GB, say) at a width that
+    asmhip_matmul_fused does not normalise: the RMSNorm launch and the matvec."""
+    class Refusing:
+        def __init__(self, lib):
+            self.lib, self.refusals = lib, 0
+
+        def __getattr__(self, name):
+            return getattr(self.lib, name)
+
+        def asmhip_matmul_rmsnorm(self, *args):
+            if refused == "lm_head" and args[6] != STORIES_15M.vocab:
+                return self.lib.asmhip_matmul_rmsnorm(*args)
+            self.refusals += 1
+            return native.ERR_UNSUPPORTED
+
+    eng = DecodeEngine(STORIES_15M, max_ctx=48, output_type=native.Q8_0)
+    eng.init_random(seed=7)
+    eng.lib = Refusing(eng.lib)
+    ref = _oracle_model(eng, nt=4)
+    token = 5
+    for pos in (29, 30):
+        got, want = eng.forward_token(token, pos), ref.forward_token(token, pos)
+        _check_logits(got, want, f"pos {pos}")
+        token = int(np.argmax(want))
+    assert eng.lib.refusals == 2 * (1 if refused == "lm_head" else 2 * STORIES_15M.n_layers + 1)
+    eng.close()
+
+
 def test_graph_replay_matches_eager_launches():
     shape = SMALL[0]
     eng = DecodeEngine(shape, max_ctx=64)
