@@ -25,12 +25,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_at(const float* x, int b,
     return make_rsrc(x + (size_t)b * 16 * hd, (uint32_t)(seq - 16 * b) * (uint32_t)hd * 4u);
 }
 
-// The online softmax of one query, in powers of two: p = 2^(s - m) for scores s =
-// q.k * scale * log2(e).  m follows the maximum only when it has grown by more than
-// kSlack (weights up to 2^kSlack cost no precision in fp32, and the rescaling of the
-// sums is left out for all but a wave's first block as a rule).  base stands for m
-// while every score so far is -inf: such scores then weigh 0, and a NaN stays one.
-constexpr float kSlack = 10.f;
+// The online softmax of one query, in powers of two: p = 2^-kSlack 2^(s - m) for scores
+// s = q.k * scale * log2(e).  m follows the maximum only when it has grown by more than
+// kSlack (the rescaling of the sums is left out for all but a wave's first block as a
+// rule), so that a weight is at most 1 and the sums reach no further than the values do;
+// the power of two costs no precision.  base stands for m while every score so far is
+// -inf: such scores then weigh 0, and a NaN stays one.
+constexpr float kSlack = 10.f, kUnit = 0x1p-10f;
 __device__ __forceinline__ float base_of(float m) { return m == -INFINITY ? 0.f : m; }
 
 // The merge of NW softmax states of one row, a quad of dimensions: state w is
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
         const float base = base_of(m);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            p[i] = exp2_fast(p[i] - base);
+            p[i] = exp2_fast(p[i] - base) * kUnit;
             l += p[i];
         }
 #pragma unroll
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
         const float base = base_of(m);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            p[i] = exp2_fast(p[i] - base);
+            p[i] = exp2_fast(p[i] - base) * kUnit;
             l += p[i];
         }
 #pragma unroll

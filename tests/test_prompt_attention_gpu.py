@@ -77,3 +77,17 @@ def test_attention_infinite_scores(hip, hd):
     k[:, 0] = 1.0
     k[77, 3] = np.nan
     assert np.all(np.isnan(_run(hip, q, k, v, 0.5)))
+
+
+@pytest.mark.parametrize("seq,hd", [(64, 64), (600, 128), (1100, 64), (1100, 48), (40, 30)])
+def test_attention_values_near_the_largest_float(hip, seq, hd):
+    """Weights stay at most 1 while later keys' scores rise above the first ones', so
+    values whose sum over the keys is a third of the largest float come through."""
+    rng = np.random.default_rng(seq + hd)
+    q, k = np.zeros((seq, hd), np.float32), np.zeros((seq, hd), np.float32)
+    q[:, 0] = 1.0
+    k[:, 0] = np.linspace(0, 6.8, seq)  # 9.8 in powers of two
+    v = (rng.uniform(0.5, 1.0, (seq, hd)) * 1e38 / seq).astype(np.float32)
+    y = _run(hip, q, k, v, 1.0)
+    assert np.isfinite(y).all()
+    assert np.all(np.abs(y - _ref(q, k, v, 1.0)) <= _bound(q, k, v, 1.0))
