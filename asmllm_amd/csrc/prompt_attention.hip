@@ -55,7 +55,7 @@ __device__ __forceinline__ v4f merge_states(const float* acc, const float* m, co
 
 // A wave's 16 keys of NJ 16-dimension groups in LDS: loaded with four consecutive
 // lanes on 64 bytes of a row (lane l: key l / 4, quads 4 j + l % 4), written and read
-// back by the same wave (LDS operations of a wave complete in order, so no barrier).
+// back by the same wave (wave_lds_order, no barrier).
 // Quad p of key r stands at p ^ fold(r), where fold spreads eight consecutive lanes
 // over the banks on both sides: consecutive keys differ in bit 2 (the write: two keys
 // of four quads), and the read's eight keys in all three bits (SPREAD 8: lanes on keys
@@ -159,6 +159,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
 #pragma unroll
             for (int u = 0; u < NU; ++u) vv[u][i] = load4(vr, voff[u][i]);
         if (b + NW < nblk) load_k(b + NW);
+        wave_lds_order();
         v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;  // two chains: consecutive steps do not wait for each other
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -168,6 +169,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
             s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[2], qv[j][2], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[3], qv[j][3], s1, 0, 0, 0);
         }
+        wave_lds_order();  // the next block's K takes the tile
         float p[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[i] = (s0[i] + s1[i]) * scale;
@@ -303,6 +305,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
         for (int n = 0; n < NV; ++n) vv[n] = load4(vr, voff[n]);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) *reinterpret_cast<v4f*>(tile + put.at(j)) = kv[j];
+        wave_lds_order();
         v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -312,6 +315,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
             s0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kk[2], qv[j][2], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_4x4x1f32(kk[3], qv[j][3], s1, 0, 0, 0);
         }
+        wave_lds_order();  // the next block's K takes the tile
         float p[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[i] = add_row_slices(s0[i] + s1[i]) * scale;
