@@ -12,7 +12,7 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kRowPastEnd = 0xFFFFFF00u;  // buffer offset that loads zeros
+constexpr uint32_t kRowPastEnd = 0x80000000u;  // buffer offset that loads zeros, with room for a block's rows above it
 
 __device__ __forceinline__ v4f load4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     const uint4 u = buf_load_b128(r, off);
@@ -25,17 +25,22 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_at(const float* x, int b,
     return make_rsrc(x + (size_t)b * 16 * hd, (uint32_t)(seq - 16 * b) * (uint32_t)hd * 4u);
 }
 
-// The online softmax of one query, in powers of two: p = 2^-kSlack 2^(s - m) for scores
-// s = q.k * scale * log2(e).  m follows the maximum only when it has grown by more than
-// kSlack (the rescaling of the sums is left out for all but a wave's first block as a
-// rule), so that a weight is at most 1 and the sums reach no further than the values do;
-// the power of two costs no precision.  base stands for m while every score so far is
-// -inf: such scores then weigh 0, and a NaN stays one.
+// The online softmax of one query, in powers of two: p = 2^-kSlack 2^(s scale - base),
+// base = m scale, for scores s = q.k and scale > 0 (log2(e) included; q takes its sign).
+// m follows the maximum of s only when that has grown by more than kSlack / scale (the
+// rescaling of the sums is left out for all but a wave's first block as a rule), so that
+// a weight is at most 1 and the sums reach no further than the values do; the power of
+// two costs no precision.  base is 0 while every score so far is -inf: such scores then
+// weigh 0, and a NaN stays one.
 constexpr float kSlack = 10.f, kUnit = 0x1p-10f;
 __device__ __forceinline__ float base_of(float m) { return m == -INFINITY ? 0.f : m; }
+__device__ __forceinline__ float scaled(float m, float scale) {  // one rounding wherever it is used: never part of an fma
+#pragma clang fp contract(off)
+    return m * scale;
+}
 
 // The merge of NW softmax states of one row, a quad of dimensions: state w is
-// acc[w * stride], m[w * n], l[w * n].
+// acc[w * stride], m[w * n] (times scale), l[w * n].
 template <int NW>
 __device__ __forceinline__ v4f merge_states(const float* acc, const float* m, const float* l, int stride, int n) {
     float M = -INFINITY;
@@ -55,7 +60,7 @@ __device__ __forceinline__ v4f merge_states(const float* acc, const float* m, co
 
 // A wave's 16 keys of NJ 16-dimension groups in LDS: loaded with four consecutive
 // lanes on 64 bytes of a row (lane l: key l / 4, quads 4 j + l % 4), written and read
-// back by the same wave (wave_lds_order, no barrier).
+// back by the same wave (LDS operations of a wave complete in order, so no barrier).
 // Quad p of key r stands at p ^ fold(r), where fold spreads eight consecutive lanes
 // over the banks on both sides: consecutive keys differ in bit 2 (the write: two keys
 // of four quads), and the read's eight keys in all three bits (SPREAD 8: lanes on keys
@@ -68,6 +73,10 @@ struct KTile {
     static __device__ __forceinline__ int fold(int r) {
         return ((r & 1) << 2) | (SPREAD == 8 ? (r >> 1) & 3 : r & 2);
     }
+    // The compiler sees one lane: a reader hides its offsets from it, so that it never
+    // finds them apart from the lane's own writes and reorders the two (a fence between
+    // them also held V's loads back, 1024 x 128 15.6 -> 16.0 us).
+    __device__ __forceinline__ void hide() { asm("" : "+v"(even), "+v"(odd)); }
     // byte offset of quad 4 j + s of key r, as two bases (even and odd j) and 64 j
     int even, odd;
     __device__ __forceinline__ KTile(int r, int s) {
@@ -114,7 +123,9 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
     const uint32_t row_bytes = (uint32_t)hd * 4u;
     using KT = KTile<NJ, 8>;
     uint8_t* tile = reinterpret_cast<uint8_t*>(smem) + wave * KT::kBytes;
-    const KT put(lane >> 2, lane & 3), get(c, g);
+    const KT put(lane >> 2, lane & 3);
+    KT get(c, g);
+    get.hide();
     // offsets within a block's rows; dimensions past head_dim are sent past the end
     auto off = [&](int row, int d) { return FULL || d < hd ? (uint32_t)row * row_bytes + 4u * (uint32_t)d : kRowPastEnd; };
     uint32_t koff[NJ], voff[NU][4];
@@ -146,8 +157,12 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
     for (int u = 0; u < NU; ++u)
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[u][t] = v4f{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    scale *= 1.44269504088896340736f;
+    float m = -INFINITY, ms = m, l = 0.f;  // ms: m scale
+    const float sign = scale < 0.f ? -1.f : scale == 0.f ? 0.f : 1.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) qv[j] *= sign;
+    scale = scale == 0.f ? 1.f : fabsf(scale) * 1.44269504088896340736f;
+    const float slack = kSlack / scale;
 
     for (int b = wave; b < nblk; b += NW) {
         const auto vr = rows_at(v, b, seq, hd);
@@ -159,7 +174,6 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
 #pragma unroll
             for (int u = 0; u < NU; ++u) vv[u][i] = load4(vr, voff[u][i]);
         if (b + NW < nblk) load_k(b + NW);
-        wave_lds_order();
         v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;  // two chains: consecutive steps do not wait for each other
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -169,30 +183,29 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
             s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[2], qv[j][2], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[3], qv[j][3], s1, 0, 0, 0);
         }
-        wave_lds_order();  // the next block's K takes the tile
         float p[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] = (s0[i] + s1[i]) * scale;
+        for (int i = 0; i < 4; ++i) p[i] = s0[i] + s1[i];
         if (16 * b + 16 > seq) {  // the last block: keys past the end weigh nothing
 #pragma unroll
             for (int i = 0; i < 4; ++i) p[i] = 16 * b + 4 * g + i < seq ? p[i] : -INFINITY;
         }
         float mb = fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3]));
-        if (__any(mb > m + kSlack || m == -INFINITY)) {
+        if (__any(mb > m + slack || m == -INFINITY)) {
             mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
             mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
-            const float mn = fmaxf(m, mb), f = exp2_fast(m - base_of(mn));
-            m = mn;
+            const float mn = fmaxf(m, mb), msn = scaled(mn, scale), f = exp2_fast(ms - base_of(msn));
+            m = mn, ms = msn;
             l *= f;
 #pragma unroll
             for (int u = 0; u < NU; ++u)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) acc[u][t] *= f;
         }
-        const float base = base_of(m);
+        const float base = base_of(ms);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            p[i] = exp2_fast(p[i] - base) * kUnit;
+            p[i] = exp2_fast(fmaf(p[i], scale, -base)) * kUnit;
             l += p[i];
         }
 #pragma unroll
@@ -217,7 +230,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
         for (int i = 0; i < 4; ++i)  // row r = 4 g + i of the tiles: dimensions 64 u + 4 r + t
             *reinterpret_cast<v4f*>(mine + 64 * u + 16 * g + 4 * i) =
                 v4f{acc[u][0][i], acc[u][1][i], acc[u][2][i], acc[u][3][i]};
-    if (g == 0) sm_m[wave * 16 + c] = m, sm_l[wave * 16 + c] = l;
+    if (g == 0) sm_m[wave * 16 + c] = ms, sm_l[wave * 16 + c] = l;
     __syncthreads();
     constexpr int kQuads = 16 * HDP / 4;  // output quads, in row order
     for (int e = threadIdx.x; e < kQuads; e += NW * 64) {
@@ -273,16 +286,16 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
     const uint32_t row_bytes = (uint32_t)hd * 4u;
     using KT = KTile<NJ, 4>;
     uint8_t* tile = reinterpret_cast<uint8_t*>(smem) + wave * KT::kBytes;
-    const KT put(lane >> 2, lane & 3), get(4 * row + qi, (lane >> 2) & 3);
+    const KT put(lane >> 2, lane & 3);
+    KT get(4 * row + qi, (lane >> 2) & 3);
+    get.hide();
     auto off = [&](int r, int d) { return FULL || d < hd ? (uint32_t)r * row_bytes + 4u * (uint32_t)d : kRowPastEnd; };
-    uint32_t koff[NJ], voff[NV];
+    uint32_t koff[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) koff[j] = off(lane >> 2, 16 * j + 4 * (lane & 3));
     // load n of V: at HDP = 64 key 4 (l / 16) + n, at 128 key 8 (l / 32) + n
     const int vkey = HDP == 64 ? 4 * row : 8 * (lane >> 5), vdim = 4 * (lane % (HDP / 4));
-#pragma unroll
-    for (int n = 0; n < NV; ++n)
-        voff[n] = vdim < hd ? (uint32_t)(vkey + n) * row_bytes + 4u * (uint32_t)vdim : kRowPastEnd;
+    const uint32_t voff0 = vdim < hd ? (uint32_t)vkey * row_bytes + 4u * (uint32_t)vdim : kRowPastEnd;
     v4f qv[NJ];
     const int nblk = (seq + 15) >> 4;
     {
@@ -293,19 +306,26 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
     v4f acc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f, lo, hi;
-    scale *= 1.44269504088896340736f;
+    float m = -INFINITY, ms = m, l = 0.f, lo, hi;  // ms: m scale
+    const float sign = scale < 0.f ? -1.f : scale == 0.f ? 0.f : 1.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) qv[j] *= sign;
+    scale = scale == 0.f ? 1.f : fabsf(scale) * 1.44269504088896340736f;
+    const float slack = kSlack / scale;
 
     for (int b = wave; b < nblk; b += NW) {
         const auto kr = rows_at(k, b, seq, hd), vr = rows_at(v, b, seq, hd);
         v4f kv[NJ], vv[NV];
+        // the rows' offsets formed anew in every block where head_dim is no constant: eight
+        // of them kept in registers went to scratch memory (head_dim 116, 1000 rows 14.4 us, 13.6 so)
+        uint32_t voff = voff0;
+        if (!FULL) asm("" : "+v"(voff));
 #pragma unroll
         for (int j = 0; j < NJ; ++j) kv[j] = load4(kr, koff[j]);
 #pragma unroll
-        for (int n = 0; n < NV; ++n) vv[n] = load4(vr, voff[n]);
+        for (int n = 0; n < NV; ++n) vv[n] = load4(vr, voff + (uint32_t)n * row_bytes);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) *reinterpret_cast<v4f*>(tile + put.at(j)) = kv[j];
-        wave_lds_order();
         v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -315,29 +335,28 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
             s0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kk[2], qv[j][2], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_4x4x1f32(kk[3], qv[j][3], s1, 0, 0, 0);
         }
-        wave_lds_order();  // the next block's K takes the tile
         float p[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] = add_row_slices(s0[i] + s1[i]) * scale;
+        for (int i = 0; i < 4; ++i) p[i] = add_row_slices(s0[i] + s1[i]);
         if (16 * b + 16 > seq) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) p[i] = 16 * b + 4 * row + i < seq ? p[i] : -INFINITY;
         }
         float mb = fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3]));
-        if (__any(mb > m + kSlack || m == -INFINITY)) {
+        if (__any(mb > m + slack || m == -INFINITY)) {
             row_pair(mb, &lo, &hi);
             mb = fmaxf(lo, hi);
             half_pair(mb, &lo, &hi);
-            const float mn = fmaxf(m, fmaxf(lo, hi)), f = exp2_fast(m - base_of(mn));
-            m = mn;
+            const float mn = fmaxf(m, fmaxf(lo, hi)), msn = scaled(mn, scale), f = exp2_fast(ms - base_of(msn));
+            m = mn, ms = msn;
             l *= f;
 #pragma unroll
             for (int t = 0; t < 4; ++t) acc[t] *= f;
         }
-        const float base = base_of(m);
+        const float base = base_of(ms);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            p[i] = exp2_fast(p[i] - base) * kUnit;
+            p[i] = exp2_fast(fmaf(p[i], scale, -base)) * kUnit;
             l += p[i];
         }
 #pragma unroll
@@ -383,7 +402,7 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
         for (int i = 0; i < 4; ++i)
             *reinterpret_cast<v4f*>(mine + 4 * i) = v4f{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
     }
-    if (lane < 4) sm_m[wave * 4 + lane] = m, sm_l[wave * 4 + lane] = l;
+    if (lane < 4) sm_m[wave * 4 + lane] = ms, sm_l[wave * 4 + lane] = l;
     __syncthreads();
     if (threadIdx.x < HDP) {  // 4 rows x HDP / 4 quads
         const int r = threadIdx.x / (HDP / 4), d = 4 * (threadIdx.x % (HDP / 4));

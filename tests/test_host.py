@@ -164,3 +164,28 @@ def test_matmul_rmsnorm_obeys_the_kernel_selection():
         assert lib.asmhip_matmul_rmsnorm(native.Q4_0, p, p, p, 1e-5, p, 288, 288, 0, None) == native.ERR_UNSUPPORTED
     finally:
         lib.asmhip_set_q4_kernel(native.Q4_KERNEL_AUTO)
+
+
+def test_no_kernel_uses_scratch_memory(tmp_path):
+    """Registers that do not fit go to scratch memory without a warning: no kernel of the
+    built objects has any."""
+    import re
+    import subprocess
+    from pathlib import Path
+
+    from asmllm_amd import build
+
+    tools = Path("/opt/rocm/llvm/bin")
+    objects = sorted(build.OBJ_DIR.glob("*.o"))
+    if not objects or not (tools / "clang-offload-bundler").exists():
+        pytest.skip("the objects of a build or the LLVM tools missing")
+    kernels = {}
+    for o in objects:
+        bundle, code = tmp_path / (o.name + ".bundle"), tmp_path / (o.name + ".code")
+        subprocess.run([tools / "llvm-objcopy", f"--dump-section=.hip_fatbin={bundle}", o, tmp_path / "copy.o"], check=True)
+        subprocess.run([tools / "clang-offload-bundler", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
+                        f"--input={bundle}", f"--output={code}", "--unbundle"], check=True)
+        notes = subprocess.run([tools / "llvm-readelf", "--notes", code], capture_output=True, text=True, check=True).stdout
+        kernels.update(re.findall(r"\.name:\s+(\S+)\n\s+\.private_segment_fixed_size: (\d+)", notes))
+    assert len(kernels) > 100
+    assert [k for k, n in kernels.items() if n != "0"] == []

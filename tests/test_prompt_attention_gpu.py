@@ -91,3 +91,11 @@ def test_attention_values_near_the_largest_float(hip, seq, hd):
     y = _run(hip, q, k, v, 1.0)
     assert np.isfinite(y).all()
     assert np.all(np.abs(y - _ref(q, k, v, 1.0)) <= _bound(q, k, v, 1.0))
+
+
+@pytest.mark.parametrize("seq,hd", [(300, 128), (1100, 64)])
+@pytest.mark.parametrize("scale", [-0.25, 0.0, 1e-30])
+def test_attention_scale_of_any_sign(hip, seq, hd, scale):
+    rng = np.random.default_rng(seq)
+    q, k, v = (rng.standard_normal((seq, hd)).astype(np.float32) for _ in range(3))
+    assert np.all(np.abs(_run(hip, q, k, v, scale) - _ref(q, k, v, scale)) <= _bound(q, k, v, abs(scale)))
