@@ -720,7 +720,7 @@ extern "C" int asmhip_matmul_attn_output(int qtype, const void* blocks, const fl
     o.attn_hd = head_dim;
     // one launch where the matvec kernel of the shape takes the merge as its x prologue
     const int bits = qt == QuantType::Q4_0 ? 4 : 8, sel = get_q4_kernel();
-    if (rows_before_stream(M, K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0) &&
+    if (rows_before_stream(K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0) &&
         matvec_rows_takes(bits, true, blocks, nullptr, nullptr, workspace, M, K, o))
         return matvec_rows_launch(bits, true, blocks, nullptr, nullptr, workspace, y, M, K, st, o);
     if (sel != kQ4KernelFp32) {

@@ -79,6 +79,15 @@ __device__ __forceinline__ float half_hi(uint32_t v) {
     return __half2float(__ushort_as_half((unsigned short)(v >> 16)));
 }
 
+// Between one wave's LDS writes and its reads of what other lanes wrote (or those reads
+// and the next writes): no instruction, LDS operations of a wave complete in order, but
+// the compiler, which sees one lane, keeps them in order too.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Sum over the 64 lanes of a wave; every lane gets the total.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -14,14 +14,14 @@ enum class QuantType { Q4_0, Q8_0 };
 // whether y is overwritten or accumulated into.
 enum PreOp : int {
     kPreNone = 0,
-    kPreRmsNorm = 1,  // x <- (x * 1/sqrt(mean(x^2) + eps)) * arg[k] (the MFMA stream: W (x * arg)
+    kPreRmsNorm = 1,  // x <- (x * 1/sqrt(mean(x^2) + eps)) * arg[k] (the MFMA stream and the row kernels: W (x * arg)
                       // scaled by the 1/sqrt factor per row, which needs no barrier before x's digits)
     kPreSwiGlu = 2,   // x <- x / (1 + exp(-x)) * arg[k]
     // x is the decode attention output, merged from its split partials: arg is
     // the [n_heads][attn_splits][kAttnPartStride(attn_hd)] workspace that
     // attn_decode_launch(..., out = nullptr) filled, K = n_heads * attn_hd
-    // (x itself is not read).  Q4_0 int8-MFMA stream only, attn_splits <=
-    // kAttnMergeMaxSplits.
+    // (x itself is not read).  The row kernels up to kSmallK columns and the Q4_0
+    // int8-MFMA stream, attn_splits <= kAttnMergeMaxSplits.
     kPreAttnMerge = 3,
 };
 
@@ -88,15 +88,14 @@ int split_mfma_launch(int bits, const void* qs, const uint8_t* qh, const float* 
 // The fp32 row kernels over GGUF blocks or split planes (bits = 4, 5 or 8; qh for
 // split Q5, scales for split): any K % 32 == 0 whose x fits LDS, 4-byte aligned
 // operands, every pre-op and post-op (kPreAttnMerge: rows_before_stream; kPostSwiGlu8: M %
-// 16).  Up to kSmallK they are also faster than the int8-MFMA stream, whose units of
-// 256 columns then leave 12 of its 16 waves idle (Q4_0 288 x 768 3.1 -> 2.3 us, 1536 x
-// 768 3.2 -> 2.5, 32000 x 256 6.9 -> 4.5; at K = 1536 from 4096 rows on it is not: 3.5
-// against 3.7).
-// Past 512 columns only up to 6144 rows (6000 x 1024 Q4_0 4% faster, 8192 x 1024 2% slower,
-// 16384 x 768 9%).  A wave holds whole rows there, whose 64-bit sums leave less error than
-// the stream's integers and fp32 sums.
+// 16).  Up to kSmallK they come before the int8-MFMA stream, whose units of 256 columns
+// then leave 12 of its 16 waves idle, at every M, so that a row's bits do not depend on it
+// (rows / stream, us: Q4_0 300 x 768 2.0 / 3.2, 8192 x 768 3.6 / 4.0, 32000 x 768 6.8 / 7.8,
+// 32000 x 1024 7.6 / 8.1; the worst are Q5_0's, 20000 x 1024 7.5 / 6.8; at K = 1536 the
+// stream is the faster from 4096 rows on, 3.5 / 3.7).  64-bit sums there leave less error
+// than the stream's integers and fp32 sums (4.7e-8 against 6.8e-8 of the result's norm).
 constexpr int kSmallK = 1024;
-inline bool rows_before_stream(int64_t M, int64_t K) { return K <= 512 || (K <= kSmallK && M <= 6144); }
+inline bool rows_before_stream(int64_t K) { return K <= kSmallK; }
 bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const float* scales, const float* x,
                        int64_t M, int64_t K, const MatvecOpts& opts);
 int matvec_rows_launch(int bits, bool gguf, const void* w, const uint8_t* qh, const float* scales, const float* x,
@@ -170,8 +169,9 @@ int silu_launch(float* g, const float* u, int64_t dim, hipStream_t st);
 int swiglu_pairs_launch(const float* gu, float* h, int64_t H, hipStream_t st);
 // h = silu(W_gate x) * (W_up x) over GGUF blocks whose 2H rows interleave gate
 // and up in groups of 8 (kPostSwiGlu8), x transformed by o.pre on the way in.
-// One launch where the int8-MFMA stream takes the shape; otherwise the matvec
-// writes its 2H outputs to `work` and swiglu_pairs_launch combines them.
+// One launch where the int8-MFMA stream or the row kernels take the shape and h overlaps
+// neither x nor the pre-op's argument; otherwise the matvec writes its 2H outputs to
+// `work` and swiglu_pairs_launch combines them.
 int matvec_swiglu_launch(QuantType qt, const void* w, const float* x, float* h, int64_t H, int64_t K, float* work,
                          hipStream_t st, const MatvecOpts& o);
 int attention_launch(const float* q, const float* k, const float* v, float* y, int64_t seq, int64_t hd, float scale,

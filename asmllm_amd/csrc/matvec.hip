@@ -661,7 +661,7 @@ int matvec_launch(QuantType qt, bool gguf, const void* w, const float* scales, c
     // pre-ops: only for the shapes the pair kernels take (the entry points' contract)
     const bool rows = (opts.pre == kPreNone || pairs) &&
                       matvec_rows_takes(bits, gguf, w, nullptr, scales, x, M, K, opts);
-    if (rows && rows_before_stream(M, K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
+    if (rows && rows_before_stream(K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
         return matvec_rows_launch(bits, gguf, w, nullptr, scales, x, y, M, K, stream, opts);
     if (qt == QuantType::Q4_0 && gguf) {
         const bool mfma_ok = q4_0_mfma_eligible(w, x, opts, M, K);
@@ -769,7 +769,7 @@ int matvec_swiglu_launch(QuantType qt, const void* w, const float* x, float* h, 
     // the row kernels combine the pairs of a shape that their plain launch takes too
     const bool rows = one && (opts.pre == kPreNone || (opts.pre <= kPreSwiGlu && K % 64 == 0)) &&
                       matvec_rows_takes(bits, true, w, nullptr, nullptr, x, M, K, po);
-    if (rows && rows_before_stream(M, K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
+    if (rows && rows_before_stream(K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0))
         return matvec_rows_launch(bits, true, w, nullptr, nullptr, x, h, M, K, stream, po);
     if (one && sel != kQ4KernelFp32) {
         if (qt == QuantType::Q4_0 && q4_0_mfma_eligible(w, x, po, M, K)) return q4_0_mfma_launch(w, x, h, M, K, stream, po);
@@ -799,7 +799,7 @@ int q5_matvec_launch(bool gguf, const void* w, const uint8_t* qh, const float* s
     int rc = kOk;
     const int sel = g_q4_kernel.load(std::memory_order_relaxed);
     const bool mfma = sel != kQ4KernelFp32, rows = matvec_rows_takes(5, gguf, w, qh, scales, x, M, K, MatvecOpts());
-    if (rows && rows_before_stream(M, K))
+    if (rows && rows_before_stream(K))
         return matvec_rows_launch(5, gguf, w, qh, scales, x, y, M, K, stream, MatvecOpts());
     if (mfma && gguf && q5_0_mfma_eligible(w, x, M, K)) return q5_0_mfma_launch(w, x, y, M, K, stream);
     if (mfma && !gguf && split_mfma_eligible(5, w, qh, scales, x, M, K))

@@ -6,15 +6,26 @@
 // reference's asm_matmul_q4 / _q5 / _q8 (src/kernels/x86_64/matmul_q4_avx2.asm:57-287,
 // matmul_q5_avx2.asm:52-238, matmul_q8_avx2.asm:51-194).
 //
-// matvec_rows.  A unit is one wave's contiguous run of blocks: `rw` whole rows (small K: a row of 9
-// blocks would leave most lanes idle), or a row's chunk of at most 64 NI blocks.  Its
+// Two kernels, and one order of the sums, so that a row's bits do not depend on which of
+// them a matrix's size picks (a weight cut by rows gives the rows of the whole).  An item
+// is the 8 columns 4g..4g+3 and 16+4g..16+4g+3 of a block (Q8: 8g..8g+7), g = 0..3, and t
+// its products with x added by fused multiply-adds:
+//   K <= 1024  t in two halves, d (t0 + t1) in 64 bits; the four items of a block as
+//              (v0 + v1) + (v2 + v3); blocks j and j + 16; the 16 j in fours as (e0 + e2) +
+//              (e1 + e3); the fours as (h0 + h1) + (h2 + h3), all in 64 bits;
+//   above      for each of 64 columns of blocks 64 p + l one chain of fused d t over p for
+//              every item; the four items, then 16 l as above, in fp32, and the four
+//              sixteens in order.
+//
+// matvec_rows.  A unit is one wave's contiguous run of blocks: `rw` whole rows, or a
+// row's chunk of 64 NI blocks.  Its
 // bytes are requested as consecutive 16-byte pieces (split planes: each lane its own
 // block), parked in the wave's own piece of LDS, and read back one block a lane: a
 // lane's block is 18, 22 or 34 bytes at a 2-byte address, and loads of those strides
 // touch three lines per four lanes.  The next unit is requested as soon as the
 // registers are parked, so a wave always has one unit in flight; waves wait for no
 // one but at the start, for x.  x is staged once per workgroup (36 floats per block:
-// the 16-byte reads of eight consecutive blocks fall on distinct banks), and a
+// the 16-byte reads of eight consecutive blocks fall on distinct banks), and the
 // workgroup of 16 waves walks the tiles of 16 rw rows b, b + grid, ...
 // Every weight becomes an exact float by one sign-extending byte conversion: a Q4
 // nibble n as the byte 16 (n - 8), a Q5 value b as 8 (b - 16), with x staged as x / 16
@@ -32,13 +43,31 @@ namespace asmhip {
 
 namespace {
 
-constexpr int kWaves = 16;
-constexpr int kThreads = kWaves * 64;
 constexpr uint32_t kPastEnd = 0xFFFFFF00u;  // buffer offset that loads zeros
 constexpr int kXPitch = 36;                 // floats of x per block in LDS
 constexpr int kXEarly = 6;                  // x values a thread requests before the first weights
+constexpr int kWaves = 16;                  // of a matvec_rows workgroup
+constexpr int kShortK = 1024, kWaveK = 8192;  // 64-bit sums up to, matvec_wave up to
 
 enum RowsFmt : int { kRows4 = 0, kRows5 = 1, kRows8 = 2 };
+
+// What a unit of matvec_rows holds: kPack64 (K <= 1024) and kPack32 (K <= 2048) the blocks
+// of up to 16 rows, one after another on the lanes, so that no pass is half empty; kTwo
+// (K <= 4096) two rows of two blocks a lane; 1..4 so many blocks a lane of one row, a chunk
+// of it.
+enum RowsMode : int { kPack64 = 0, kPack32 = 5, kTwo = 6 };
+template <int MODE>
+struct RowsShape {
+    static constexpr bool kPacked = MODE == kPack64 || MODE == kPack32;
+    static constexpr bool kChunked = MODE >= 1 && MODE <= 4;
+    static constexpr int NP = kPacked ? 1 : MODE == kTwo ? 2 : MODE;  // blocks a lane of one row
+    static constexpr int RU = MODE == kTwo ? 2 : 1;                   // rows
+    static constexpr int NI = kPacked ? 3 : NP * RU;
+    static constexpr int kMaxRows = kPacked ? 16 : RU;
+    // passes of RMSNorm's squares: as matvec_wave's, at most four (above kWaveK by threads)
+    static constexpr int kSq = MODE == kPack64 ? 2 : kChunked ? 4 : NP;
+    using Sum = std::conditional_t<MODE == kPack64, double, float>;  // of a packed block's products
+};
 
 template <int QT, bool GGUF, int NI>
 struct RowsUnit {
@@ -64,39 +93,151 @@ __device__ __forceinline__ uint32_t spread_bits(uint32_t h, int g) {
     return __umul24((s >= 0 ? h >> s : h << -s) & 0x780u, 0x204081u);
 }
 
-// sum_j q[j] xb[j] of one block, q its dwords (Q5: nh the inverted fifth bits)
+// An item's two groups of four weights as signed bytes, from its dwords of a block (Q4,
+// Q5: one; Q8: two; nh: the inverted fifth bits, the item's from 4 g on)
 template <int QT>
-__device__ __forceinline__ float block_dot(const uint32_t* q, uint32_t nh, const float* xb) {
-    float t0 = 0.f, t1 = 0.f;
-    const float4* x4 = reinterpret_cast<const float4*>(xb);
-    auto four = [&](uint32_t v, const float4& x, float t) {
-        t = fmaf(sbyte(v, 0), x.x, t);
-        t = fmaf(sbyte(v, 1), x.y, t);
-        t = fmaf(sbyte(v, 2), x.z, t);
-        return fmaf(sbyte(v, 3), x.w, t);
-    };
+__device__ __forceinline__ void item_bytes(uint32_t q0, uint32_t q1, uint32_t nh, int g, uint32_t* lo, uint32_t* hi) {
     if constexpr (QT == kRows8) {
+        *lo = q0, *hi = q1;
+    } else if constexpr (QT == kRows4) {
+        *lo = ((q0 << 4) ^ 0x80808080u) & 0xF0F0F0F0u;
+        *hi = (q0 ^ 0x80808080u) & 0xF0F0F0F0u;
+    } else {
+        *lo = ((q0 << 3) & 0x78787878u) | (spread_bits(nh, g) & 0x80808080u);
+        *hi = ((q0 >> 1) & 0x78787878u) | (spread_bits(nh, 4 + g) & 0x80808080u);
+    }
+    *lo = opaque(*lo), *hi = opaque(*hi);
+}
+
+// An item's sum of a short row: d (t0 + t1), rounded once to 64 bits
+__device__ __forceinline__ double item_short(uint32_t lo, uint32_t hi, const float* xl, const float* xh, float d) {
+#pragma clang fp contract(off)
+    float t0 = 0.f, t1 = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            t0 = four(opaque(q[i]), x4[i], t0);
-            t1 = four(opaque(q[4 + i]), x4[4 + i], t1);
-        }
+    for (int k = 0; k < 4; ++k) {
+        t0 = fmaf(sbyte(lo, k), xl[k], t0);
+        t1 = fmaf(sbyte(hi, k), xh[k], t1);
+    }
+    return (double)d * ((double)t0 + (double)t1);
+}
+__device__ __forceinline__ float item_long(uint32_t lo, uint32_t hi, const float* xl, const float* xh) {
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        t = fmaf(sbyte(lo, k), xl[k], t);
+        t = fmaf(sbyte(hi, k), xh[k], t);
+    }
+    return t;
+}
+
+// Item g of the block whose dwords are q
+template <int QT>
+__device__ __forceinline__ void item_of(const uint32_t* q, uint32_t nh, const float* xb, int g, uint32_t* lo,
+                                        uint32_t* hi, const float** xl, const float** xh) {
+    constexpr bool k8 = QT == kRows8;
+    item_bytes<QT>(q[k8 ? 2 * g : g], k8 ? q[2 * g + 1] : 0u, nh, g, lo, hi);
+    *xl = xb + (k8 ? 8 * g : 4 * g), *xh = xb + (k8 ? 8 * g + 4 : 16 + 4 * g);
+}
+
+// Sum over the squares of x (RMSNorm) in the order of the items: one wave's NP passes from
+// item `first` on
+template <int QT, int NP>
+__device__ __forceinline__ float item_squares(const float (*x)[8], const bool* live) {
+    float ss = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) ss = live[p] ? fmaf(x[p][t], x[p][t], ss) : ss;
+    return wave_total_dpp(ss);
+}
+
+template <typename T>
+__device__ __forceinline__ T load_at(const void* p) {  // any 2-byte aligned address
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+
+// The 8 values of item `it` (of a vector of K floats, 4-byte aligned)
+template <int QT>
+__device__ __forceinline__ void item_load(const float* src, int it, float* to) {
+    const int b = it >> 2, g = it & 3;
+    const int e0 = 32 * b + (QT == kRows8 ? 8 : 4) * g, e1 = e0 + (QT == kRows8 ? 4 : 16);
+    const float4 u = load_at<float4>(src + e0), v = load_at<float4>(src + e1);
+    to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w;
+    to[4] = v.x, to[5] = v.y, to[6] = v.z, to[7] = v.w;
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __longlong_as_double((long long)hi << 32 | (uint32_t)lo);
+}
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;  // 16-lane rows rotated
+
+// v of the even and of the odd 16-lane row of each half-wave, and of the halves
+__device__ __forceinline__ void row_pair(float v, float* even, float* odd) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    *even = __uint_as_float(r[0]), *odd = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void half_pair(float v, float* low, float* high) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    *low = __uint_as_float(r[0]), *high = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void row_pair(double v, double* even, double* odd) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const auto l = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    *even = __longlong_as_double((long long)((uint64_t)h[0] << 32 | l[0]));
+    *odd = __longlong_as_double((long long)((uint64_t)h[1] << 32 | l[1]));
+}
+__device__ __forceinline__ void half_pair(double v, double* low, double* high) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const auto l = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    *low = __longlong_as_double((long long)((uint64_t)h[0] << 32 | l[0]));
+    *high = __longlong_as_double((long long)((uint64_t)h[1] << 32 | l[1]));
+}
+
+// The quads' sums (v0 + v1) + (v2 + v3) of R rows at once: lane l's result is row l % R's.
+// The rows are dealt to the lanes as the sums halve, so that R of them take little more
+// than one (one after another, with a readlane from each 16 lanes, the sums were a third of
+// a short row's instructions).
+template <int R, typename T>
+__device__ __forceinline__ T quad_sums(const T (&v)[R], int lane) {
+    T t[R > 1 ? R / 2 : 1];
+    if constexpr (R == 1) {
+        t[0] = v[0] + dpp<kDppQuadXor1>(v[0]);
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t lo, hi;
-            if constexpr (QT == kRows4) {
-                lo = ((q[i] << 4) ^ 0x80808080u) & 0xF0F0F0F0u;
-                hi = (q[i] ^ 0x80808080u) & 0xF0F0F0F0u;
-            } else {
-                lo = ((q[i] << 3) & 0x78787878u) | (spread_bits(nh, i) & 0x80808080u);
-                hi = ((q[i] >> 1) & 0x78787878u) | (spread_bits(nh, 4 + i) & 0x80808080u);
-            }
-            t0 = four(opaque(lo), x4[i], t0);
-            t1 = four(opaque(hi), x4[4 + i], t1);
+        for (int i = 0; i < R / 2; ++i) {
+            const T keep = lane & 1 ? v[2 * i + 1] : v[2 * i], send = lane & 1 ? v[2 * i] : v[2 * i + 1];
+            t[i] = keep + dpp<kDppQuadXor1>(send);
         }
     }
-    return t0 + t1;
+    if constexpr (R < 4) {
+        return t[0] + dpp<kDppQuadXor2>(t[0]);
+    } else {
+        const T keep = lane & 2 ? t[1] : t[0], send = lane & 2 ? t[0] : t[1];
+        return keep + dpp<kDppQuadXor2>(send);
+    }
+}
+// The sum over the quads of a wave, lane by lane of a quad: of each 16 lanes as (q0 + q2) +
+// (q1 + q3), of these as (h0 + h1) + (h2 + h3)
+template <typename T>
+__device__ __forceinline__ T over_quads(T q) {
+    T a, b;
+    q += dpp<kDppRor8>(q);
+    q += dpp<kDppRor4>(q);
+    row_pair(q, &a, &b);
+    half_pair(a + b, &a, &b);
+    return a + b;
 }
 
 struct RowsArgs {
@@ -106,20 +247,20 @@ struct RowsArgs {
     const float* x;
     const float* pre_arg;
     float* y;
-    int M, K, pre, accumulate, post, rw, chunk, nchunk, splits, hd;
+    int M, K, pre, accumulate, post, rw, nchunk, splits, hd;
     float eps;
 };
 
-template <int QT, bool GGUF, int NI>
-__global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
+template <int QT, bool GGUF, int MODE>
+__global__ __launch_bounds__(kWaves * 64) void matvec_rows(const RowsArgs a) {
+    using S = RowsShape<MODE>;
+    constexpr int NI = S::NI, NP = S::NP, kThreads = kWaves * 64;
     using U = RowsUnit<QT, GGUF, NI>;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    __shared__ float red[kWaves], ybuf[2][kWaves * 64];
+    __shared__ float red[kWaves], ybuf[2][kWaves * S::kMaxRows];
     const int nb = a.K >> 5, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rw = a.rw, tile_rows = kWaves * rw, nchunk = a.nchunk, G = gridDim.x;
-    const int n_tiles = (a.M + tile_rows - 1) / tile_rows;
-    const int my_tiles = (n_tiles - (int)blockIdx.x + G - 1) / G, L = my_tiles * nchunk;
+    const int rw = a.rw, tile_rows = kWaves * rw, nchunk = S::kChunked ? a.nchunk : 1, G = gridDim.x;
     const uint32_t nblocks = (uint32_t)a.M * (uint32_t)nb;
     // whole dwords: an odd number of GGUF blocks ends inside one (of the 4-byte aligned
     // buffer), and a dword that reaches past the descriptor would read as zero
@@ -128,20 +269,26 @@ __global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
     const auto sr = make_rsrc(a.wsc, GGUF ? 0u : nblocks * 4u);
     float* xs = reinterpret_cast<float*>(lds);
     uint8_t* slot = lds + (size_t)nb * kXPitch * 4 + wave * U::kSlot;
-    float* prod = reinterpret_cast<float*>(lds + (size_t)nb * kXPitch * 4 + kWaves * U::kSlot) + wave * 64 * NI;
+    typename S::Sum* prod = reinterpret_cast<typename S::Sum*>(lds + (size_t)nb * kXPitch * 4 + kWaves * U::kSlot) + wave * 64 * NI;
 
-    // unit s: tile i = s / nchunk, chunk s % nchunk; its first block and number of blocks
-    auto unit = [&](int s, uint32_t* b0) {
-        const int i = s / nchunk, c = s - i * nchunk;
-        const int row0 = ((int)blockIdx.x + G * i) * tile_rows + wave * rw;
-        *b0 = (uint32_t)row0 * (uint32_t)nb + (uint32_t)(c * a.chunk);
-        const int n = rw > 1 ? min(rw, a.M - row0) * nb : min(a.chunk, nb - c * a.chunk);
-        return s < L && row0 < a.M ? n : 0;
+    // chunk c of a tile from row `row` on: this wave's first block and number of blocks
+    auto unit = [&](int row, int c, uint32_t* b0) {
+        const int row0 = row + wave * rw;
+        *b0 = (uint32_t)row0 * (uint32_t)nb + (uint32_t)(c * 64 * NI);
+        const int n = S::kChunked ? min(64 * NI, nb - c * 64 * NI) : min(rw, a.M - row0) * nb;
+        return row0 < a.M ? n : 0;
+    };
+    // the place of the lane's k-th block in a unit: from the unit's end on if there is none
+    // (a row's last pass is not full)
+    auto place = [&](int k) {
+        if (S::kPacked || S::RU == 1) return lane + 64 * k;
+        const int col = lane + 64 * (k % NP);
+        return col < nb ? k / NP * nb + col : 1 << 30;
     };
     U u;
-    auto load = [&](int s) {
+    auto load = [&](int row, int c) {
         uint32_t b0;
-        const int n = unit(s, &b0);
+        const int n = unit(row, c, &b0);
         if constexpr (GGUF) {
             const uint32_t begin = b0 * (uint32_t)U::kBB, end = begin + (uint32_t)(n * U::kBB);
             const uint32_t p0 = (begin & ~15u) + 16u * (uint32_t)lane;
@@ -153,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
         } else {
 #pragma unroll
             for (int k = 0; k < NI; ++k) {
-                const int b = lane + 64 * k;
+                const int b = place(k);
                 const uint32_t blk = b0 + (uint32_t)b;
 #pragma unroll
                 for (int h = 0; h < U::kQs / 16; ++h)
@@ -174,15 +321,28 @@ __global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
         xv[i] = e < a.K ? a.x[e] : 0.f;
         gv[i] = pre != kPreNone && e < a.K ? a.pre_arg[e] : 0.f;
     }
+    // RMSNorm's sum of squares as matvec_wave forms it, by as many waves as share a row there
+    const bool by_items = a.K <= kWaveK;
+    const int sq_waves = MODE == kPack64 ? 1 : 4;
+    float xq[S::kSq][8];
+    bool live[S::kSq];
+    if (pre == kPreRmsNorm && by_items && wave < sq_waves) {
+#pragma unroll
+        for (int p = 0; p < S::kSq; ++p) {
+            const int it = lane + 64 * (sq_waves * p + wave);
+            live[p] = it < 4 * nb;
+            item_load<QT>(a.x, live[p] ? it : 0, xq[p]);
+        }
+    }
     __builtin_amdgcn_sched_barrier(0);
-    load(0);
+    load((int)blockIdx.x * tile_rows, 0);
     __builtin_amdgcn_sched_barrier(0);
     float ss = 0.f;
     auto stage = [&](int e, float x, float g) {
         if (pre == kPreRmsNorm) {
             // y = W (inv (x g)) = inv (W (x g)): the row totals are scaled, so no
             // barrier comes before the staging
-            ss = fmaf(x, x, ss);
+            if (!by_items) ss = fmaf(x, x, ss);
             x = __fmul_rn(x, g);
         } else if (pre == kPreSwiGlu) {
             x = __fmul_rn(x / (1.0f + expf(-x)), g);
@@ -197,56 +357,60 @@ __global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
     for (int e = (int)threadIdx.x + kThreads * kXEarly; e < a.K; e += kThreads)
         stage(e, a.x[e], pre != kPreNone ? a.pre_arg[e] : 0.f);
     if (pre == kPreRmsNorm) {
-        ss = wave_total_dpp(ss);
+        if (!by_items)
+            ss = wave_total_dpp(ss);
+        else if (wave < sq_waves)
+            ss = item_squares<QT, S::kSq>(xq, live);
         if (lane == 0) red[wave] = ss;
     }
-    // rw > 1: the column block of the lane's k-th block, the same in every unit
-    int cb[NI];
+    // packed: the column block of the lane's k-th block, the same in every unit
+    int cb[S::kPacked ? NI : 1];
+    if constexpr (S::kPacked) {
 #pragma unroll
-    for (int k = 0; k < NI; ++k) cb[k] = rw > 1 ? (lane + 64 * k) % nb : lane + 64 * k;
+        for (int k = 0; k < NI; ++k) cb[k] = (lane + 64 * k) % nb;
+    }
     __syncthreads();
     float inv = 1.f;
     if (pre == kPreRmsNorm) {
         float tot = 0.f;
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) tot += red[k];
+        for (int k = 0; k < kWaves; ++k)
+            if (k < (by_items ? sq_waves : kWaves)) tot += red[k];
         inv = 1.0f / sqrtf(tot / (float)a.K + a.eps);
     }
 
     // 2) the stream
-    float acc = 0.f;
-    for (int s = 0; s < L; ++s) {
+    float part[4] = {0.f, 0.f, 0.f, 0.f};  // the lane's chain of each item
+    for (int tile_row = (int)blockIdx.x * tile_rows, c = 0, buf = 0; tile_row < a.M;) {
         uint32_t b0;
-        const int n = unit(s, &b0);
-        const int i = s / nchunk, c = s - i * nchunk;
+        const int n = unit(tile_row, c, &b0), next = tile_row + G * tile_rows;
         uint32_t shift = 0;
         U cur;
         if constexpr (GGUF) {
             shift = (b0 * (uint32_t)U::kBB) & 15u;
 #pragma unroll
             for (int k = 0; k < U::kPieces; ++k) *reinterpret_cast<uint4*>(slot + 1024 * k + 16 * lane) = u.v[k];
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();
         } else {
             cur = u;
         }
-        load(s + 1);
+        if (c < nchunk - 1)
+            load(tile_row, c + 1);
+        else
+            load(next, 0);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int k = 0; k < NI; ++k) {
-            if (64 * k >= n) break;  // wave-uniform
-            const int b = min(lane + 64 * k, n - 1);
-            uint32_t q[U::kQs / 4], nh = 0;
-            float d;
+        // the block at place b of the unit, the lane's k-th
+        auto block = [&](int k, int b, uint32_t* q, uint32_t* nh, float* d) {
             if constexpr (GGUF) {
                 const uint32_t o = shift + (uint32_t)b * (uint32_t)U::kBB;  // even
-                d = __half2float(__ushort_as_half(*reinterpret_cast<const uint16_t*>(slot + o)));
+                *d = __half2float(__ushort_as_half(*reinterpret_cast<const uint16_t*>(slot + o)));
                 const uint32_t* p = reinterpret_cast<const uint32_t*>(slot + ((o + 2u) & ~3u));
                 const uint32_t sh = (o + 2u) & 3u;
                 constexpr int kHead = QT == kRows5 ? 1 : 0;
                 uint32_t r[U::kQs / 4 + kHead + 1];
 #pragma unroll
                 for (int t = 0; t < U::kQs / 4 + kHead + 1; ++t) r[t] = p[t];
-                if constexpr (QT == kRows5) nh = ~__builtin_amdgcn_alignbyte(r[1], r[0], sh);
+                if constexpr (QT == kRows5) *nh = ~__builtin_amdgcn_alignbyte(r[1], r[0], sh);
 #pragma unroll
                 for (int t = 0; t < U::kQs / 4; ++t) q[t] = __builtin_amdgcn_alignbyte(r[t + kHead + 1], r[t + kHead], sh);
             } else {
@@ -255,47 +419,122 @@ __global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
                     const uint4 v = cur.v[k * (U::kQs / 16) + h];
                     q[4 * h] = v.x, q[4 * h + 1] = v.y, q[4 * h + 2] = v.z, q[4 * h + 3] = v.w;
                 }
-                if constexpr (QT == kRows5) nh = ~cur.qh[k];
-                d = __uint_as_float(cur.sc[k]);
+                if constexpr (QT == kRows5) *nh = ~cur.qh[k];
+                *d = __uint_as_float(cur.sc[k]);
             }
-            const int col = rw > 1 ? cb[k] : c * a.chunk + b;
-            const float t = block_dot<QT>(q, nh, xs + col * kXPitch);
-            if (rw > 1)
-                prod[lane + 64 * k] = d * t;
-            else if (lane + 64 * k < n)
-                acc = fmaf(d, t, acc);
-        }
-        if (c < nchunk - 1) continue;
-        const int row0 = ((int)blockIdx.x + G * i) * tile_rows + wave * rw;
-        float sum;  // rw > 1: lane r holds row r's total; else every lane the row's
-        if (rw > 1) {
-            __builtin_amdgcn_wave_barrier();
-            sum = 0.f;
-            if (lane * nb < n)
-                for (int j = 0; j < nb; ++j) sum += prod[lane * nb + j];
-            __builtin_amdgcn_wave_barrier();
+        };
+        float sum = 0.f;  // the total of row row0 + r of lanes where `owner`
+        int r = lane;
+        bool owner = lane < rw;
+        if constexpr (S::kPacked) {
+#pragma clang fp contract(off)
+#pragma unroll
+            for (int k = 0; k < NI; ++k) {
+                if (64 * k >= n) break;  // wave-uniform
+                uint32_t q[U::kQs / 4], nh = 0, lo, hi;
+                float d;
+                block(k, min(lane + 64 * k, n - 1), q, &nh, &d);
+                typename S::Sum v[4];
+                const float *xl, *xh;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    item_of<QT>(q, nh, xs + cb[k] * kXPitch, g, &lo, &hi, &xl, &xh);
+                    if constexpr (MODE == kPack64)
+                        v[g] = item_short(lo, hi, xl, xh, d);
+                    else
+                        v[g] = fmaf(d, item_long(lo, hi, xl, xh), 0.f);
+                }
+                prod[lane + 64 * k] = (v[0] + v[1]) + (v[2] + v[3]);
+            }
+            wave_lds_order();
+            // four lanes a row
+            r = lane >> 2;
+            const int part4 = lane & 3;
+            owner = part4 == 0 && r < rw;
+            const typename S::Sum* row = prod + r * nb;
+            if constexpr (MODE == kPack64) {  // four j each
+                const int j0 = 4 * part4;
+                double e[4] = {};
+                if (r * nb < n) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) e[j] = row[j0 + j] + (j0 + 16 + j < nb ? row[j0 + 16 + j] : 0.0);
+                }
+                double h = (e[0] + e[2]) + (e[1] + e[3]);
+                h += dpp<kDppQuadXor1>(h);
+                h += dpp<kDppQuadXor2>(h);
+                sum = (float)h;
+            } else {  // a sixteen each
+                float h[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float e[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int l = 16 * part4 + 4 * i + j;
+                        e[j] = r * nb < n && l < nb ? row[l] : 0.f;
+                    }
+                    h[i] = (e[0] + e[2]) + (e[1] + e[3]);
+                }
+                const float t = (h[0] + h[1]) + (h[2] + h[3]);
+                sum = (((0.f + dpp<0x00>(t)) + dpp<0x55>(t)) + dpp<0xAA>(t)) + dpp<0xFF>(t);  // lanes 0..3 of the quad
+            }
         } else {
-            sum = wave_total_dpp(acc);
-            acc = 0.f;
+#pragma unroll
+            for (int t = 0; t < S::RU; ++t) {
+                if (t >= rw) break;  // wave-uniform
+#pragma unroll
+                for (int p = 0; p < NP; ++p) {
+                    const int k = t * NP + p, b = place(k);
+                    if (b < n) {
+                        uint32_t q[U::kQs / 4], nh = 0, lo, hi;
+                        float d;
+                        block(k, b, q, &nh, &d);
+                        const float *xl, *xh, *xb = xs + (S::kChunked ? c * 64 * NI + b : lane + 64 * p) * kXPitch;
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            item_of<QT>(q, nh, xb, g, &lo, &hi, &xl, &xh);
+                            part[g] = fmaf(d, item_long(lo, hi, xl, xh), part[g]);
+                        }
+                    }
+                }
+                if (c < nchunk - 1) break;
+                float h = (part[0] + part[1]) + (part[2] + part[3]);
+                h += dpp<kDppQuadXor2>(h);
+                h += dpp<kDppQuadXor1>(h);
+                h += dpp<kDppRowHalfMirror>(h);
+                h += dpp<kDppRowMirror>(h);
+                const int v = __float_as_int(h);
+                float tot = 0.f;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) tot += __int_as_float(__builtin_amdgcn_readlane(v, 16 * w));
+                sum = lane == t ? tot : sum;
+                part[0] = part[1] = part[2] = part[3] = 0.f;
+            }
+        }
+        wave_lds_order();  // the next unit's bytes (and products) take the place of this one's
+        if (c < nchunk - 1) {
+            ++c;
+            continue;
         }
         sum = __fmul_rn(sum, inv);
-        const int row = row0 + lane;
+        const int row = tile_row + wave * rw + r;
         if (a.post == kPostNone) {
-            if (lane < rw && row < a.M) a.y[row] = a.accumulate ? a.y[row] + sum : sum;
+            if (owner && row < a.M) a.y[row] = a.accumulate ? a.y[row] + sum : sum;
         } else {
             // groups of 8 gate rows and their 8 up rows (tiles are whole groups): the
             // totals meet in LDS, two buffers so that one barrier a tile is enough
-            float* yb = ybuf[i & 1];
-            if (lane < rw) yb[wave * rw + lane] = sum;
+            float* yb = ybuf[buf];
+            if (owner) yb[wave * rw + r] = sum;
             __syncthreads();
             for (int j = threadIdx.x; j < tile_rows / 2; j += kThreads) {
-                const int r = 16 * (j >> 3) + (j & 7), g = ((int)blockIdx.x + G * i) * tile_rows + r;
+                const int r = 16 * (j >> 3) + (j & 7), g = tile_row + r;
                 if (g < a.M) {
                     const float gs = yb[r], us = yb[r + 8];
                     a.y[8 * (g >> 4) + (j & 7)] = __fmul_rn(gs / (1.0f + expf(-gs)), us);
                 }
             }
         }
+        tile_row = next, c = 0, buf ^= 1;
     }
 }
 
@@ -310,31 +549,6 @@ __global__ __launch_bounds__(kThreads) void matvec_rows(const RowsArgs a) {
 // up pairs, 8 rows apart.
 // ---------------------------------------------------------------------------
 constexpr int kWaveThreads = 256;
-
-template <typename T>
-__device__ __forceinline__ T load_at(const uint8_t* p) {  // any 2-byte aligned address
-    T v;
-    __builtin_memcpy(&v, p, sizeof(T));
-    return v;
-}
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
-    return v + __longlong_as_double((long long)hi << 32 | (uint32_t)lo);
-}
-__device__ __forceinline__ double lane_value(double v, int l) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double((long long)hi << 32 | (uint32_t)lo);
-}
-__device__ __forceinline__ double wave_total64(double v) {
-    v = dpp_add<kDppQuadXor1>(v), v = dpp_add<kDppQuadXor2>(v);
-    v = dpp_add<kDppRowHalfMirror>(v), v = dpp_add<kDppRowMirror>(v);
-    return ((lane_value(v, 0) + lane_value(v, 16)) + lane_value(v, 32)) + lane_value(v, 48);
-}
 
 template <int QT, bool GGUF, int NP, int R, int W>
 __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
@@ -356,16 +570,11 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
     int blk[NP], g[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-        const int it = lane + 64 * (W == 1 ? p : wave * NP + p);
+        const int it = lane + 64 * (W * p + (W == 1 ? 0 : wave));
         live[p] = it < items;
         const int ic = live[p] ? it : 0;
         blk[p] = ic >> 2, g[p] = ic & 3;
         const int e0 = 32 * blk[p] + (QT == kRows8 ? 8 : 4) * g[p], e1 = e0 + (QT == kRows8 ? 4 : 16);
-        auto get8 = [&](const float* src, float* to) {
-            const float4 u = *reinterpret_cast<const float4*>(src + e0), v = *reinterpret_cast<const float4*>(src + e1);
-            to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w;
-            to[4] = v.x, to[5] = v.y, to[6] = v.z, to[7] = v.w;
-        };
         if (pre == kPreAttnMerge) {
             // the heads of the two quads (head_dim need not hold a whole block)
             const int stride = kAttnPartStride(a.hd);
@@ -392,8 +601,8 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
                 x[p][4 * q + 3] = none ? 0.f : s.w / l;
             }
         } else {
-            get8(a.x, x[p]);
-            if (pre != kPreNone) get8(a.pre_arg, gn[p]);
+            item_load<QT>(a.x, ic, x[p]);
+            if (pre != kPreNone) item_load<QT>(a.pre_arg, ic, gn[p]);
         }
     }
     uint32_t q[R][NP][kQs / 16], qh[R][QT == kRows5 ? NP : 1], sc[R][NP];
@@ -418,104 +627,77 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
                 sc[r][p] = __float_as_uint(a.wsc[b]);
         }
     }
+    // one branch for all of x: a pre-op looked at element by element was a branch for each
     float ss = 0.f;
+    auto each = [&](auto f) {
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
+        for (int p = 0; p < NP; ++p)
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            float v = x[p][t];
-            if (pre == kPreRmsNorm) {  // y = W (inv (x g)) = inv (W (x g))
-                ss = live[p] ? fmaf(v, v, ss) : ss;
-                v = __fmul_rn(v, gn[p][t]);
-            } else if (pre == kPreSwiGlu) {
-                v = __fmul_rn(v / (1.0f + expf(-v)), gn[p][t]);
-            }
-            x[p][t] = v * RowsUnit<QT, GGUF, 1>::kXScale;
-        }
-    ss = wave_total_dpp(ss);
-    float tot[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        // a wave per row (K <= 1024) adds its fours of products in 64 bits: in fp32 throughout
-        // the error was 1.5 times the int8-MFMA stream's (15122 x 256 8.4e-8 against 5.6e-8
-        // of the result's norm), so it is 4.7e-8, for 0.1 us at 288 x 288 and 0.7 at 32000 x 288
-        std::conditional_t<W == 1, double, float> acc = 0;
+            for (int t = 0; t < 8; ++t) x[p][t] = f(x[p][t], gn[p][t]);
+    };
+    if (pre == kPreRmsNorm) {  // y = W (inv (x g)) = inv (W (x g))
+        ss = item_squares<QT, NP>(x, live);
+        each([](float v, float g) { return __fmul_rn(v, g); });
+    } else if (pre == kPreSwiGlu) {
+        each([](float v, float g) { return __fmul_rn(v / (1.0f + expf(-v)), g); });
+    }
+    each([](float v, float) { return v * RowsUnit<QT, GGUF, 1>::kXScale; });
+    // lane l: the total of row l % R.  A wave per row (K <= 1024) adds in 64 bits: in fp32
+    // throughout the error was 1.5 times the int8-MFMA stream's (15122 x 256 8.4e-8 against
+    // 5.6e-8 of the result's norm), so it is 4.7e-8
+    float tot;
+    auto bytes = [&](int r, int p, uint32_t* lo, uint32_t* hi) {
+        item_bytes<QT>(q[r][p][0], q[r][p][kQs / 16 - 1], QT == kRows5 ? ~qh[r][QT == kRows5 ? p : 0] >> (4 * g[p]) : 0u, 0,
+                       lo, hi);
+        return GGUF ? half_lo(sc[r][p]) : __uint_as_float(sc[r][p]);
+    };
+    if constexpr (W == 1) {
+        double sum = 0.0;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            uint32_t lo, hi;
-            if constexpr (QT == kRows8) {
-                lo = q[r][p][0], hi = q[r][p][1];
-            } else if constexpr (QT == kRows4) {
-                lo = ((q[r][p][0] << 4) ^ 0x80808080u) & 0xF0F0F0F0u;
-                hi = (q[r][p][0] ^ 0x80808080u) & 0xF0F0F0F0u;
-            } else {
-                const uint32_t nh = ~qh[r][p] >> (4 * g[p]);
-                lo = ((q[r][p][0] << 3) & 0x78787878u) | (spread_bits(nh, 0) & 0x80808080u);
-                hi = ((q[r][p][0] >> 1) & 0x78787878u) | (spread_bits(nh, 4) & 0x80808080u);
-            }
-            lo = opaque(lo), hi = opaque(hi);
-            const float d = GGUF ? half_lo(sc[r][p]) : __uint_as_float(sc[r][p]);
-            if constexpr (W == 1) {
-                float t0 = 0.f, t1 = 0.f;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    t0 = fmaf(sbyte(lo, k), x[p][k], t0);
-                    t1 = fmaf(sbyte(hi, k), x[p][4 + k], t1);
-                }
-                acc = live[p] ? fma((double)d, (double)t0 + (double)t1, acc) : acc;
-            } else {
-                float t = 0.f;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    t = fmaf(sbyte(lo, k), x[p][k], t);
-                    t = fmaf(sbyte(hi, k), x[p][4 + k], t);
-                }
-                acc = live[p] ? fmaf(d, t, acc) : acc;
-            }
-        }
-        if constexpr (W == 1)
-            tot[r] = (float)wave_total64(acc);
-        else
-            tot[r] = wave_total_dpp(acc);
-    }
-    if constexpr (W > 1) {  // the waves' parts of K meet in LDS, added in order
-        __shared__ float red[R + 1][W];
-        if (lane == 0) {
-            red[R][wave] = ss;
-#pragma unroll
-            for (int r = 0; r < R; ++r) red[r][wave] = tot[r];
-        }
-        __syncthreads();
-        if (wave != 0) return;
-        ss = 0.f;
-#pragma unroll
-        for (int k = 0; k < W; ++k) ss += red[R][k];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            tot[r] = 0.f;
-#pragma unroll
-            for (int k = 0; k < W; ++k) tot[r] += red[r][k];
-        }
-    }
-    if (pre == kPreRmsNorm) {
-        const float inv = 1.0f / sqrtf(ss / (float)a.K + a.eps);
-#pragma unroll
-        for (int r = 0; r < R; ++r) tot[r] = __fmul_rn(tot[r], inv);
-    }
-    if (lane == 0) {
-        if (a.post == kPostNone) {
+#pragma clang fp contract(off)
+            double v[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const int row = gw * R + r;
-                if (row < a.M) a.y[row] = a.accumulate ? a.y[row] + tot[r] : tot[r];
+                uint32_t lo, hi;
+                const float d = bytes(r, p, &lo, &hi);
+                v[r] = item_short(lo, hi, x[p], x[p] + 4, d);
+                v[r] = live[p] ? v[r] : 0.0;
             }
-        } else {
+            const double s = quad_sums(v, lane);
+            sum = p == 0 ? s : sum + s;
+        }
+        tot = (float)over_quads(sum);
+    } else {
+        __shared__ float red[R + 1][W];  // the waves' parts of K, added in order
+        float acc[R] = {};
 #pragma unroll
-            for (int r = 0; r + 1 < R; r += 2) {
-                const int j = gw * (R / 2) + (r >> 1);
-                if (2 * j < a.M) a.y[j] = __fmul_rn(tot[r] / (1.0f + expf(-tot[r])), tot[r + 1]);
+        for (int p = 0; p < NP; ++p) {
+            if (64 * (W * p + wave) >= items) break;  // wave-uniform
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                uint32_t lo, hi;
+                const float d = bytes(r, p, &lo, &hi), v = fmaf(d, item_long(lo, hi, x[p], x[p] + 4), acc[r]);
+                acc[r] = live[p] ? v : acc[r];
             }
         }
+        tot = over_quads(quad_sums(acc, lane));
+        if (lane < R) red[lane][wave] = tot;
+        if (lane == 0) red[R][wave] = ss;
+        __syncthreads();
+        if (wave != 0) return;
+        ss = 0.f, tot = 0.f;
+#pragma unroll
+        for (int k = 0; k < W; ++k) ss += red[R][k], tot += red[lane % R][k];
+    }
+    if (pre == kPreRmsNorm) tot = __fmul_rn(tot, 1.0f / sqrtf(ss / (float)a.K + a.eps));
+    if (a.post == kPostNone) {
+        const int row = gw * R + lane;
+        if (lane < R && row < a.M) a.y[row] = a.accumulate ? a.y[row] + tot : tot;
+    } else {
+        const float up = dpp<kDppQuadXor1>(tot);  // lanes 0 and 2: a gate row's total, its up row's beside it
+        const int j = gw * (R / 2) + (lane >> 1);
+        if (lane < R && !(lane & 1) && 2 * j < a.M) a.y[j] = __fmul_rn(tot / (1.0f + expf(-tot)), up);
     }
 }
 
@@ -531,39 +713,48 @@ int row_units() {  // compute units of the current device
     return n;
 }
 
-template <int QT, bool GGUF, int NI>
-size_t rows_lds(int nb, int rw) {
+template <int QT, bool GGUF, int MODE>
+size_t rows_lds(int nb) {
+    constexpr int NI = RowsShape<MODE>::NI;
     return (size_t)nb * kXPitch * 4 + (size_t)kWaves * RowsUnit<QT, GGUF, NI>::kSlot +
-           (rw > 1 ? (size_t)kWaves * 64 * NI * 4 : 0);
+           (RowsShape<MODE>::kPacked ? (size_t)kWaves * 64 * NI * sizeof(typename RowsShape<MODE>::Sum) : 0);
 }
 
-// Rows per wave: as many tiles as compute units while a unit holds the rows.
-int rows_per_wave(int64_t M, int nb, int cus, int most) {
-    const int64_t want = (M + (int64_t)kWaves * cus - 1) / ((int64_t)kWaves * cus);
-    return (int)std::max<int64_t>(1, std::min<int64_t>({want, most / nb, 64}));
-}
-
-template <int QT, bool GGUF, int NI>
-int rows_launch_ni(RowsArgs a, hipStream_t st) {
+template <int QT, bool GGUF, int MODE>
+int rows_launch_mode(RowsArgs a, hipStream_t st) {
+    using S = RowsShape<MODE>;
     const int nb = a.K / 32, cus = row_units();
-    a.rw = rows_per_wave(a.M, nb, cus, 64 * NI);
-    a.nchunk = a.rw > 1 ? 1 : (nb + 64 * NI - 1) / (64 * NI);
-    a.chunk = (nb + a.nchunk - 1) / a.nchunk;
-    const size_t lds = rows_lds<QT, GGUF, NI>(nb, a.rw);
-    const int rc = dynamic_lds((const void*)matvec_rows<QT, GGUF, NI>, lds);
+    // rows a wave: what gives the busiest compute unit's waves the fewest passes, with one
+    // more for a unit's loads and sums (26000 x 1024 12.8 us with the fewest rows, one a unit)
+    auto tiles = [&](int rw) { return ((int64_t)a.M + kWaves * rw - 1) / (kWaves * rw); };
+    auto cost = [&](int rw) {
+        const int passes = S::kPacked ? (rw * nb + 63) / 64 : rw * S::NP;
+        return (tiles(rw) + cus - 1) / cus * (passes + 1);
+    };
+    a.rw = std::min(S::kMaxRows, S::kPacked ? 64 * S::NI / nb : S::RU);
+    for (int rw = a.rw - 1; rw >= 1; --rw)
+        if (cost(rw) < cost(a.rw)) a.rw = rw;
+    a.nchunk = S::kChunked ? (nb + 64 * S::NI - 1) / (64 * S::NI) : 1;
+    const size_t lds = rows_lds<QT, GGUF, MODE>(nb);
+    const int rc = dynamic_lds((const void*)matvec_rows<QT, GGUF, MODE>, lds);
     if (rc) return rc;
-    const int tiles = (int)(((int64_t)a.M + kWaves * a.rw - 1) / (kWaves * a.rw));
-    hipLaunchKernelGGL((matvec_rows<QT, GGUF, NI>), dim3((unsigned)std::min(tiles, cus)), dim3(kThreads), lds, st, a);
+    hipLaunchKernelGGL((matvec_rows<QT, GGUF, MODE>), dim3((unsigned)std::min<int64_t>(tiles(a.rw), cus)),
+                       dim3(kWaves * 64), lds, st, a);
     ASMHIP_TRY(hipGetLastError());
     return kOk;
 }
 
-// Three blocks a lane where the unit's LDS fits beside x, else one.
+// More than 512 columns (16 blocks)
 template <int QT, bool GGUF>
 int rows_launch_fmt(const RowsArgs& a, hipStream_t st) {
-    const int nb = a.K / 32;
-    return rows_lds<QT, GGUF, 3>(nb, 2) <= kLdsBudget ? rows_launch_ni<QT, GGUF, 3>(a, st)
-                                                      : rows_launch_ni<QT, GGUF, 1>(a, st);
+    if (a.K <= kShortK) return rows_launch_mode<QT, GGUF, kPack64>(a, st);
+    if (a.K <= 2048) return rows_launch_mode<QT, GGUF, kPack32>(a, st);
+    // as many blocks a lane as LDS holds beside x
+    if (a.K <= 4096) return rows_launch_mode<QT, GGUF, QT == kRows8 ? 2 : kTwo>(a, st);
+    if (a.K <= 6144) return rows_launch_mode<QT, GGUF, 3>(a, st);
+    if (a.K <= 8192) return rows_launch_mode<QT, GGUF, QT == kRows8 ? 2 : 4>(a, st);
+    return rows_lds<QT, GGUF, 3>(a.K / 32) <= kLdsBudget ? rows_launch_mode<QT, GGUF, 3>(a, st)
+                                                         : rows_launch_mode<QT, GGUF, 1>(a, st);
 }
 
 template <int QT, bool GGUF, int NP, int R, int W>
@@ -584,36 +775,52 @@ int wave_launch_r(const RowsArgs& a, int r, hipStream_t st) {
 
 // Rows per wave (or per workgroup at W = 4): fewer while there are too few rows to
 // fill the chip, more once x's registers and reduction are what a row costs (Q4_0,
-// 1 / 2 / 4 rows: 864 x 288 2.0 / 2.1 / 2.5 us, 2000 x 4064 4.04 / 3.82 / 3.98, 4096 x
-// 4064 6.6 / 5.8 / 5.5, 32000 x 288 6.6 / 4.9 / 4.4).
+// 1 / 2 / 4 rows: 300 x 768 2.03 / 2.15 / 2.67 us, 2048 x 768 2.57 / 2.47 / 2.92, 8192 x 768
+// 3.99 / 3.59 / 3.69, 32000 x 288 7.3 / 5.5 / 4.5; 2 / 4 rows: 1000 x 2080 2.81 / 2.94, 4096 x
+// 2080 4.41 / 4.06).
 template <int QT, bool GGUF>
 int wave_launch_fmt(const RowsArgs& a, hipStream_t st) {
-    const int np = (a.K / 8 + 63) / 64;
-    const int64_t weights = (int64_t)a.M * a.K;
-    int r = a.M <= 512 || (a.M <= 2048 && a.K <= 1024) ? 1 : weights <= (int64_t)8 << 20 && a.M <= 8192 ? 2 : 4;
+    int r = a.K <= kShortK ? (a.M <= 1024 ? 1 : a.M <= 10000 ? 2 : 4) : (a.M <= 512 ? 1 : a.M <= 3000 ? 2 : 4);
     if (a.post != kPostNone) r = std::max(r, 2);
-    if (np <= 1) return wave_launch_r<QT, GGUF, 1, 1>(a, r, st);
-    if (np <= 2) return wave_launch_r<QT, GGUF, 2, 1>(a, r, st);
+    const int np = (a.K / 8 + 63) / 64;  // passes of 64 items
+    if (a.K <= kShortK) return np <= 1 ? wave_launch_r<QT, GGUF, 1, 1>(a, r, st) : wave_launch_r<QT, GGUF, 2, 1>(a, r, st);
     // four waves share a row's columns: a wave holds at most 4 passes of x
-    if (np <= 4) return wave_launch_r<QT, GGUF, 1, 4>(a, r, st);
-    if (np <= 8) return wave_launch_r<QT, GGUF, 2, 4>(a, r, st);
-    if (np <= 12) return wave_launch_r<QT, GGUF, 3, 4>(a, r, st);
-    return wave_launch_r<QT, GGUF, 4, 4>(a, r, st);
+    switch ((np + 3) / 4) {
+        case 1: return wave_launch_r<QT, GGUF, 1, 4>(a, r, st);
+        case 2: return wave_launch_r<QT, GGUF, 2, 4>(a, r, st);
+        case 3: return wave_launch_r<QT, GGUF, 3, 4>(a, r, st);
+        default: return wave_launch_r<QT, GGUF, 4, 4>(a, r, st);
+    }
 }
 
-// matvec_wave up to 24 M weights (4096 x 5504 Q4_0 6.9 us against 7.7 of matvec_rows,
-// 11008 x 2080 9.3 / 10.8, 1000 x 5504 Q8_0 3.8 / 6.7), where a row's columns fit its
-// registers (K <= 8192); matvec_rows above (33000 x 4128 Q4_0 31 / 29 us, 4096 x 8032
-// Q8_0 11.5 / 10.3), and for many short rows past 512 columns (33000 x 544 8.0 / 6.9;
-// 32000 x 288 4.4 / 5.7).
+// Whether matvec_rows is faster than matvec_wave, which takes up to kWaveK columns: wide
+// loads and x shared by 16 waves, against no barrier before the weights.  Wave / rows, us:
+//   many short rows, several of them a pass: 32000 x 544 Q4_0 8.0 / 6.5, 20000 x 544 5.2 / 5.1,
+//     24000 x 1216 9.0 / 8.1, 16384 x 1216 7.1 / 6.8, 33000 x 1376 (four rows a unit no more)
+//     11.2 / 12.4; Q5_0, whose wave is the slowest, 12000 x 1216 7.8 / 6.4; Q8_0 24000 x 1216
+//     11.8 / 10.1, but 32000 x 768 8.8 / 9.2;
+//   Q5_0 blocks: 12000 x 1376 8.0 / 7.4, 8192 x 2080 9.5 / 8.5, 4096 x 3008 5.8 / 6.2;
+//   Q8_0: 8192 x 2080 8.4 / 7.6, 4096 x 2080 5.5 / 5.6, 16384 x 4128 21.3 / 18.0, 8192 x 5504
+//     13.5 / 13.0, 8192 x 4128 11.8 / 11.6, 4096 x 8032 10.5 / 10.9;
+//   Q4_0 blocks: 16384 x 4128 16.2 / 15.0, 33000 x 3008 20.2 / 22.0, 8192 x 5504 9.8 / 10.3;
+//   split Q4 and Q5: 33000 x 8032 39.8 / 36.2, 33000 x 5504 27.2 / 27.8.
+template <int QT, bool GGUF>
+bool rows_faster(const RowsArgs& a) {
+    constexpr bool k5 = QT == kRows5 && GGUF;
+    const int64_t m = (int64_t)a.M * a.K >> 20;  // weights, in 2^20
+    if (a.K > kWaveK) return true;
+    if (a.K <= 512) return false;
+    if (a.K <= kShortK) return QT != kRows8 && a.M > (k5 ? 14000 : 24000);
+    if (a.K <= 1344) return a.M > (k5 ? 10000 : 20000);
+    if (k5) return m >= (a.K <= 2048 ? 15 : 16);
+    if (QT == kRows8) return a.K > 2048 && m >= (a.K <= 4096 ? 16 : 40);
+    return GGUF ? a.K > 4096 && m >= 60 : a.K > 6144 && m >= 120;
+}
+
 template <int QT, bool GGUF>
 int rows_or_wave(const RowsArgs& a, hipStream_t st) {
-    const bool aligned = ((uintptr_t)a.x | (uintptr_t)(a.pre != kPreNone ? a.pre_arg : nullptr)) % 16 == 0;
-    const int64_t weights = (int64_t)a.M * a.K;
-    if (a.pre == kPreAttnMerge ||
-        (aligned && a.K <= 8192 && (a.K <= 512 || (a.M <= 16384 && weights <= (int64_t)24 << 20))))
-        return wave_launch_fmt<QT, GGUF>(a, st);
-    return rows_launch_fmt<QT, GGUF>(a, st);
+    return a.pre != kPreAttnMerge && rows_faster<QT, GGUF>(a) ? rows_launch_fmt<QT, GGUF>(a, st)
+                                                              : wave_launch_fmt<QT, GGUF>(a, st);
 }
 
 }  // namespace
@@ -626,7 +833,7 @@ bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const
     const size_t lds = (size_t)nb * kXPitch * 4 + (size_t)kWaves * (slot + 64 * 4);
     // the merge runs in every wave that reads x: small K only, and the head_dims of the merge launch
     if (o.pre == kPreAttnMerge &&
-        (!rows_before_stream(M, K) || o.attn_splits < 1 || o.attn_splits > kAttnMergeMaxSplits ||
+        (!rows_before_stream(K) || o.attn_splits < 1 || o.attn_splits > kAttnMergeMaxSplits ||
          !attn_head_dim(o.attn_hd) || K % o.attn_hd || (uintptr_t)o.pre_arg % 16))
         return false;
     return K > 0 && K % 32 == 0 && M > 0 && M <= INT32_MAX - 4096 && bytes < (int64_t)kPastEnd && lds <= kLdsBudget &&
@@ -637,7 +844,7 @@ bool matvec_rows_takes(int bits, bool gguf, const void* w, const void* qh, const
 int matvec_rows_launch(int bits, bool gguf, const void* w, const uint8_t* qh, const float* scales, const float* x,
                        float* y, int64_t M, int64_t K, hipStream_t st, const MatvecOpts& o) {
     RowsArgs a{static_cast<const uint8_t*>(w), qh, scales, x, o.pre_arg, y, (int)M, (int)K, o.pre, (int)o.accumulate,
-               o.post, 1, 0, 1, o.attn_splits, o.attn_hd, o.eps};
+               o.post, 1, 1, o.attn_splits, o.attn_hd, o.eps};
     switch (bits) {
         case 4: return gguf ? rows_or_wave<kRows4, true>(a, st) : rows_or_wave<kRows4, false>(a, st);
         case 5: return gguf ? rows_or_wave<kRows5, true>(a, st) : rows_or_wave<kRows5, false>(a, st);

@@ -53,8 +53,8 @@ extern "C" {
 
 /* Work fused into a matvec's read of x (asmhip_matmul_fused). */
 #define ASMHIP_PRE_NONE 0
-#define ASMHIP_PRE_RMSNORM 1 /* x <- (x * 1/sqrt(mean(x^2) + eps)) * pre_arg (the int8-MFMA stream
-                                * reads x * pre_arg and scales each row total by the
+#define ASMHIP_PRE_RMSNORM 1 /* x <- (x * 1/sqrt(mean(x^2) + eps)) * pre_arg (the int8-MFMA stream and the row kernels
+                                * read x * pre_arg and scale each row total by the
                                 * 1/sqrt factor: the same product, rounded in another
                                 * order, within the matvec bar) */
 #define ASMHIP_PRE_SWIGLU 2  /* x <- x / (1 + exp(-x)) * pre_arg             */
@@ -64,7 +64,7 @@ extern "C" {
  * keeps Q5_0 and Q8_0 on the fp32 kernels.  The MFMA stream needs
  * K % 256 == 0, K <= 16384 and 16-byte aligned x (and, for split planes,
  * 16-byte aligned planes). */
-#define ASMHIP_Q4_KERNEL_AUTO 0 /* int8 MFMA kernel where eligible and K > 1024 (K > 512 past 6144 rows), else fp32 */
+#define ASMHIP_Q4_KERNEL_AUTO 0 /* int8 MFMA kernel where eligible and K > 1024, else fp32 */
 #define ASMHIP_Q4_KERNEL_FP32 1 /* fp32 VALU kernel only                                   */
 #define ASMHIP_Q4_KERNEL_MFMA 2 /* int8 MFMA kernel only (GGUF shapes it cannot take:
                                    UNSUPPORTED; split planes fall back to fp32) */
@@ -302,8 +302,7 @@ ASMHIP_API int asmhip_attention_decode_rope_table(const float* qkv, void* k_cach
  * asmhip_matmul_attn_output then computes y = W . attn (accumulate: y += W .
  * attn) for GGUF blocks W [M][n_heads * head_dim / 32] (qtype Q4_0 or Q8_0),
  * where attn is the merged attention output.  The merge runs inside the matvec's
- * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024
- * (512 past 6144 rows),
+ * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024,
  * and for Q4_0 where the int8-MFMA stream takes the shape (head_dim 64 or 128, n_heads
  * * head_dim a multiple of 256 and at most 8192); otherwise a merge launch writes attn
  * to `work` (n_heads * head_dim floats) and a matvec reads it.  Results equal the

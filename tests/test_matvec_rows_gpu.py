@@ -91,6 +91,93 @@ def test_row_kernels_sums_in_64_bits(hip, q, split, M, K):
     assert (np.abs(y - e) <= bar).all()
 
 
+ROWS_KS = [288, 544, 768, 1024, 1056, 1376, 2048 + 32, 3008, 4128, 5504, 6176, 8160, 8224]
+
+
+def _prefixes(M):
+    return [m for m in (1, 5, 47, 300, 1000, 2049, 4097, 8193, 16400) if m < M]
+
+
+@pytest.mark.parametrize("q", [4, 5, 8])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("K", ROWS_KS)
+def test_rows_do_not_depend_on_the_number_of_rows(hip, q, split, K):
+    """A row's bits are the same for every M, whichever kernel its size picks: the leading
+    m rows of a matrix give the first m outputs of the whole."""
+    M = max(33001 if K <= 1056 else 0, (25 << 20) // K + 17)
+    rng = np.random.default_rng(K + q)
+    b, _ = _weights(rng, q, M, K)
+    x = (rng.standard_normal(K) * np.exp(rng.standard_normal(K))).astype(np.float32)
+    parts = {4: gguf.split_q4_0, 5: gguf.split_q5_0, 8: gguf.split_q8_0}[q](b) if split else [b]
+    bufs = [DeviceBuffer.from_numpy(np.ascontiguousarray(p).view(np.uint8)) for p in parts]
+    name = f"asmhip_matmul_q{q}_split" if split else f"asmhip_matmul_q{q}_0"
+    dx, dy = DeviceBuffer.from_numpy(x), DeviceBuffer(4 * M)
+
+    def run(m):
+        assert getattr(hip, name)(*[t.ptr for t in bufs], dx.ptr, dy.ptr, m, K, None) == 0, hip.asmhip_last_error()
+        return dy.download(np.uint32, (m,))
+
+    whole = run(M)
+    for m in _prefixes(M):
+        assert np.array_equal(run(m), whole[:m]), m
+
+
+@pytest.mark.parametrize("q", [4, 8])
+@pytest.mark.parametrize("K", [576, 768, 1088, 3008, 4160, 6208])
+@pytest.mark.parametrize("pre", ["rmsnorm", "swiglu"])
+@pytest.mark.parametrize("form", ["accumulate", "pairs"])
+def test_fused_rows_do_not_depend_on_the_number_of_rows(hip, q, K, pre, form):
+    M = max(33008 if K <= 1024 else 0, ((25 << 20) // K + 31) // 16 * 16)
+    rng = np.random.default_rng(K + q)
+    b, _ = _weights(rng, q, M, K)
+    x, arg, y0 = (rng.standard_normal(n).astype(np.float32) for n in (K, K, M))
+    op = {"rmsnorm": native.PRE_RMSNORM, "swiglu": native.PRE_SWIGLU}[pre]
+    qt = native.Q4_0 if q == 4 else native.Q8_0
+    db, dx, da, work = DeviceBuffer.from_numpy(b), DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(arg), DeviceBuffer(4 * M)
+
+    def run(m):
+        dy = DeviceBuffer.from_numpy(y0)
+        if form == "pairs":
+            rc = hip.asmhip_matmul_swiglu(qt, db.ptr, dx.ptr, dy.ptr, m // 2, K, op, da.ptr, 1e-5, work.ptr, None)
+        else:
+            rc = hip.asmhip_matmul_fused(qt, db.ptr, dx.ptr, dy.ptr, m, K, op, da.ptr, 1e-5, 1, None)
+        assert rc == 0, hip.asmhip_last_error()
+        return dy.download(np.uint32, (m // 2 if form == "pairs" else m,))
+
+    whole = run(M)
+    for m in (m // 16 * 16 + 16 for m in _prefixes(M - 16)):
+        y = run(m)
+        assert np.array_equal(y, whole[: len(y)]), m
+
+
+@pytest.mark.parametrize("q", [4, 8])
+@pytest.mark.parametrize("M,K", [(33000, 544), (26000, 1088), (13000, 2112), (9000, 3008), (4096, 5504), (17000, 4128)])
+def test_row_kernels_error_of_the_norm(hip, q, M, K):
+    """|y - y64| of a few thousand rows: 1.0e-7 of the norm with a lane's chains and a tree
+    above them (4.8e-8 with 64-bit sums, K <= 1024); a row's block products added one after
+    another in fp32 left 1.4e-7 to 2.0e-7 at these K from 1088 to 3008."""
+    rng = np.random.default_rng(M + K + q)
+    b, _ = _weights(rng, q, M, K)
+    x = rng.standard_normal(K).astype(np.float32)
+    y, n = _call(hip, q, False, b, x, M, K).astype(np.float64), 4000
+    w = (gguf.dequantize_q4_0 if q == 4 else gguf.dequantize_q8_0)(b[:n]).astype(np.float64).reshape(n, K)
+    e = w @ x.astype(np.float64)
+    assert np.linalg.norm(y[:n] - e) / np.linalg.norm(e) < (6e-8 if K <= 1024 else 1.2e-7)
+
+
+@pytest.mark.parametrize("q", [4, 5, 8])
+@pytest.mark.parametrize("M,K", [(300, 288), (2000, 1024), (700, 1088), (33000, 1088), (600, 5504), (70, 8224)])
+def test_row_kernels_x_off_16_bytes(hip, q, M, K):
+    rng = np.random.default_rng(M + K)
+    b, _ = _weights(rng, q, M, K)
+    x = rng.standard_normal(K + 4).astype(np.float32)
+    db, dx, dy = DeviceBuffer.from_numpy(b), DeviceBuffer.from_numpy(x), DeviceBuffer(4 * M)
+    fn = {4: hip.asmhip_matmul_q4_0, 5: hip.asmhip_matmul_q5_0, 8: hip.asmhip_matmul_q8_0}[q]
+    for off in (1, 2, 3):
+        assert fn(db.ptr, dx.ptr + 4 * off, dy.ptr, M, K, None) == 0, hip.asmhip_last_error()
+        assert np.array_equal(dy.download(np.float32, (M,)), _call(hip, q, False, b, x[off:off + K], M, K)), off
+
+
 @pytest.mark.parametrize("M,K", [(4096, 5504), (16400, 2080), (5000, 8224)])
 def test_row_kernels_many_units(hip, M, K):
     """Several units per wave, and rows cut into chunks (matvec_rows' stream)."""
