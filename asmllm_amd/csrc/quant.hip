@@ -94,67 +94,82 @@ __global__ __launch_bounds__(kThreads) void quantize_q4_kernel(const float* __re
 // values each, so that reads and writes are whole lines (one thread a block, with 128
 // bytes in and 34 out at its own stride: 200 x 11008 4.5 us a launch, 3.5 so, 24 x 4096
 // 2.6 / 2.0, of which an empty launch is 1.6).
-// OUT: GGUF blocks, the GEMM tile layout of activations (gemm_tiled_offset with
-// kGemmTileA-row tiles; padding rows are not written), or the split layout (qs planes
-// and the fp16 d widened to fp32).
-enum Q8Out : int { kOutBlocks = 0, kOutTiled = 1, kOutSplit = 2 };
 
-template <int OUT>
-__global__ __launch_bounds__(kThreads) void quantize_q8_kernel(const float* __restrict__ w, uint8_t* __restrict__ out,
-                                                               float* __restrict__ scales, int64_t nblocks, int64_t nb) {
+// A lane's four quants of the block whose values 4 part.. are v, and the block's fp16 d.
+__device__ __forceinline__ uint32_t quant_q8_lane(const float (&v)[4], unsigned short* dh) {
 #pragma clang fp contract(off)
+    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    amax = fmaxf(amax, 0.f);  // NaN values count for nothing, as in the host quantizer's maximum
+    auto with = [&](int o) { amax = fmaxf(amax, __int_as_float(o)); };
+    with(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), kDppQuadXor1, 0xF, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), kDppQuadXor2, 0xF, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), kDppRowHalfMirror, 0xF, 0xF, false));
+    const float d = amax / 127.0f;
+    const float inv = amax == 0.0f ? 0.0f : 127.0f / amax;
+    uint32_t q = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float r = rintf(v[j] * inv);
+        r = fminf(fmaxf(r, -128.0f), 127.0f);
+        q |= (uint32_t)(uint8_t)(int8_t)(int)r << (8 * j);
+    }
+    *dh = __half_as_ushort(__float2half_rn(d));
+    return q;
+}
+
+// GGUF blocks, or the split layout (qs planes and the fp16 d widened to fp32).
+template <bool SPLIT>
+__global__ __launch_bounds__(kThreads) void quantize_q8_kernel(const float* __restrict__ w, uint8_t* __restrict__ out,
+                                                               float* __restrict__ scales, int64_t nblocks) {
     const int part = threadIdx.x & 7;
     const int64_t stride = (int64_t)gridDim.x * (kThreads / 8);
     for (int64_t i = (int64_t)blockIdx.x * (kThreads / 8) + (threadIdx.x >> 3); i < nblocks; i += stride) {
         float v[4];
         __builtin_memcpy(v, w + i * 32 + 4 * part, sizeof(v));
-        float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-        amax = fmaxf(amax, 0.f);  // NaN values count for nothing, as in the host quantizer's maximum
-        auto with = [&](int o) { amax = fmaxf(amax, __int_as_float(o)); };
-        with(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), kDppQuadXor1, 0xF, 0xF, false));
-        with(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), kDppQuadXor2, 0xF, 0xF, false));
-        with(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), kDppRowHalfMirror, 0xF, 0xF, false));
-        const float d = amax / 127.0f;
-        const float inv = amax == 0.0f ? 0.0f : 127.0f / amax;
-        uint32_t q = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float r = rintf(v[j] * inv);
-            r = fminf(fmaxf(r, -128.0f), 127.0f);
-            q |= (uint32_t)(uint8_t)(int8_t)(int)r << (8 * j);
-        }
-        const unsigned short dh = __half_as_ushort(__float2half_rn(d));
-        if constexpr (OUT == kOutSplit) {
+        unsigned short dh;
+        const uint32_t q = quant_q8_lane(v, &dh);
+        if constexpr (SPLIT) {
             __builtin_memcpy(out + i * 32 + 4 * part, &q, 4);
             if (part == 0) scales[i] = __half2float(__ushort_as_half(dh));
         } else {
-            uint8_t* o = out;
-            if constexpr (OUT == kOutTiled) {
-                int64_t row, blk;
-                if (nblocks <= (int64_t)UINT32_MAX) {
-                    row = (uint32_t)i / (uint32_t)nb;
-                    blk = (uint32_t)i - (uint32_t)row * (uint32_t)nb;
-                } else {
-                    row = i / nb;
-                    blk = i - row * nb;
-                }
-                o += gemm_tiled_offset(row, blk, nb, kGemmTileA);
-            } else {
-                o += i * 34;
-            }
-            __builtin_memcpy(o + 2 + 4 * part, &q, 4);
-            if (part == 0) __builtin_memcpy(o, &dh, 2);
+            __builtin_memcpy(out + i * 34 + 2 + 4 * part, &q, 4);
+            if (part == 0) __builtin_memcpy(out + i * 34, &dh, 2);
         }
     }
 }
 
-int launch_q8(int out_kind, const float* w, void* out, float* scales, int64_t nblocks, int64_t nb, hipStream_t st) {
-    const int64_t groups = (nblocks + kThreads / 8 - 1) / (kThreads / 8);
-    const dim3 grid((unsigned)(groups < (1 << 22) ? groups : (1 << 22)));
-    const auto kern = out_kind == kOutSplit   ? quantize_q8_kernel<kOutSplit>
-                      : out_kind == kOutTiled ? quantize_q8_kernel<kOutTiled>
-                                              : quantize_q8_kernel<kOutBlocks>;
-    hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, st, w, (uint8_t*)out, scales, nblocks, nb);
+// The GEMM tile layout of activations (gemm_tiled_offset with kGemmTileA-row tiles; padding
+// rows are not written).  A workgroup takes 16 rows of one step of two blocks, which are
+// 1088 consecutive bytes there: 32 blocks of one row land 4352 bytes apart, and the 68
+// bytes of a row's step share their lines with other rows', which other dies then wrote
+// (512 x 4096 4.4 us so, 3.9 now, 200 x 11008 4.8 / 4.0; 32 or 64 rows a workgroup, whole
+// lines of them, 4.3 and 4.9).
+constexpr int kQuantRows = kThreads / 16;
+static_assert(kGemmTileA % kQuantRows == 0, "a workgroup's rows lie in one tile");
+__global__ __launch_bounds__(kThreads) void quantize_q8_tiled_kernel(const float* __restrict__ w,
+                                                                     uint8_t* __restrict__ out, int64_t rows, int64_t nb,
+                                                                     int64_t groups) {
+    const int part = threadIdx.x & 7, odd = (threadIdx.x >> 3) & 1, r = threadIdx.x >> 4;
+    const int64_t steps = nb >> 1;
+    for (int64_t g = blockIdx.x; g < groups; g += gridDim.x) {
+        const int64_t band = g / steps, blk = 2 * (g - band * steps) + odd, row = band * kQuantRows + r;
+        if (row >= rows) continue;  // the same for all eight lanes of a block
+        float v[4];
+        __builtin_memcpy(v, w + (row * nb + blk) * 32 + 4 * part, sizeof(v));
+        unsigned short dh;
+        const uint32_t q = quant_q8_lane(v, &dh);
+        uint8_t* o = out + gemm_tiled_offset(row, blk, nb, kGemmTileA);
+        __builtin_memcpy(o + 2 + 4 * part, &q, 4);
+        if (part == 0) __builtin_memcpy(o, &dh, 2);
+    }
+}
+
+unsigned capped_grid(int64_t groups) { return (unsigned)(groups < (1 << 22) ? groups : (1 << 22)); }
+
+int launch_q8(bool split, const float* w, void* out, float* scales, int64_t nblocks, hipStream_t st) {
+    const dim3 grid(capped_grid((nblocks + kThreads / 8 - 1) / (kThreads / 8)));
+    const auto kern = split ? quantize_q8_kernel<true> : quantize_q8_kernel<false>;
+    hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, st, w, (uint8_t*)out, scales, nblocks);
     ASMHIP_TRY(hipGetLastError());
     return kOk;
 }
@@ -223,7 +238,7 @@ int quantize_launch(QuantType qt, const float* w, void* blocks, int64_t rows, in
         hipLaunchKernelGGL(quantize_q4_kernel, dim3((unsigned)grid_for(nb)), dim3(kThreads), 0, st, w,
                            (uint8_t*)blocks, nb);
     else
-        return launch_q8(kOutBlocks, w, blocks, nullptr, nb, K / 32, st);
+        return launch_q8(false, w, blocks, nullptr, nb, st);
     ASMHIP_TRY(hipGetLastError());
     return kOk;
 }
@@ -233,7 +248,7 @@ int quantize_q8_split_launch(const float* w, int8_t* qs, float* scales, int64_t 
     if ((uintptr_t)qs % 16) return fail(kInvalidArgument, "quantize_q8_split: qs must be 16-byte aligned");
     const int64_t nb = rows * (K / 32);
     if (grid_for(nb) > INT32_MAX) return fail(kInvalidArgument, "quantize_q8_split: tensor too large");
-    return launch_q8(kOutSplit, w, qs, scales, nb, K / 32, st);
+    return launch_q8(true, w, qs, scales, nb, st);
 }
 
 int quantize_q8_0_tiled_launch(const float* x, void* tiled, int64_t rows, int64_t K, hipStream_t st) {
@@ -241,7 +256,11 @@ int quantize_q8_0_tiled_launch(const float* x, void* tiled, int64_t rows, int64_
     if (!x || !tiled) return fail(kInvalidArgument, "quantize_q8_0_tiled: null pointer");
     const int64_t nb = rows * (K / 32);
     if (grid_for(nb) > INT32_MAX) return fail(kInvalidArgument, "quantize_q8_0_tiled: tensor too large");
-    return launch_q8(kOutTiled, x, tiled, nullptr, nb, K / 32, st);
+    const int64_t groups = (rows + kQuantRows - 1) / kQuantRows * (K / 64);
+    hipLaunchKernelGGL(quantize_q8_tiled_kernel, dim3(capped_grid(groups)), dim3(kThreads), 0, st, x, (uint8_t*)tiled, rows,
+                       K / 32, groups);
+    ASMHIP_TRY(hipGetLastError());
+    return kOk;
 }
 
 int random_blocks_launch(QuantType qt, void* blocks, int64_t rows, int64_t K, uint64_t seed, float stddev,

@@ -335,3 +335,22 @@ def test_gemm_tiled_rejects_bad_arguments(hip):
     assert hip.asmhip_gemm_q8_0_tile_weights(p, p, 4, 96, None) == bad
     assert hip.asmhip_gemm_q8_0_tile_activations(p + 2, p, 4, 64, None) == bad
     assert hip.asmhip_quantize_q8_0_tiled(p, p, 4, 32, None) == bad
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 63, 64, 65, 129, 200])
+@pytest.mark.parametrize("K", [64, 192, 4096])
+def test_tiled_quantizer_edges(hip, T, K):
+    """Bands of 16 rows that end inside, at and past the last row and the 64-row tile: the
+    blocks of asmhip_quantize in the tile layout, an infinity and a NaN among the values,
+    and no byte of the padding rows written."""
+    x = np.random.default_rng(T + K).standard_normal((T, K)).astype(np.float32)
+    x[T // 2, 0], x[T - 1, K - 1], x[0, 33] = np.inf, np.nan, 0.0
+    dx, db = DeviceBuffer.from_numpy(x), DeviceBuffer(gguf.q8_0_nbytes(T, K))
+    n = hip.asmhip_gemm_q8_0_tiled_activation_bytes(T, K)
+    dt = DeviceBuffer.from_numpy(np.full(n, 0xA5, np.uint8))
+    assert hip.asmhip_quantize(native.Q8_0, dx.ptr, db.ptr, T, K, None) == 0, hip.asmhip_last_error()
+    assert hip.asmhip_quantize_q8_0_tiled(dx.ptr, dt.ptr, T, K, None) == 0, hip.asmhip_last_error()
+    got = dt.download(np.uint8, n).reshape(-1, K // 64, 64, 68).transpose(0, 2, 1, 3).reshape(-1, K // 64, 68)
+    want = db.download(np.uint8, (T, K // 64, 68))  # a step's two blocks of a row are consecutive in both layouts
+    assert np.array_equal(got[:T], want)
+    assert np.all(got[T:] == 0xA5)
