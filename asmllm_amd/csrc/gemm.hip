@@ -758,6 +758,7 @@ struct Narrow {
     // two such workgroups share a unit (200 x 4096 x 11008 split 71 us; 101 with three)
     static constexpr int S = MW > 1 ? 2 : 3;
     static_assert((S - 1) * kPerWave < 64, "the wait counts to 63");
+    static_assert(FORM != kNarrowBlocks || 34 * B % 16 == 0, "a step moves a row's aligned window by whole 16 bytes");
 };
 
 struct NarrowArgs {
@@ -830,9 +831,7 @@ __global__ __launch_bounds__((Narrow<FORM, NW, MW>::kThreads)) void gemm_narrow(
         off[u] = o;
     }
     auto fetch = [&](int stage, int s) {
-        // blocks: in whole 16 bytes, so that the loads stay aligned (a step of four starts 8
-        // bytes on in its rows' windows every other time)
-        const uint32_t wofs = (uint32_t)s * (uint32_t)(FORM == kNarrowTiled ? N::B / 2 * kGemmTileW * 68 : FORM == kNarrowSplit ? 32 * N::B : 34 * N::B) & (FORM == kNarrowBlocks ? ~15u : ~0u);
+        const uint32_t wofs = (uint32_t)s * (uint32_t)(FORM == kNarrowTiled ? N::B / 2 * kGemmTileW * 68 : FORM == kNarrowSplit ? 32 * N::B : 34 * N::B);
         const uint32_t aofs = FORM == kNarrowTiled ? (uint32_t)s * (uint32_t)(N::B / 2 * kGemmTileA * 68) : wofs;
         const v4i wr = raw_rsrc(wbase + wofs, wsize - wofs), ar = raw_rsrc(abase + aofs, asize - aofs);
 #pragma unroll
@@ -937,7 +936,7 @@ __global__ __launch_bounds__((Narrow<FORM, NW, MW>::kThreads)) void gemm_narrow(
         // stage `next` was read in step s - 1, which every wave finished before the
         // barrier; past the end the last step is loaded again
         if (loads) fetch(next, min(s + N::S - 1, nsteps - 1));
-        const uint8_t* stage = lds + cur * N::kStage + (FORM == kNarrowBlocks ? (34 * N::B * s) & 15 : 0);
+        const uint8_t* stage = lds + cur * N::kStage;
         if (wave < N::kTiles) {
             // the step's operands, then its matrix instructions, then its sums: one block
             // after another a wave waited for each read, product and conversion in turn
