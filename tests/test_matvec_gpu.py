@@ -520,7 +520,7 @@ def _swiglu(hip, qtype, gu, x, pre, arg, eps):
 
 @pytest.mark.parametrize("qt,kernel,H,K,pre", [
     ("q4", native.Q4_KERNEL_AUTO, 5504, 4096, "rmsnorm"),   # the 7B FFN: one MFMA-stream launch
-    ("q4", native.Q4_KERNEL_FP32, 5504, 4096, "rmsnorm"),   # fp32 kernel into work, then the pairs kernel
+    ("q4", native.Q4_KERNEL_FP32, 5504, 4096, "rmsnorm"),   # the row kernels: one launch too
     ("q4", native.Q4_KERNEL_AUTO, 768, 288, "none"),        # stories15M: K = 288 is no MFMA-stream shape
     ("q4", native.Q4_KERNEL_AUTO, 1000, 2048, "none"),      # 125 tiles, the general (K != 4096) stream
     ("q8", native.Q4_KERNEL_AUTO, 1000, 4096, "none"),

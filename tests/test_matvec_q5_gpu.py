@@ -6,8 +6,8 @@ fp32 scales; the GPU also reads the same values as 22-byte GGUF Q5_0 blocks
 in place.  Bar: dequantized values bit-exact; every output row within
 1e-4 x sum_k |w[m,k]| |x[k]| of the oracle on the same bytes; the
 reference's golden inputs within TOLERANCE_Q5 (test_runner.py:35).  GGUF
-blocks with K % 256 == 0 take the int8-MFMA stream, everything else the fp32
-VALU kernels.
+blocks and split planes with K % 256 == 0 above 1024 take the int8-MFMA stream,
+everything else the fp32 VALU kernels.
 """
 
 import numpy as np
@@ -88,8 +88,8 @@ def test_q5_mt_and_dispatch_bitwise(hip, oracle):
     np.testing.assert_array_equal(dy.download(np.float32, 1000), ref)
 
 
-# (M, K): pair kernel at R = 1, 2, 4 (rows per wave); odd K/32 and K too large
-# for the LDS copy of x take the generic kernel.
+# (M, K): the row kernels (K <= 1024, and every K % 256 != 0), the int8-MFMA stream (the
+# other K), and the generic kernel where x is too large for LDS.
 SHAPES = [(1, 64), (7, 64), (33, 256), (64, 4096), (3000, 4096), (11008, 4096), (4096, 11008),
           (1, 32), (300, 2336), (5, 40000)]
 
@@ -104,19 +104,20 @@ def test_q5_split_and_gguf_match_oracle(hip, oracle, M, K):
     blocks = gguf.pack_q5_0(ql, qh, d)
     y_gguf = _gguf_device(hip, blocks, x)
     assert_matvec_close(y_gguf, oracle.matmul_q5_0_gguf(blocks, x, NT), w, x)
-    # the same values in the two layouts (GGUF blocks take the int8-MFMA stream where
-    # K % 256 == 0, the split planes the fp32 VALU kernel): within the bar of each other
+    # the same values in the two layouts: within the bar of each other
     assert_matvec_close(y_gguf, y_split, w, x)
 
 
 def test_q5_unaligned_qh_takes_the_generic_kernel(hip, oracle):
     ql, qh, d, x = _q5(42, 200, 1024)
     s = d.astype(np.float32)
-    y_pairs = _split_device(hip, ql, qh, s, x)
-    y_generic = _split_device(hip, ql, qh, s, x, qh_offset=4)  # qh only dword aligned
+    y_rows = _split_device(hip, ql, qh, s, x)
+    y_dword = _split_device(hip, ql, qh, s, x, qh_offset=4)    # dword aligned: the row kernels still
+    y_generic = _split_device(hip, ql, qh, s, x, qh_offset=2)  # they refuse it
     w = ops_ref.dequantize_q5_0(ql, qh, s)
     ref = oracle.matmul_q5(ql, qh, s, x)
-    assert_matvec_close(y_pairs, ref, w, x)
+    assert_matvec_close(y_rows, ref, w, x)
+    np.testing.assert_array_equal(y_dword, y_rows)
     assert_matvec_close(y_generic, ref, w, x)
 
 
