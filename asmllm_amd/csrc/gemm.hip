@@ -721,8 +721,8 @@ __global__ __launch_bounds__(kSplitThreads) void gemm_q8_split(const int8_t* __r
 // two steps in flight.  Bound by the issue of one wave's operand reads, matrix
 // instructions and sums at the smallest T (about 1000 cycles for eight blocks: the sums
 // of an output follow each other, so its blocks stay with one wave), and by the LDS reads
-// and vector work of 16x16 tiles, about 1.6 times the 32x32 tile's per output, at larger
-// T.
+// (58% of the time at 200 x 4096 x 11008 split, half of it bank conflicts) and vector work
+// (39%) of 16x16 tiles, about 1.6 times the 32x32 tile's per output, at larger T.
 // ---------------------------------------------------------------------------
 enum NarrowForm : int { kNarrowBlocks = 0, kNarrowTiled = 1, kNarrowSplit = 2 };
 
@@ -733,9 +733,9 @@ struct Narrow {
     // unit (200 x 4096 x 11008 71 -> 65 us; 93 -> 102 for the split planes' 128-byte runs)
     static constexpr int B = FORM == kNarrowTiled && NW == 4 ? 4 : 8;
     // 16-byte slots of a region: rows of kPitchSlots (blocks: the 34 B bytes of a step in
-    // their aligned window, plus one; split: 32 B bytes plus one; all pitches keep the
-    // operand reads of 16 rows on distinct banks), or the B / 2 16-row pair steps of the
-    // tile layout (68 bytes a row)
+    // their aligned window, plus one; split: 32 B bytes plus one: eight rows on distinct
+    // banks, rows m and m + 8 of an operand read on the same, half of the cycles LDS is
+    // active), or the B / 2 16-row pair steps of the tile layout (68 bytes a row)
     static constexpr int kReal = FORM == kNarrowSplit ? 2 * B : (34 * B + 12 + 15) / 16, kPitchSlots = kReal + 1;
     static constexpr int kPitch = 16 * kPitchSlots;
     static constexpr int kRowSlots = FORM == kNarrowTiled ? B / 2 * 68 : 16 * kPitchSlots;  // of 16 rows
