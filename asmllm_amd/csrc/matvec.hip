@@ -13,7 +13,7 @@
 //
 // The dispatch at the end sends a shape to the int8-MFMA stream (matvec_mfma.hip), to
 // the row kernels (matvec_rows.hip), or here: the pair kernels take rows too long for
-// the row kernels' LDS (K above about 21000, K % 64 == 0), the generic ones everything
+// the row kernels' LDS (K above about 25400, Q8 21700, and K % 64 == 0), the generic ones everything
 // else (operands without 4-byte alignment, x too large for LDS).
 //
 // Work mapping (one wave = 64 lanes):

@@ -744,15 +744,20 @@ int rows_launch_mode(RowsArgs a, hipStream_t st) {
     return kOk;
 }
 
-// More than 512 columns (16 blocks)
+// More than 512 columns (16 blocks): the shapes that rows_faster sends here, as many
+// blocks a lane as LDS holds beside x.
 template <int QT, bool GGUF>
 int rows_launch_fmt(const RowsArgs& a, hipStream_t st) {
-    if (a.K <= kShortK) return rows_launch_mode<QT, GGUF, kPack64>(a, st);
+    if constexpr (QT != kRows8)
+        if (a.K <= kShortK) return rows_launch_mode<QT, GGUF, kPack64>(a, st);
     if (a.K <= 2048) return rows_launch_mode<QT, GGUF, kPack32>(a, st);
-    // as many blocks a lane as LDS holds beside x
-    if (a.K <= 4096) return rows_launch_mode<QT, GGUF, QT == kRows8 ? 2 : kTwo>(a, st);
-    if (a.K <= 6144) return rows_launch_mode<QT, GGUF, 3>(a, st);
-    if (a.K <= 8192) return rows_launch_mode<QT, GGUF, QT == kRows8 ? 2 : 4>(a, st);
+    if constexpr (QT == kRows5 && GGUF)
+        if (a.K <= 4096) return rows_launch_mode<QT, GGUF, kTwo>(a, st);
+    if constexpr (QT == kRows8) {
+        if (a.K <= 4096 || (a.K > 6144 && a.K <= 8192)) return rows_launch_mode<QT, GGUF, 2>(a, st);
+    } else {
+        if (a.K > 6144 && a.K <= 8192) return rows_launch_mode<QT, GGUF, 4>(a, st);
+    }
     return rows_lds<QT, GGUF, 3>(a.K / 32) <= kLdsBudget ? rows_launch_mode<QT, GGUF, 3>(a, st)
                                                          : rows_launch_mode<QT, GGUF, 1>(a, st);
 }

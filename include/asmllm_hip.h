@@ -180,7 +180,7 @@ ASMHIP_API int asmhip_matmul_swiglu(int qtype, const void* blocks, const float* 
  * swiglu != 0: W's rows interleave gate and up in groups of 8 (M % 16 == 0) and
  * h = silu(gate) * up is written instead, M / 2 floats, as asmhip_matmul_swiglu
  * writes it.  y must not overlap x.  ASMHIP_ERR_UNSUPPORTED where the row kernels do
- * not take the shape (K above about 21000, a matrix of 4 GB, operands not 4-byte
+ * not take the shape (K above about 25400, Q8_0 21700, a matrix of 4 GB, operands not 4-byte
  * aligned), and for Q4_0 under ASMHIP_Q4_KERNEL_MFMA. */
 ASMHIP_API int asmhip_matmul_rmsnorm(int qtype, const void* blocks, const float* x, const float* norm, float eps,
                                      float* y, int64_t M, int64_t K, int swiglu, void* stream);
