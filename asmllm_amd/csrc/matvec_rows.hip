@@ -139,6 +139,12 @@ __device__ __forceinline__ void item_of(const uint32_t* q, uint32_t nh, const fl
     *xl = xb + (k8 ? 8 * g : 4 * g), *xh = xb + (k8 ? 8 * g + 4 : 16 + 4 * g);
 }
 
+// A row's total times RMSNorm's factor, rounded in both kernels: never part of an fma with y
+__device__ __forceinline__ float scaled_total(float tot, float inv) {
+#pragma clang fp contract(off)
+    return tot * inv;
+}
+
 // Sum over the squares of x (RMSNorm) in the order of the items: one wave's NP passes from
 // item `first` on
 template <int QT, int NP>
@@ -516,7 +522,7 @@ __global__ __launch_bounds__(kWaves * 64) void matvec_rows(const RowsArgs a) {
             ++c;
             continue;
         }
-        sum = __fmul_rn(sum, inv);
+        sum = scaled_total(sum, inv);
         const int row = tile_row + wave * rw + r;
         if (a.post == kPostNone) {
             if (owner && row < a.M) a.y[row] = a.accumulate ? a.y[row] + sum : sum;
@@ -690,7 +696,7 @@ __global__ __launch_bounds__(kWaveThreads) void matvec_wave(const RowsArgs a) {
 #pragma unroll
         for (int k = 0; k < W; ++k) ss += red[R][k], tot += red[lane % R][k];
     }
-    if (pre == kPreRmsNorm) tot = __fmul_rn(tot, 1.0f / sqrtf(ss / (float)a.K + a.eps));
+    if (pre == kPreRmsNorm) tot = scaled_total(tot, 1.0f / sqrtf(ss / (float)a.K + a.eps));
     if (a.post == kPostNone) {
         const int row = gw * R + lane;
         if (lane < R && row < a.M) a.y[row] = a.accumulate ? a.y[row] + tot : tot;

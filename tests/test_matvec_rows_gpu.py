@@ -38,6 +38,12 @@ def _weights(rng, q, M, K):
     return np.ascontiguousarray(b), (v * d[..., None].astype(np.float64)).reshape(M, K)
 
 
+def _long(rng, q, M, K):
+    """M rows, the first 256 again and again, and their exact matrix."""
+    b, w = _weights(rng, q, 256, K)
+    return np.ascontiguousarray(np.concatenate([b] * (M // 256 + 1))[:M]), w, np.arange(M) % 256
+
+
 def _bar(w, x, K):
     return (48 + min(K / 32, 96) + K / 2048) * 2.0 ** -24 * (np.abs(w) @ np.abs(x).astype(np.float64)) + 1e-30
 
@@ -98,6 +104,11 @@ def test_row_kernels_sums_in_64_bits(hip, q, split, M, K):
 ROWS_KS = [288, 544, 768, 1024, 1056, 1376, 2048 + 32, 3008, 4128, 5504, 6176, 8160, 8224]
 
 
+def _rows_of_both_kernels(K):
+    """Rows enough for every format that leaves matvec_wave at this K."""
+    return max(33008, (25 << 20) // K + 31) // 16 * 16 if K <= 1376 else ((122 if K > 4096 else 25) << 20) // K // 16 * 16 + 16
+
+
 def _prefixes(M):
     return [m for m in (1, 5, 47, 300, 1000, 2049, 4097, 8193, 16400) if m < M]
 
@@ -106,11 +117,12 @@ def _prefixes(M):
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("K", ROWS_KS)
 def test_rows_do_not_depend_on_the_number_of_rows(hip, q, split, K):
-    """A row's bits are the same for every M, whichever kernel its size picks: the leading
-    m rows of a matrix give the first m outputs of the whole."""
-    M = max(33001 if K <= 1056 else 0, (25 << 20) // K + 17)
+    """A row's bits are the same for every M, whichever kernel its size picks, and wherever
+    the row stands: the leading m rows of a matrix give the first m outputs of the whole,
+    whose 256 rows come again and again."""
+    M = _rows_of_both_kernels(K) + 1
     rng = np.random.default_rng(K + q)
-    b, _ = _weights(rng, q, M, K)
+    b, _, row = _long(rng, q, M, K)
     x = (rng.standard_normal(K) * np.exp(rng.standard_normal(K))).astype(np.float32)
     parts = {4: gguf.split_q4_0, 5: gguf.split_q5_0, 8: gguf.split_q8_0}[q](b) if split else [b]
     bufs = [DeviceBuffer.from_numpy(np.ascontiguousarray(p).view(np.uint8)) for p in parts]
@@ -122,18 +134,19 @@ def test_rows_do_not_depend_on_the_number_of_rows(hip, q, split, K):
         return dy.download(np.uint32, (m,))
 
     whole = run(M)
+    assert np.array_equal(whole, whole[row])
     for m in _prefixes(M):
         assert np.array_equal(run(m), whole[:m]), m
 
 
 @pytest.mark.parametrize("q", [4, 8])
-@pytest.mark.parametrize("K", [576, 768, 1088, 3008, 4160, 6208])
+@pytest.mark.parametrize("K", [576, 768, 1088, 3008, 4160, 6208, 8000])
 @pytest.mark.parametrize("pre", ["rmsnorm", "swiglu"])
 @pytest.mark.parametrize("form", ["accumulate", "pairs"])
 def test_fused_rows_do_not_depend_on_the_number_of_rows(hip, q, K, pre, form):
-    M = max(33008 if K <= 1024 else 0, ((25 << 20) // K + 31) // 16 * 16)
+    M = _rows_of_both_kernels(K)
     rng = np.random.default_rng(K + q)
-    b, _ = _weights(rng, q, M, K)
+    b = _long(rng, q, M, K)[0]
     x, arg, y0 = (rng.standard_normal(n).astype(np.float32) for n in (K, K, M))
     op = {"rmsnorm": native.PRE_RMSNORM, "swiglu": native.PRE_SWIGLU}[pre]
     qt = native.Q4_0 if q == 4 else native.Q8_0
@@ -312,12 +325,6 @@ def test_swiglu_over_its_inputs(hip, qt, H, K, pre, over):
 # Above about 25400 columns (Q8: 21700) x no longer fits LDS beside a unit of the row kernels:
 # up to 38400 the pair kernels take K % 64 == 0, in forms of 1, 2, 4 and (Q4) 8 rows a wave.
 LONG = [(40, 25600), (7, 38400), (4100, 25600), (8200, 32768), (16400, 25600)]
-
-
-def _long(rng, q, M, K):
-    """M rows, the first 256 again and again, and their exact matrix."""
-    b, w = _weights(rng, q, 256, K)
-    return np.ascontiguousarray(np.concatenate([b] * (M // 256 + 1))[:M]), w, np.arange(M) % 256
 
 
 @pytest.mark.parametrize("q", [4, 5, 8])
