@@ -111,8 +111,8 @@ struct KTile {
 template <int NJ, bool FULL, int NW>
 __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restrict__ q,
                                                             const float* __restrict__ k,
-                                                            const float* __restrict__ v, float* y, int seq, int hd_,
-                                                            float scale) {
+                                                            const float* __restrict__ v, int seq, int hd_,
+                                                            float scale, float sign, float slack, float* y) {
     constexpr int NU = (NJ + 3) / 4;  // 64-dimension groups of the second product
     constexpr int HDP = 64 * NU;
     const int hd = FULL ? 16 * NJ : hd_;
@@ -158,11 +158,10 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma16(const float* __restr
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[u][t] = v4f{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, ms = m, l = 0.f;  // ms: m scale
-    const float sign = scale < 0.f ? -1.f : scale == 0.f ? 0.f : 1.f;
+    if (sign != 1.f) {  // not otherwise: no wait for q before the first keys are requested
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) qv[j] *= sign;
-    scale = scale == 0.f ? 1.f : fabsf(scale) * 1.44269504088896340736f;
-    const float slack = kSlack / scale;
+        for (int j = 0; j < NJ; ++j) qv[j] *= sign;
+    }
 
     for (int b = wave; b < nblk; b += NW) {
         const auto vr = rows_at(v, b, seq, hd);
@@ -274,8 +273,8 @@ __device__ __forceinline__ void half_pair(float v, float* lo, float* hi) {
 
 template <int NJ, bool FULL, int NW>
 __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restrict__ q, const float* __restrict__ k,
-                                                           const float* __restrict__ v, float* y, int seq, int hd_,
-                                                           float scale) {
+                                                           const float* __restrict__ v, int seq, int hd_, float scale,
+                                                           float sign, float slack, float* y) {
     constexpr int HDP = NJ <= 4 ? 64 : 128;
     constexpr int NV = HDP / 16;  // 16-byte-a-lane loads of V per block
     const int hd = FULL ? 16 * NJ : hd_;
@@ -298,20 +297,21 @@ __global__ __launch_bounds__(NW * 64) void attention_mfma4(const float* __restri
     const uint32_t voff0 = vdim < hd ? (uint32_t)vkey * row_bytes + 4u * (uint32_t)vdim : kRowPastEnd;
     v4f qv[NJ];
     const int nblk = (seq + 15) >> 4;
-    {
+    // the idle waves of a short prompt leave q alone, whose requests would hold up the others'
+    // (64 x 128 6.3 us with them, 4.3 without)
+    if (wave < nblk) {
         const auto qr = make_rsrc(q + (size_t)row0 * hd, (uint32_t)(seq - row0) * row_bytes);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) qv[j] = load4(qr, off(qi, 16 * j + (lane & 12)));
+        if (sign != 1.f) {  // not otherwise: no wait for q before the first keys are requested
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) qv[j] *= sign;
+        }
     }
     v4f acc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, ms = m, l = 0.f, lo, hi;  // ms: m scale
-    const float sign = scale < 0.f ? -1.f : scale == 0.f ? 0.f : 1.f;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) qv[j] *= sign;
-    scale = scale == 0.f ? 1.f : fabsf(scale) * 1.44269504088896340736f;
-    const float slack = kSlack / scale;
 
     for (int b = wave; b < nblk; b += NW) {
         const auto kr = rows_at(k, b, seq, hd), vr = rows_at(v, b, seq, hd);
@@ -462,12 +462,17 @@ __global__ __launch_bounds__(kRowThreads) void attention_rows(const float* __res
 // head_dim 128, 1024 rows 15.9 us against 22.3 with 16-row tiles on 64 units (one
 // workgroup per row and scalar dots before: 274), 64 x 128 4.3 against 4.5, head_dim
 // 64, 1024 rows 10.1 against 12.8.  Past that they take a second round and read k and
-// v four times as often: 1100 rows 29.2 against 24.2, 2048 rows 49.2 against 39.9.
+// v four times as often: 1100 rows 29.2 against 22.7, 2048 rows 49.2 against 37.9.
 constexpr int kFourRowSeq = 1024;
 
 template <int NJ, bool FULL>
-int launch_mfma(const float* q, const float* k, const float* v, float* y, int seq, int hd, float scale,
+int launch_mfma(const float* q, const float* k, const float* v, float* y, int seq, int hd, float factor,
                 hipStream_t st) {
+    // the score's scale as the kernels take it: > 0 with log2(e); its slack; q's factor 1, -1 or
+    // 0.  The first ten dwords of the arguments are in registers when a wave starts; a factor
+    // that came by a load, before the first keys were requested, cost 64 x 128 2 us of 4.3.
+    const float scale = factor == 0.f ? 1.f : fabsf(factor) * 1.44269504088896340736f, slack = kSlack / scale;
+    const float sign = factor < 0.f ? -1.f : factor == 0.f ? 0.f : 1.f;
     if constexpr (NJ <= 8) {
         if (seq <= kFourRowSeq) {
             constexpr int NW = 16, HDP = NJ <= 4 ? 64 : 128;
@@ -475,7 +480,7 @@ int launch_mfma(const float* q, const float* k, const float* v, float* y, int se
             const int rc = dynamic_lds((const void*)attention_mfma4<NJ, FULL, NW>, lds);
             if (rc) return rc;
             hipLaunchKernelGGL((attention_mfma4<NJ, FULL, NW>), dim3((unsigned)((seq + 3) / 4)), dim3(NW * 64), lds, st,
-                               q, k, v, y, seq, hd, scale);
+                               q, k, v, seq, hd, scale, sign, slack, y);
             return kOk;
         }
     }
@@ -484,7 +489,7 @@ int launch_mfma(const float* q, const float* k, const float* v, float* y, int se
     const int rc = dynamic_lds((const void*)attention_mfma16<NJ, FULL, NW>, lds);
     if (rc) return rc;
     hipLaunchKernelGGL((attention_mfma16<NJ, FULL, NW>), dim3((unsigned)((seq + 15) / 16)), dim3(NW * 64), lds, st, q,
-                       k, v, y, seq, hd, scale);
+                       k, v, seq, hd, scale, sign, slack, y);
     return kOk;
 }
 
