@@ -104,7 +104,7 @@ struct KTile {
 // consecutive lanes, as the operand wants them, touches four cache lines per four
 // lanes.  The next block's K is in flight while a block is multiplied.  Bound by the
 // fp32 matrix rate of the compute units a prompt's tiles reach (2048 x 128: 128 of
-// 256, 39.9 us for 2.1 GFLOP) and the vector work beside it: 46 us with a rescaling
+// 256, 37.3 us for 2.1 GFLOP) and the vector work beside it: 46 us with a rescaling
 // and expf in every block.
 // NJ: 16-dimension groups; FULL: head_dim = 16 NJ, else the dimensions past it load
 // zeros.
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(kRowThreads) void attention_rows(const float* __res
 // head_dim 128, 1024 rows 15.9 us against 22.3 with 16-row tiles on 64 units (one
 // workgroup per row and scalar dots before: 274), 64 x 128 4.3 against 4.5, head_dim
 // 64, 1024 rows 10.1 against 12.8.  Past that they take a second round and read k and
-// v four times as often: 1100 rows 29.2 against 22.7, 2048 rows 49.2 against 37.9.
+// v four times as often: 1100 rows 29.2 against 22.7, 2048 rows 49.2 against 37.3.
 constexpr int kFourRowSeq = 1024;
 
 template <int NJ, bool FULL>
