@@ -721,9 +721,11 @@ extern "C" int asmhip_matmul_attn_output(int qtype, const void* blocks, const fl
     // one launch where the matvec kernel of the shape takes the merge as its x prologue
     const int bits = qt == QuantType::Q4_0 ? 4 : 8, sel = get_q4_kernel();
     if (rows_before_stream(K) && !(sel == kQ4KernelMfma && qt == QuantType::Q4_0) &&
-        matvec_rows_takes(bits, true, blocks, nullptr, nullptr, workspace, M, K, o))
-        return matvec_rows_launch(bits, true, blocks, nullptr, nullptr, workspace, y, M, K, st, o);
-    if (sel != kQ4KernelFp32) {
+        matvec_rows_takes(bits, true, blocks, nullptr, nullptr, workspace, M, K, o)) {
+        // every wave merges all of x: not for many rows (the same bits either way)
+        if (K <= 512 || M <= 6144)
+            return matvec_rows_launch(bits, true, blocks, nullptr, nullptr, workspace, y, M, K, st, o);
+    } else if (sel != kQ4KernelFp32) {
         if (qt == QuantType::Q4_0 && q4_0_mfma_eligible(blocks, workspace, o, M, K))
             return q4_0_mfma_launch(blocks, workspace, y, M, K, st, o);
         if (qt == QuantType::Q8_0 && q8_0_mfma_eligible(blocks, workspace, o, M, K))

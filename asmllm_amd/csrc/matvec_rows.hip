@@ -754,8 +754,7 @@ int rows_launch_mode(RowsArgs a, hipStream_t st) {
 // blocks a lane as LDS holds beside x.
 template <int QT, bool GGUF>
 int rows_launch_fmt(const RowsArgs& a, hipStream_t st) {
-    if constexpr (QT != kRows8)
-        if (a.K <= kShortK) return rows_launch_mode<QT, GGUF, kPack64>(a, st);
+    if (a.K <= kShortK) return rows_launch_mode<QT, GGUF, kPack64>(a, st);
     if (a.K <= 2048) return rows_launch_mode<QT, GGUF, kPack32>(a, st);
     if constexpr (QT == kRows5 && GGUF)
         if (a.K <= 4096) return rows_launch_mode<QT, GGUF, kTwo>(a, st);
@@ -792,6 +791,10 @@ int wave_launch_r(const RowsArgs& a, int r, hipStream_t st) {
 template <int QT, bool GGUF>
 int wave_launch_fmt(const RowsArgs& a, hipStream_t st) {
     int r = a.K <= kShortK ? (a.M <= 1024 ? 1 : a.M <= 10000 ? 2 : 4) : (a.M <= 512 ? 1 : a.M <= 3000 ? 2 : 4);
+    // every wave forms the SwiGLU of x anew, eight exponentials and divisions a pass and lane,
+    // for R rows (Q4_0, 2 / 4 rows: 2048 x 576 3.25 / 3.62 us, 4096 x 576 4.21 / 3.69; 512 x 2112
+    // 3.36 / 3.60, 1024 x 2112 4.28 / 3.67)
+    if (a.pre == kPreSwiGlu) r = a.K <= kShortK ? (a.M <= 1024 ? 1 : a.M <= 3000 ? 2 : 4) : a.M <= 700 ? 2 : 4;
     if (a.post != kPostNone) r = std::max(r, 2);
     const int np = (a.K / 8 + 63) / 64;  // passes of 64 items
     if (a.K <= kShortK) return np <= 1 ? wave_launch_r<QT, GGUF, 1, 1>(a, r, st) : wave_launch_r<QT, GGUF, 2, 1>(a, r, st);
@@ -821,6 +824,10 @@ bool rows_faster(const RowsArgs& a) {
     const int64_t m = (int64_t)a.M * a.K >> 20;  // weights, in 2^20
     if (a.K > kWaveK) return true;
     if (a.K <= 512) return false;
+    // matvec_rows forms the SwiGLU of x once for 16 waves and all their rows (wave / rows, us:
+    // Q4_0 8192 x 576 5.0 / 4.3, 4096 x 576 3.7 / 4.3; 4096 x 2112 6.4 / 4.8, 2048 x 2112 4.6 / 4.7;
+    // 4096 x 8000 11.7 / 9.3, 2048 x 8000 7.6 / 7.9; Q8_0 alike)
+    if (a.pre == kPreSwiGlu) return a.M > (a.K <= 1344 ? 6000 : 2500);
     if (a.K <= kShortK) return QT != kRows8 && a.M > (k5 ? 14000 : 24000);
     if (a.K <= 1344) return a.M > (k5 ? 10000 : 20000);
     if (k5) return m >= (a.K <= 2048 ? 15 : 16);

@@ -302,8 +302,9 @@ ASMHIP_API int asmhip_attention_decode_rope_table(const float* qkv, void* k_cach
  * asmhip_matmul_attn_output then computes y = W . attn (accumulate: y += W .
  * attn) for GGUF blocks W [M][n_heads * head_dim / 32] (qtype Q4_0 or Q8_0),
  * where attn is the merged attention output.  The merge runs inside the matvec's
- * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024,
- * and for Q4_0 where the int8-MFMA stream takes the shape (head_dim 64 or 128, n_heads
+ * read of x for at most 8 splits (max_ctx <= 4096) where n_heads * head_dim <= 1024
+ * (past 512, up to 6144 rows), and for Q4_0 above that where the int8-MFMA stream takes
+ * the shape (head_dim 64 or 128, n_heads
  * * head_dim a multiple of 256 and at most 8192); otherwise a merge launch writes attn
  * to `work` (n_heads * head_dim floats) and a matvec reads it.  Results equal the
  * merge launch + asmhip_matmul_fused, bit for bit.
