@@ -52,20 +52,16 @@ constexpr int kShortK = 1024, kWaveK = 8192;  // 64-bit sums up to, matvec_wave 
 enum RowsFmt : int { kRows4 = 0, kRows5 = 1, kRows8 = 2 };
 
 // What a unit of matvec_rows holds: kPack64 (K <= 1024) and kPack32 (K <= 2048) the blocks
-// of up to 16 rows, one after another on the lanes, so that no pass is half empty; kTwo
-// (K <= 4096) two rows of two blocks a lane; 1..4 so many blocks a lane of one row, a chunk
-// of it.
-enum RowsMode : int { kPack64 = 0, kPack32 = 5, kTwo = 6 };
+// of up to 16 rows, one after another on the lanes, so that no pass is half empty; 1 and 2
+// so many blocks a lane of one row, a chunk of it.
+enum RowsMode : int { kPack64 = 0, kPack32 = 3 };
 template <int MODE>
 struct RowsShape {
     static constexpr bool kPacked = MODE == kPack64 || MODE == kPack32;
-    static constexpr bool kChunked = MODE >= 1 && MODE <= 4;
-    static constexpr int NP = kPacked ? 1 : MODE == kTwo ? 2 : MODE;  // blocks a lane of one row
-    static constexpr int RU = MODE == kTwo ? 2 : 1;                   // rows
-    static constexpr int NI = kPacked ? 3 : NP * RU;
-    static constexpr int kMaxRows = kPacked ? 16 : RU;
+    static constexpr int NI = kPacked ? 3 : MODE;
+    static constexpr int kMaxRows = kPacked ? 16 : 1;
     // passes of RMSNorm's squares: as matvec_wave's, at most four (above kWaveK by threads)
-    static constexpr int kSq = MODE == kPack64 ? 2 : kChunked ? 4 : NP;
+    static constexpr int kSq = MODE == kPack64 ? 2 : MODE == kPack32 ? 1 : 4;
     using Sum = std::conditional_t<MODE == kPack64, double, float>;  // of a packed block's products
 };
 
@@ -260,13 +256,13 @@ struct RowsArgs {
 template <int QT, bool GGUF, int MODE>
 __global__ __launch_bounds__(kWaves * 64) void matvec_rows(const RowsArgs a) {
     using S = RowsShape<MODE>;
-    constexpr int NI = S::NI, NP = S::NP, kThreads = kWaves * 64;
+    constexpr int NI = S::NI, kThreads = kWaves * 64;
     using U = RowsUnit<QT, GGUF, NI>;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ float red[kWaves], ybuf[2][kWaves * S::kMaxRows];
     const int nb = a.K >> 5, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rw = a.rw, tile_rows = kWaves * rw, nchunk = S::kChunked ? a.nchunk : 1, G = gridDim.x;
+    const int rw = a.rw, tile_rows = kWaves * rw, nchunk = S::kPacked ? 1 : a.nchunk, G = gridDim.x;
     const uint32_t nblocks = (uint32_t)a.M * (uint32_t)nb;
     // whole dwords: an odd number of GGUF blocks ends inside one (of the 4-byte aligned
     // buffer), and a dword that reaches past the descriptor would read as zero
@@ -281,15 +277,8 @@ __global__ __launch_bounds__(kWaves * 64) void matvec_rows(const RowsArgs a) {
     auto unit = [&](int row, int c, uint32_t* b0) {
         const int row0 = row + wave * rw;
         *b0 = (uint32_t)row0 * (uint32_t)nb + (uint32_t)(c * 64 * NI);
-        const int n = S::kChunked ? min(64 * NI, nb - c * 64 * NI) : min(rw, a.M - row0) * nb;
+        const int n = S::kPacked ? min(rw, a.M - row0) * nb : min(64 * NI, nb - c * 64 * NI);
         return row0 < a.M ? n : 0;
-    };
-    // the place of the lane's k-th block in a unit: from the unit's end on if there is none
-    // (a row's last pass is not full)
-    auto place = [&](int k) {
-        if (S::kPacked || S::RU == 1) return lane + 64 * k;
-        const int col = lane + 64 * (k % NP);
-        return col < nb ? k / NP * nb + col : 1 << 30;
     };
     U u;
     auto load = [&](int row, int c) {
@@ -306,7 +295,7 @@ __global__ __launch_bounds__(kWaves * 64) void matvec_rows(const RowsArgs a) {
         } else {
 #pragma unroll
             for (int k = 0; k < NI; ++k) {
-                const int b = place(k);
+                const int b = lane + 64 * k;
                 const uint32_t blk = b0 + (uint32_t)b;
 #pragma unroll
                 for (int h = 0; h < U::kQs / 16; ++h)
@@ -486,34 +475,29 @@ __global__ __launch_bounds__(kWaves * 64) void matvec_rows(const RowsArgs a) {
             }
         } else {
 #pragma unroll
-            for (int t = 0; t < S::RU; ++t) {
-                if (t >= rw) break;  // wave-uniform
+            for (int k = 0; k < NI; ++k) {
+                const int b = lane + 64 * k;
+                if (b < n) {
+                    uint32_t q[U::kQs / 4], nh = 0, lo, hi;
+                    float d;
+                    block(k, b, q, &nh, &d);
+                    const float *xl, *xh;
 #pragma unroll
-                for (int p = 0; p < NP; ++p) {
-                    const int k = t * NP + p, b = place(k);
-                    if (b < n) {
-                        uint32_t q[U::kQs / 4], nh = 0, lo, hi;
-                        float d;
-                        block(k, b, q, &nh, &d);
-                        const float *xl, *xh, *xb = xs + (S::kChunked ? c * 64 * NI + b : lane + 64 * p) * kXPitch;
-#pragma unroll
-                        for (int g = 0; g < 4; ++g) {
-                            item_of<QT>(q, nh, xb, g, &lo, &hi, &xl, &xh);
-                            part[g] = fmaf(d, item_long(lo, hi, xl, xh), part[g]);
-                        }
+                    for (int g = 0; g < 4; ++g) {
+                        item_of<QT>(q, nh, xs + (c * 64 * NI + b) * kXPitch, g, &lo, &hi, &xl, &xh);
+                        part[g] = fmaf(d, item_long(lo, hi, xl, xh), part[g]);
                     }
                 }
-                if (c < nchunk - 1) break;
+            }
+            if (c == nchunk - 1) {
                 float h = (part[0] + part[1]) + (part[2] + part[3]);
                 h += dpp<kDppQuadXor2>(h);
                 h += dpp<kDppQuadXor1>(h);
                 h += dpp<kDppRowHalfMirror>(h);
                 h += dpp<kDppRowMirror>(h);
                 const int v = __float_as_int(h);
-                float tot = 0.f;
 #pragma unroll
-                for (int w = 0; w < 4; ++w) tot += __int_as_float(__builtin_amdgcn_readlane(v, 16 * w));
-                sum = lane == t ? tot : sum;
+                for (int w = 0; w < 4; ++w) sum += __int_as_float(__builtin_amdgcn_readlane(v, 16 * w));
                 part[0] = part[1] = part[2] = part[3] = 0.f;
             }
         }
@@ -734,13 +718,12 @@ int rows_launch_mode(RowsArgs a, hipStream_t st) {
     // more for a unit's loads and sums (26000 x 1024 12.8 us with the fewest rows, one a unit)
     auto tiles = [&](int rw) { return ((int64_t)a.M + kWaves * rw - 1) / (kWaves * rw); };
     auto cost = [&](int rw) {
-        const int passes = S::kPacked ? (rw * nb + 63) / 64 : rw * S::NP;
-        return (tiles(rw) + cus - 1) / cus * (passes + 1);
+        return (tiles(rw) + cus - 1) / cus * ((rw * nb + 63) / 64 + 1);
     };
-    a.rw = std::min(S::kMaxRows, S::kPacked ? 64 * S::NI / nb : S::RU);
+    a.rw = S::kPacked ? std::min(S::kMaxRows, 64 * S::NI / nb) : 1;
     for (int rw = a.rw - 1; rw >= 1; --rw)
         if (cost(rw) < cost(a.rw)) a.rw = rw;
-    a.nchunk = S::kChunked ? (nb + 64 * S::NI - 1) / (64 * S::NI) : 1;
+    a.nchunk = (nb + 64 * S::NI - 1) / (64 * S::NI);
     const size_t lds = rows_lds<QT, GGUF, MODE>(nb);
     const int rc = dynamic_lds((const void*)matvec_rows<QT, GGUF, MODE>, lds);
     if (rc) return rc;
@@ -750,21 +733,18 @@ int rows_launch_mode(RowsArgs a, hipStream_t st) {
     return kOk;
 }
 
-// More than 512 columns (16 blocks): the shapes that rows_faster sends here, as many
-// blocks a lane as LDS holds beside x.
+// More than 512 columns (16 blocks).  Small units: a wave multiplies one while the next is
+// under way, and starts sooner (8192 x 5504 Q8_0 one, two and three blocks a lane 11.0 / 12.3 /
+// 12.9 us, Q4_0 9.1 / 9.6 / 10.3); two for Q4 and Q5 rows that are many, short or above 8192
+// columns (33000 x 2080 Q5_0 24.2 / 23.4 / 24.7, 33000 x 8032 Q4_0 38.9 / 38.4 / 38.9).
 template <int QT, bool GGUF>
 int rows_launch_fmt(const RowsArgs& a, hipStream_t st) {
     if (a.K <= kShortK) return rows_launch_mode<QT, GGUF, kPack64>(a, st);
     if (a.K <= 2048) return rows_launch_mode<QT, GGUF, kPack32>(a, st);
-    if constexpr (QT == kRows5 && GGUF)
-        if (a.K <= 4096) return rows_launch_mode<QT, GGUF, kTwo>(a, st);
-    if constexpr (QT == kRows8) {
-        if (a.K <= 4096 || (a.K > 6144 && a.K <= 8192)) return rows_launch_mode<QT, GGUF, 2>(a, st);
-    } else {
-        if (a.K > 6144 && a.K <= 8192) return rows_launch_mode<QT, GGUF, 4>(a, st);
-    }
-    return rows_lds<QT, GGUF, 3>(a.K / 32) <= kLdsBudget ? rows_launch_mode<QT, GGUF, 3>(a, st)
-                                                         : rows_launch_mode<QT, GGUF, 1>(a, st);
+    if constexpr (QT != kRows8)
+        if ((a.K <= 4096 || a.K > kWaveK || a.M > 10000) && rows_lds<QT, GGUF, 2>(a.K / 32) <= kLdsBudget)
+            return rows_launch_mode<QT, GGUF, 2>(a, st);
+    return rows_launch_mode<QT, GGUF, 1>(a, st);
 }
 
 template <int QT, bool GGUF, int NP, int R, int W>
@@ -808,31 +788,36 @@ int wave_launch_fmt(const RowsArgs& a, hipStream_t st) {
 }
 
 // Whether matvec_rows is faster than matvec_wave, which takes up to kWaveK columns: wide
-// loads and x shared by 16 waves, against no barrier before the weights.  Wave / rows, us:
-//   many short rows, several of them a pass: 32000 x 544 Q4_0 8.0 / 6.5, 20000 x 544 5.2 / 5.1,
-//     24000 x 1216 9.0 / 8.1, 16384 x 1216 7.1 / 6.8, 33000 x 1376 (four rows a unit no more)
-//     11.2 / 12.4; Q5_0, whose wave is the slowest, 12000 x 1216 7.8 / 6.4; Q8_0 24000 x 1216
-//     11.8 / 10.1, but 32000 x 768 8.8 / 9.2;
-//   Q5_0 blocks: 12000 x 1376 8.0 / 7.4, 8192 x 2080 9.5 / 8.5, 4096 x 3008 5.8 / 6.2;
-//   Q8_0: 8192 x 2080 8.4 / 7.6, 4096 x 2080 5.5 / 5.6, 16384 x 4128 21.3 / 18.0, 8192 x 5504
-//     13.5 / 13.0, 8192 x 4128 11.8 / 11.6, 4096 x 8032 10.5 / 10.9;
-//   Q4_0 blocks: 16384 x 4128 16.2 / 15.0, 33000 x 3008 20.2 / 22.0, 8192 x 5504 9.8 / 10.3;
-//   split Q4 and Q5: 33000 x 8032 39.8 / 36.2, 33000 x 5504 27.2 / 27.8.
+// loads and x shared by 16 waves, against no barrier before the weights.  Wave / rows, us,
+// with weights from memory, then with weights that stay in the caches:
+//   many short rows, several of them a pass: 33000 x 544 Q4_0 8.3 / 6.7, 7.3 / 5.8, 24000 x 544
+//     6.2 / 5.1, 5.7 / 5.0, 33000 x 1376 (four rows a unit no more) 11.2 / 12.3, 8.8 / 11.5;
+//     from memory 24000 x 1216 9.0 / 8.1; Q5_0, whose wave is the slowest, 12000 x 1216 7.8 /
+//     6.4; Q8_0 24000 x 1216 11.8 / 10.1, 33000 x 544 8.7 / 8.3, 6.7 / 6.3 (split 7.8 / 8.3,
+//     6.5 / 5.6), but 32000 x 768 8.8 / 9.2;
+//   longer rows, a wave each and nearly all waves of the device the same number of them: Q8_0
+//     8192 x 4128 11.9 / 9.9, 8.4 / 8.7, but 5000 x 4128 8.4 / 9.5, 5.9 / 8.4, and 4096 x 4128
+//     7.4 / 6.7, 5.1 / 5.7, 4096 x 6208 10.1 / 8.9, 6.8 / 7.1; Q5_0 4096 x 4128 8.0 / 6.6, 6.1 /
+//     6.2; Q4_0 8192 x 4128 9.2 / 8.5, 7.4 / 8.0, 16384 x 4128 16.0 / 14.4, 12.7 / 13.3, 8192 x
+//     8032 13.3 / 11.4, 10.4 / 10.4; split Q4 16384 x 4128 13.6 / 13.5, 11.2 / 12.4, 8192 x 8032
+//     12.3 / 11.2, 9.9 / 9.5; split Q8 16384 x 4128 18.9 / 17.2, 13.5 / 13.7.
+// matvec_rows also forms the SwiGLU of x once for 16 waves and all their rows (Q4_0 8192 x 576
+// 5.0 / 4.3, 4096 x 576 3.7 / 4.3; 4096 x 2112 6.4 / 4.8, 2048 x 2112 4.6 / 4.7; Q8_0 alike).
 template <int QT, bool GGUF>
 bool rows_faster(const RowsArgs& a) {
     constexpr bool k5 = QT == kRows5 && GGUF;
-    const int64_t m = (int64_t)a.M * a.K >> 20;  // weights, in 2^20
     if (a.K > kWaveK) return true;
     if (a.K <= 512) return false;
-    // matvec_rows forms the SwiGLU of x once for 16 waves and all their rows (wave / rows, us:
-    // Q4_0 8192 x 576 5.0 / 4.3, 4096 x 576 3.7 / 4.3; 4096 x 2112 6.4 / 4.8, 2048 x 2112 4.6 / 4.7;
-    // 4096 x 8000 11.7 / 9.3, 2048 x 8000 7.6 / 7.9; Q8_0 alike)
     if (a.pre == kPreSwiGlu) return a.M > (a.K <= 1344 ? 6000 : 2500);
-    if (a.K <= kShortK) return QT != kRows8 && a.M > (k5 ? 14000 : 24000);
-    if (a.K <= 1344) return a.M > (k5 ? 10000 : 20000);
-    if (k5) return m >= (a.K <= 2048 ? 15 : 16);
-    if (QT == kRows8) return a.K > 2048 && m >= (a.K <= 4096 ? 16 : 40);
-    return GGUF ? a.K > 4096 && m >= 60 : a.K > 6144 && m >= 120;
+    if (a.K <= kShortK && QT == kRows8) return a.K <= 640 && a.M > 28000;
+    if (a.K <= kShortK) return a.M > (k5 ? 14000 : a.K <= 768 ? 20000 : 24000);
+    if (a.K <= 1344) return a.M > (k5 ? 10000 : GGUF ? 16000 : 20000);
+    if (a.K <= 2048) return k5 && a.M > 11000;
+    const int64_t round = (int64_t)kWaves * row_units(), rounds = (a.M + round - 1) / round;
+    if (20 * (int64_t)a.M < 17 * rounds * round) return false;  // the last round too empty
+    if (GGUF && a.K > (QT == kRows5 ? 4096 : 6144)) return a.M > 3400;
+    if (QT != kRows8 && !GGUF) return a.K > 6144 && a.M > 8000;
+    return a.M > (GGUF && QT != kRows4 ? 8000 : 11000);
 }
 
 template <int QT, bool GGUF>

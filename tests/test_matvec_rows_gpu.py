@@ -106,11 +106,11 @@ ROWS_KS = [288, 544, 768, 1024, 1056, 1376, 2048 + 32, 3008, 4128, 5504, 6176, 8
 
 def _rows_of_both_kernels(K):
     """Rows enough for every format that leaves matvec_wave at this K."""
-    return max(33008, (25 << 20) // K + 31) // 16 * 16 if K <= 1376 else ((122 if K > 4096 else 25) << 20) // K // 16 * 16 + 16
+    return 33008 if K <= 1376 else 16368
 
 
 def _prefixes(M):
-    return [m for m in (1, 5, 47, 300, 1000, 2049, 4097, 8193, 16400) if m < M]
+    return [m for m in (1, 5, 47, 300, 1000, 2049, 4000, 4097, 8100, 8193, 16400) if m < M]
 
 
 @pytest.mark.parametrize("q", [4, 5, 8])
@@ -183,7 +183,7 @@ def test_row_kernels_error_of_the_norm(hip, q, M, K):
 
 
 @pytest.mark.parametrize("q", [4, 5, 8])
-@pytest.mark.parametrize("M,K", [(300, 288), (2000, 1024), (700, 1088), (33000, 1088), (600, 5504), (70, 8224)])
+@pytest.mark.parametrize("M,K", [(300, 288), (2000, 1024), (700, 1088), (33000, 1088), (600, 5504), (70, 8224), (16380, 3008)])
 def test_row_kernels_x_off_16_bytes(hip, q, M, K):
     rng = np.random.default_rng(M + K)
     b, _ = _weights(rng, q, M, K)
@@ -195,7 +195,7 @@ def test_row_kernels_x_off_16_bytes(hip, q, M, K):
         assert np.array_equal(dy.download(np.float32, (M,)), _call(hip, q, False, b, x[off:off + K], M, K)), off
 
 
-@pytest.mark.parametrize("M,K", [(4096, 5504), (16400, 2080), (5000, 8224)])
+@pytest.mark.parametrize("M,K", [(4096, 5504), (16400, 2080), (5000, 8224), (16380, 2080), (8190, 5504)])
 def test_row_kernels_many_units(hip, M, K):
     """Several units per wave, and rows cut into chunks (matvec_rows' stream)."""
     rng = np.random.default_rng(M)
